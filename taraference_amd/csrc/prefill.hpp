@@ -13,11 +13,9 @@
 int tf_gemm_kq(bool q6, const uint8_t* w, const float* x, float* out, int n_rows, int n_cols,
                int col_bytes, int n_tok, int accumulate, tf_stream_t stream, float* ws,
                size_t ws_floats);
-// split-K workspace that serves any shape: n_split * n_tok * n_cols with
-// n_split = ceil(512 / tiles) with tiles < 384 of 32 x 128 outputs needs at
-// most 896 tiles of slices; a larger split (the tuning override) is clamped
-// to what fits.
-static const size_t kGemmWsFloats = (size_t)1152 * 32 * 128;
+// split-K workspace: n_split * n_tok * n_cols floats, n_split being what brings
+// the 32 x 256 output tiles to 512; a larger split is clamped to what fits.
+static const size_t kGemmWsFloats = (size_t)1152 * 32 * 256;
 int tf_attn_prefill_any(const float* q, const uint16_t* k_cache, const uint16_t* v_cache,
                         float* out, int n_head, int n_kv, int head_dim, int pos0,
                         const int* pos0_dev, int n_q, float scale, tf_stream_t stream);

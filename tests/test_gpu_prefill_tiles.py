@@ -1,0 +1,77 @@
+"""The prefill GEMMs (tf_gemm_q4k_f32 / tf_gemm_q6k_f32, kernels/gemm.cu:6-121)
+at the edges of their tiles and on every branch of their dispatch, against the
+fp64 product with numpy-dequantized weights (tests/_util.gemm_ref), within the
+fp32 GEMV tolerance (1e-5 relative, floor 0.1 * sum |terms|): the split of x
+keeps 22 bits of each value, 2^-23 of a term, and the rest is fp32 summation.
+
+The token tile is 32, a wave's columns 64; the dispatch goes by the number of
+32 x 64 and 32 x 256 output tiles, the Q6_K loads by where a column starts
+modulo 4 (an odd number of 210-byte blocks makes it alternate).
+"""
+import numpy as np
+import pytest
+
+from taraference_amd import synth
+from _gpu import P, S, call, dev, empty, host
+from _util import assert_gemv_close, gemm_ref
+
+pytestmark = pytest.mark.gpu
+
+
+def run(fmt, n_rows, n_cols, x, shift=0, seed=0):
+    """The GEMM with the weights `shift` bytes into their buffer."""
+    rng = np.random.default_rng(n_rows + 3 * n_cols + seed)
+    w, cb = (synth.q4k_matrix if fmt == "q4k" else synth.q6k_matrix)(rng, n_rows, n_cols)
+    if fmt == "q6k":  # scales over their whole range: products past f16's exact integers
+        blk = w.reshape(-1, 210)
+        blk[:, 192:208] = rng.integers(-128, 128, (blk.shape[0], 16)).astype(np.int8).view(np.uint8)
+    buf = dev(np.concatenate([np.zeros(shift, np.uint8), w.reshape(-1)]))
+    n_tok = x.shape[0]
+    out = empty(n_tok * n_cols)
+    print(f"gemm {fmt} {n_rows}x{n_cols} tok={n_tok} shift={shift}", flush=True)
+    call(f"tf_gemm_{fmt}_f32", P(buf) + shift, P(dev(x)), P(out), n_rows, n_cols, cb, n_tok, S())
+    y = host(out).reshape(n_tok, n_cols)
+    ref, absn = gemm_ref(fmt, w, n_rows, x)
+    for t in range(n_tok):
+        assert_gemv_close(y[t], ref[t], absn[t], f"{fmt} t={t}")
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q6k"])
+@pytest.mark.parametrize("n_rows,n_cols,n_tok", [
+    (256, 1, 1),        # one value; most K slices empty
+    (768, 63, 31),      # 3 super-blocks over 4 slices, one short of a tile each way
+    (768, 65, 33),      # one past a tile
+    (1280, 129, 32),    # 5 super-blocks
+    (512, 4100, 130),   # 128 columns and K split: 325 tiles of 64 columns
+    (1792, 3200, 200),  # the same with 7 super-blocks
+    (256, 8200, 190),   # 256 columns: 198 tiles, ragged both ways
+    (768, 6145, 260),
+])
+def test_gemm_tiles(gpu, fmt, n_rows, n_cols, n_tok):
+    x = np.random.default_rng(n_tok).standard_normal((n_tok, n_rows)).astype(np.float32)
+    run(fmt, n_rows, n_cols, x)
+
+
+@pytest.mark.parametrize("fmt,shift", [("q4k", 4), ("q4k", 8), ("q6k", 2), ("q6k", 4), ("q6k", 6)])
+@pytest.mark.parametrize("n_rows,n_cols,n_tok", [(768, 70, 5), (512, 4100, 130), (768, 6145, 260)])
+def test_gemm_unaligned_weights(gpu, fmt, shift, n_rows, n_cols, n_tok):
+    x = np.random.default_rng(n_tok).standard_normal((n_tok, n_rows)).astype(np.float32)
+    run(fmt, n_rows, n_cols, x, shift)
+
+
+@pytest.mark.parametrize("fmt", ["q4k", "q6k"])
+def test_gemm_scales_of_x(gpu, fmt):
+    """Each (token, super-block) has its own power of two: rows and
+    super-blocks of very different magnitude, zero rows, the smallest and
+    largest scales (the products stay finite)."""
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((40, 768)).astype(np.float32)
+    x[1] = 0
+    x[2, :256] = 0
+    x[3] *= np.float32(1e-30)
+    x[4] *= np.float32(1e30)
+    x[5, 256:512] *= np.float32(1e-12)
+    x[6, ::7] *= np.float32(1e4)
+    x[7] = np.float32(1e-38)  # subnormal products with the block scales still count
+    x[8] = 1
+    run(fmt, 768, 200, x)
