@@ -137,8 +137,10 @@ struct tf_model {
     int *d_forced = nullptr, *d_nforced = nullptr, *d_log = nullptr;
     // prefill workspace (n_tok-row activations of one chunk), allocated on
     // the first prefill
-    float *pf_x = nullptr, *pf_xb = nullptr, *pf_q = nullptr, *pf_k = nullptr, *pf_v = nullptr,
-          *pf_att = nullptr, *pf_g = nullptr, *pf_u = nullptr, *pf_ws = nullptr;
+    float *pf_x = nullptr, *pf_q = nullptr, *pf_att = nullptr, *pf_g = nullptr, *pf_u = nullptr,
+          *pf_ws = nullptr;
+    size_t pf_ws_floats = 0;
+    uint8_t* pf_img = nullptr;
     int* pf_tok = nullptr;
     std::vector<void*> allocs;
 
@@ -655,17 +657,11 @@ struct tf_model {
         if (path == 4 && d_trace) dump_trace();
     }
 
-    // Prompt chunk size of the prefill (types.rs MAX_BATCH).
-    static constexpr int kPrefillChunk = 256;
-
-    // x[t] (+)= W xin[t] for n rows on the matrix cores (raw GGUF bytes).
-    void gemm(hipStream_t s, const GpuMat& w, const float* xin, float* out, int n,
-              bool accumulate) {
-        tf::check(tf_gemm_kq(w.wtype == tf::WType::Q6K, w.data, xin, out, (int)w.n_rows,
-                             (int)w.n_cols, (int)w.col_bytes, n, accumulate ? 1 : 0,
-                             reinterpret_cast<tf_stream_t>(s), pf_ws, kGemmWsFloats),
-                  "prefill gemm");
-    }
+    // Tokens of a prompt that go through the layers together.  The reference
+    // takes 256 (types.rs MAX_BATCH); the weights are read and unpacked once a
+    // chunk and a chunk's tiles have to fill 256 CUs, so a longer one pays:
+    // 700 tokens of two 3B layers in one chunk / in three.
+    static constexpr int kPrefillChunk = 1024;
 
     // The prompt forward of forward.rs:42-71 forward_greedy / :360-404
     // forward_chunk: chunks of up to kPrefillChunk tokens through the
@@ -673,28 +669,29 @@ struct tf_model {
     // n_tok > 1: rms_norm rows, GEMMs, add_bias, rope, copy_kv, prefill
     // attention, GEMM + add for wo and down, silu_mul), K/V appended at
     // positions pos0 .. pos0+n-1; then the last row's logits and argmax
-    // (logits_from_last), as the decode step computes them.
+    // (logits_from_last), as the decode step computes them.  Per layer nine
+    // launches: each GEMM's K slices are added by the kernel that reads them.
     void prefill(hipStream_t s, const int* tokens, int n, int pos0) {
         const tf_model_config& c = cfg;
         if (n < 1 || pos0 < 0 || pos0 + n > c.max_seq)
             throw tf::HipError((int)hipErrorInvalidValue, "prefill range outside the KV cache");
         if (!kquant_ok())
             throw tf::HipError((int)hipErrorNotSupported, "prefill needs Q4_K/Q6_K weights");
-        const int CH = kPrefillChunk, E = c.n_embd, F = c.n_ff;
+        const int CH = std::min(kPrefillChunk, c.max_seq), E = c.n_embd, F = c.n_ff;
         const int kvd = c.n_kv * c.head_dim;
         if (!pf_x) {
-            pf_x = alloc<float>((size_t)CH * E);
-            pf_xb = alloc<float>((size_t)CH * E);
             pf_q = alloc<float>((size_t)CH * E);
             pf_att = alloc<float>((size_t)CH * E);
-            pf_k = alloc<float>((size_t)CH * kvd);
-            pf_v = alloc<float>((size_t)CH * kvd);
             pf_g = alloc<float>((size_t)CH * F);
-            pf_u = alloc<float>((size_t)CH * F);
             pf_tok = alloc<int>(CH);
-            pf_ws = alloc<float>(kGemmWsFloats);
+            pf_img = alloc<uint8_t>(tf_pg_image_bytes(std::max(E, F), CH));
+            // the GEMM slices: two of a full chunk's widest output, and more of a short one's
+            pf_ws_floats = std::max((size_t)4 * CH * (E + 2 * kvd), (size_t)4 << 20);
+            pf_ws = alloc<float>(pf_ws_floats);
+            pf_x = alloc<float>((size_t)CH * E);
         }
         const tf_stream_t ts = reinterpret_cast<tf_stream_t>(s);
+        auto blk = [](const GpuMat& w) { return w.wtype == tf::WType::Q6K ? 210 : 144; };
         int last = 0;
         for (int off = 0; off < n; off += CH) {
             const int nt = n - off < CH ? n - off : CH;
@@ -703,26 +700,54 @@ struct tf_model {
                                           hipMemcpyHostToDevice, s), "copy tokens");
             tf::check(tf_pf_embed(token_embd.data, embd_block_bytes, pf_tok, pf_x, E,
                                   (int)token_embd.col_bytes, nt, ts), "embed");
+            TfPgPart part{nullptr, 0, 0};
+            // x += W a for the image of a; the add is the next kernel's
+            auto gemm_add = [&](const GpuMat& w) {
+                const bool compact = w.wtype == tf::WType::Q6K && w.compact_data;
+                tf::check(tf_pg_gemm(compact ? w.compact_data : w.data, compact ? 212 : blk(w),
+                                     pf_img, (int)w.n_rows, (int)w.n_cols,
+                                     (int)(compact ? w.compact_col_bytes : w.col_bytes), nt, pf_ws,
+                                     pf_ws_floats, &part, ts), "prefill gemm");
+            };
             for (size_t li = 0; li < layers.size(); li++) {
                 const Layer& L = layers[li];
-                tf::check(tf_pf_rms_norm(pf_x, L.attn_norm, pf_xb, E, nt, c.rms_eps, ts), "rms");
-                gemm(s, L.wq, pf_xb, pf_q, nt, false);
-                gemm(s, L.wk, pf_xb, pf_k, nt, false);
-                gemm(s, L.wv, pf_xb, pf_v, nt, false);
-                tf::check(tf_pf_qkv_post(pf_q, pf_k, pf_v, L.bq, L.bk, L.bv, kc[li], vc[li],
-                                         c.n_head, c.n_kv, c.head_dim, p0, nt, c.rope_theta, ts),
+                tf::check(tf_pg_norm_image(pf_x, li ? &part : nullptr, L.attn_norm, c.rms_eps,
+                                           pf_img, E, nt, ts), "norm");
+                const uint8_t* w[3] = {L.wq.data, L.wk.data, L.wv.data};
+                const int bb[3] = {blk(L.wq), blk(L.wk), blk(L.wv)};
+                const int nc[3] = {(int)L.wq.n_cols, (int)L.wk.n_cols, (int)L.wv.n_cols};
+                const int cb[3] = {(int)L.wq.col_bytes, (int)L.wk.col_bytes, (int)L.wv.col_bytes};
+                tf::check(tf_pg_qkv(w, bb, nc, cb, pf_img, E, nt, pf_ws, pf_ws_floats, &part, ts),
+                          "qkv");
+                tf::check(tf_pg_qkv_post(part, L.bq, L.bk, L.bv, pf_q, kc[li], vc[li], c.n_head,
+                                         c.n_kv, c.head_dim, p0, nt, c.rope_theta, ts),
                           "qkv post");
                 tf::check(tf_attn_prefill_any(pf_q, kc[li], vc[li], pf_att, c.n_head, c.n_kv,
                                               c.head_dim, p0, nullptr, nt, fd.scale, ts),
                           "prefill attention");
-                gemm(s, L.wo, pf_att, pf_x, nt, true);
-                tf::check(tf_pf_rms_norm(pf_x, L.ffn_norm, pf_xb, E, nt, c.rms_eps, ts), "rms");
-                gemm(s, L.gate, pf_xb, pf_g, nt, false);
-                gemm(s, L.up, pf_xb, pf_u, nt, false);
-                tf::check(tf_pf_silu_mul(pf_g, pf_u, (long long)nt * F, ts), "silu_mul");
-                gemm(s, L.down, pf_g, pf_x, nt, true);
+                tf::check(tf_pg_image(pf_att, pf_img, E, nt, ts), "image");
+                gemm_add(L.wo);
+                tf::check(tf_pg_norm_image(pf_x, &part, L.ffn_norm, c.rms_eps, pf_img, E, nt, ts),
+                          "norm");
+                if (L.gate.wtype == tf::WType::Q4K && L.up.wtype == tf::WType::Q4K &&
+                    L.gate.col_bytes == L.up.col_bytes) {
+                    tf::check(tf_pg_gate_up(L.gate.data, L.up.data, pf_img, pf_g, E, F,
+                                            (int)L.gate.col_bytes, nt, ts), "gate/up");
+                } else {  // one at a time, whole (the room of one slice)
+                    if (!pf_u) pf_u = alloc<float>((size_t)CH * F);
+                    TfPgPart g;
+                    const size_t room = (size_t)nt * F;
+                    tf::check(tf_pg_gemm(L.gate.data, blk(L.gate), pf_img, E, F,
+                                         (int)L.gate.col_bytes, nt, pf_g, room, &g, ts), "gate");
+                    tf::check(tf_pg_gemm(L.up.data, blk(L.up), pf_img, E, F,
+                                         (int)L.up.col_bytes, nt, pf_u, room, &g, ts), "up");
+                    tf::check(tf_pf_silu_mul(pf_g, pf_u, (long long)nt * F, ts), "silu_mul");
+                }
+                tf::check(tf_pg_image(pf_g, pf_img, F, nt, ts), "image");
+                gemm_add(L.down);
             }
             last = nt - 1;
+            if (off + CH >= n) tf::check(tf_pg_add_row(pf_x, part, last, E, ts), "add");
         }
         // logits of the last prompt token (the decode step's head)
         const float* xl = pf_x + (size_t)last * E;

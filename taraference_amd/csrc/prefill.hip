@@ -333,10 +333,8 @@ __global__ __launch_bounds__(256) void tf_attn_prefill_mfma_kernel(
 
 // ------------------------------------------------- batched prefill glue
 //
-// The n_tok-row forms of the decode glue (kernels/ops.cu rms_norm_f32 with
-// n_tok rows :4-34, add_bias_f32 :340, rope_neox_f32 :348, copy_kv_f16
-// :471, silu_mul_f32 :202; kernels/embed.cu embed_q{4,6}_k :1-50), used by
-// the runtime's prefill step.
+// Embedding rows of a prompt (kernels/embed.cu embed_q{4,6}_k :1-50) and
+// silu_mul_f32 (kernels/ops.cu:202).
 
 template <int BB>
 __global__ __launch_bounds__(256) void tf_pf_embed_kernel(const uint8_t* __restrict__ table,
@@ -349,84 +347,6 @@ __global__ __launch_bounds__(256) void tf_pf_embed_kernel(const uint8_t* __restr
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nb * 256; i += gridDim.x * blockDim.x) {
         const uint8_t* blk = col + (size_t)(i >> 8) * BB;
         out[(size_t)t * n_rows + i] = BB == 144 ? tf_q4k_value(blk, i & 255) : tf_q6k_value(blk, i & 255);
-    }
-}
-
-// One row per workgroup, the decode RMSNorm's order (256 strided fused
-// square sums, halving tree).
-__global__ __launch_bounds__(256) void tf_pf_rms_kernel(const float* __restrict__ x,
-                                                        const float* __restrict__ w,
-                                                        float* __restrict__ out, int n, float eps) {
-    __shared__ float buf[256];
-    const float* xr = x + (size_t)blockIdx.x * n;
-    float* orow = out + (size_t)blockIdx.x * n;
-    float local = 0.f;
-    for (int i = threadIdx.x; i < n; i += 256) {
-        const float v = xr[i];
-        local = fmaf(v, v, local);
-    }
-    buf[threadIdx.x] = local;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) buf[threadIdx.x] += buf[threadIdx.x + s];
-        __syncthreads();
-    }
-    const float scale = 1.0f / sqrtf(buf[0] / (float)n + eps);
-    for (int i = threadIdx.x; i < n; i += 256) orow[i] = xr[i] * scale * w[i];
-}
-
-// q/k/v rows of token t (position pos0 + t): add the biases, rotate q and k
-// (NeoX pairs (i, i + hd/2) by (pos0+t) theta^(-2i/hd)), append k and v to
-// the f16 cache.  Grid (n_head + 2 n_kv, n_tok): head blocks of q, then k,
-// then v.
-__global__ __launch_bounds__(64) void tf_pf_qkv_post_kernel(
-    float* __restrict__ q, float* __restrict__ k, float* __restrict__ v,
-    const float* __restrict__ bq, const float* __restrict__ bk, const float* __restrict__ bv,
-    uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int n_head, int n_kv, int hd, int pos0,
-    float theta) {
-    const int t = blockIdx.y, hb = blockIdx.x;
-    const int kvd = n_kv * hd, pos = pos0 + t;
-    float* base;
-    const float* b;
-    uint16_t* cache = nullptr;
-    bool rot = true;
-    if (hb < n_head) {
-        base = q + (size_t)t * n_head * hd + hb * hd;
-        b = bq ? bq + hb * hd : nullptr;
-    } else if (hb < n_head + n_kv) {
-        const int h = hb - n_head;
-        base = k + (size_t)t * kvd + h * hd;
-        b = bk ? bk + h * hd : nullptr;
-        cache = kc + (size_t)pos * kvd + h * hd;
-    } else {
-        const int h = hb - n_head - n_kv;
-        base = v + (size_t)t * kvd + h * hd;
-        b = bv ? bv + h * hd : nullptr;
-        cache = vc + (size_t)pos * kvd + h * hd;
-        rot = false;
-    }
-    const int half = hd / 2;
-    for (int i = threadIdx.x; i < half; i += blockDim.x) {
-        float x0 = base[i], x1 = base[i + half];
-        if (b) {
-            x0 += b[i];
-            x1 += b[i + half];
-        }
-        if (rot) {
-            const float freq = powf(theta, -2.f * (float)i / (float)hd);
-            const float ang = (float)pos * freq;
-            float sn, cs;
-            sincosf(ang, &sn, &cs);
-            const float r0 = x0 * cs - x1 * sn, r1 = x0 * sn + x1 * cs;
-            x0 = r0;
-            x1 = r1;
-        }
-        base[i] = x0;
-        base[i + half] = x1;
-        if (cache) {
-            cache[i] = tf_f2h_halfup(x0);
-            cache[i + half] = tf_f2h_halfup(x1);
-        }
     }
 }
 
@@ -452,25 +372,6 @@ int tf_pf_embed(const uint8_t* table, int block_bytes, const int* tokens_dev, fl
     else
         hipLaunchKernelGGL(tf_pf_embed_kernel<210>, grid, dim3(256), 0, tf_stream(stream), table,
                            tokens_dev, out, n_rows, col_bytes);
-    return TF_LAUNCH_RESULT();
-}
-
-int tf_pf_rms_norm(const float* x, const float* w, float* out, int n, int n_tok, float eps,
-                   tf_stream_t stream) {
-    TF_CHECK_ARG(x && w && out && n > 0 && n_tok > 0);
-    hipLaunchKernelGGL(tf_pf_rms_kernel, dim3(n_tok), dim3(256), 0, tf_stream(stream), x, w, out,
-                       n, eps);
-    return TF_LAUNCH_RESULT();
-}
-
-int tf_pf_qkv_post(float* q, float* k, float* v, const float* bq, const float* bk,
-                   const float* bv, uint16_t* k_cache, uint16_t* v_cache, int n_head, int n_kv,
-                   int head_dim, int pos0, int n_tok, float theta, tf_stream_t stream) {
-    TF_CHECK_ARG(q && k && v && k_cache && v_cache && n_head > 0 && n_kv > 0 && n_tok > 0);
-    TF_CHECK_ARG(head_dim > 0 && (head_dim & 1) == 0 && pos0 >= 0);
-    hipLaunchKernelGGL(tf_pf_qkv_post_kernel, dim3(n_head + 2 * n_kv, n_tok), dim3(64), 0,
-                       tf_stream(stream), q, k, v, bq, bk, bv, k_cache, v_cache, n_head, n_kv,
-                       head_dim, pos0, theta);
     return TF_LAUNCH_RESULT();
 }
 

@@ -30,7 +30,8 @@
 // passes through LDS.  A workgroup is CW column groups x KW slices of K:
 // wide outputs take CW = 4, KW = 1 (the x image is shared by 256 columns);
 // with few tiles the waves of a workgroup split K instead and add their sums
-// at the end.
+// at the end.  The runtime's prompts bring x already split (images made by
+// the kernel that produces it), so their GEMMs only copy it into LDS.
 //
 // K order.  Within a super-block the lanes of half h (lane / 32) take bytes
 // 16 h .. 16 h + 15 of each 32-byte run of codes, so a lane reads 16 contiguous
@@ -38,6 +39,7 @@
 // h supplies values 32 s + 16 h + 8 b + {0, 2, 1, 3, 4, 6, 5, 7} (the order in
 // which nibbles come out of a dword), for x and W alike.
 #include <algorithm>
+#include <type_traits>
 
 #include "lds_dma.hpp"
 #include "prefill.hpp"
@@ -82,6 +84,13 @@ __device__ __forceinline__ tf_pg_h2 tf_pg_fma2(tf_pg_h2 a, tf_pg_h2 b, tf_pg_h2 
 // Weight formats: Q4_K, raw 210-byte Q6_K blocks in memory that starts at a
 // multiple of 4 bytes (W6), or of 2 (W6U), and 212-byte compact Q6_K blocks.
 enum { TF_PG_W4, TF_PG_W6, TF_PG_W6U, TF_PG_W6C };
+
+struct TfPgQkv {
+    const uint8_t* w[3];
+    int n_cols[3], col_bytes[3], fmt[3];
+    int ct[3];   // column tiles of 256 up to and including this matrix
+    int col[3];  // first output column
+};
 
 // What a lane holds of one column for one super-block.
 template <bool Q6>
@@ -209,38 +218,27 @@ __device__ __forceinline__ void tf_pg_store_x(const tf_pg_f4 (&xr)[NP][2], uint8
 // wave 64 columns x 32 TT tokens.  PRE: x is already in images (ximg,
 // [token tile of 32][super-block], TF_PG_SLOT bytes each) and is copied into
 // LDS; otherwise the workgroup converts x itself.
-// Waves per SIMD: 3 where the registers allow it (Q4_K without conversion
-// registers), else 2, or what four images of LDS (136 KB) leave room for.
-template <int FMT, int TT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false>
-__global__ __launch_bounds__(64 * CW * KW, KW * NBUF * TT >= 4 ? CW * KW / 4
-                                           : PRE && FMT == TF_PG_W4 && TT == 1 ? 3
-                                                                               : 2) void
-tf_gemm_kq_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
-                  const float* __restrict__ x, const uint8_t* __restrict__ ximg,
-                  float* __restrict__ out, int n_rows, int n_cols, int col_bytes, int n_tok,
-                  int accumulate, int n_split, long long split_stride) {
+// One workgroup's tile: tokens t0 .., columns c0 .. of this wave's 64 (DUAL:
+// 32 of w and 32 of w2), slice z of n_split.  out has rows of ldo floats.
+template <int FMT, int TT, int CW, int KW, bool PRE, int NBUF, bool DUAL>
+__device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint8_t* __restrict__ w,
+                                           const uint8_t* __restrict__ w2,
+                                           const float* __restrict__ x,
+                                           const uint8_t* __restrict__ ximg,
+                                           float* __restrict__ out, int ldo, int n_rows, int n_cols,
+                                           int col_bytes, int n_tok, int accumulate, int n_split,
+                                           int t0, int ctile) {
     constexpr int CPW = DUAL ? 32 : 64;  // output columns of a wave
     constexpr bool Q6 = FMT != TF_PG_W4;
     constexpr int BLK = FMT == TF_PG_W4 ? 144 : FMT == TF_PG_W6C ? 212 : 210;
     constexpr int RP = 2 * CW, NP = 32 * TT / RP;  // tokens staged per pass, passes
-    __shared__ __align__(16) uint8_t lds[KW * NBUF * TT * TF_PG_SLOT];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cw = wave % CW, kw = wave / CW;
     const int h = lane >> 5, l32 = lane & 31;
     uint8_t* const img0 = lds + kw * NBUF * TT * TF_PG_SLOT;
 
-    // XCD-aware tile order: workgroups go round-robin to the 8 XCDs, so XCD
-    // k = blockIdx.x % 8 takes the contiguous tile range [k per, (k+1) per)
-    // (token tiles fastest): a column tile's weights are fetched into one
-    // XCD's L2 and reused there by all its token tiles.
-    const int ntx = (n_tok + 32 * TT - 1) / (32 * TT);
-    const int n_tiles = ntx * ((n_cols + CPW * CW - 1) / (CPW * CW));
-    const int per = (n_tiles + 7) >> 3;
-    const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if (tile >= n_tiles) return;  // uniform, before any barrier
-    const int t0 = (tile % ntx) * (32 * TT);
-    const int c0 = (tile / ntx) * (CPW * CW) + CPW * cw;
+    const int c0 = ctile * (CPW * CW) + CPW * cw;
     const int nb = n_rows / 256;
     // slice z of nz takes super-blocks [lo, hi); every slice runs n_it rounds
     // (all waves meet all barriers), those past hi with scales of 0
@@ -248,7 +246,6 @@ tf_gemm_kq_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
     const int lo = (int)((long long)z * nb / nz), hi = (int)((long long)(z + 1) * nb / nz);
     const int n_it = KW > 1 ? (nb + nz - 1) / nz : hi - lo;
     const int last = hi > lo ? hi - 1 : (lo < nb ? lo : nb - 1);
-    out += (size_t)blockIdx.z * (size_t)split_stride;
 
     // this wave's columns: a uniform base and a lane's offset
     const int cb = c0 < n_cols ? c0 : n_cols - 1;
@@ -649,7 +646,7 @@ tf_gemm_kq_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
                 const int t = t0 + 32 * tt + 8 * (i >> 2) + 4 * h + (i & 3);
                 const float g = acc[0][tt][i];
                 if (t < n_tok)
-                    out[(size_t)t * n_cols + c] = (g / (1.f + __expf(-g))) * acc[1][tt][i];
+                    out[(size_t)t * ldo + c] = (g / (1.f + __expf(-g))) * acc[1][tt][i];
             }
         return;
     }
@@ -663,11 +660,65 @@ tf_gemm_kq_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
             for (int i = 0; i < 16; i++) {
                 const int t = t0 + 32 * tt + 8 * (i >> 2) + 4 * h + (i & 3);
                 if (t >= n_tok) continue;
-                float* o = out + (size_t)t * n_cols + c;
+                float* o = out + (size_t)t * ldo + c;
                 // accumulate: out += W x (the residual stream), one rounding
                 *o = accumulate ? *o + acc[ct][tt][i] : acc[ct][tt][i];
             }
     }
+}
+
+// XCD-aware tile order: workgroups go round-robin to the 8 XCDs, so XCD
+// k = blockIdx.x % 8 takes the contiguous tile range [k per, (k+1) per) (token
+// tiles fastest): a column tile's weights are fetched into one XCD's L2 and
+// reused there by all its token tiles.  false: a workgroup of the grid's padding.
+__device__ __forceinline__ bool tf_pg_tile(int ntx, int n_ct, int& tx, int& ct) {
+    const int n_tiles = ntx * n_ct;
+    const int per = (n_tiles + 7) >> 3;
+    const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    tx = tile % ntx;
+    ct = tile / ntx;
+    return tile < n_tiles;
+}
+
+// Waves per SIMD: 3 where the registers allow it (Q4_K without conversion
+// registers), else 2, or what four images of LDS (136 KB) leave room for.
+template <int FMT, int TT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false>
+__global__ __launch_bounds__(64 * CW * KW, KW * NBUF * TT >= 4 ? CW * KW / 4
+                                           : PRE && FMT == TF_PG_W4 && TT == 1 ? 3
+                                                                               : 2) void
+tf_gemm_kq_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
+                  const float* __restrict__ x, const uint8_t* __restrict__ ximg,
+                  float* __restrict__ out, int n_rows, int n_cols, int col_bytes, int n_tok,
+                  int accumulate, int n_split, long long split_stride) {
+    __shared__ __align__(16) uint8_t lds[KW * NBUF * TT * TF_PG_SLOT];
+    constexpr int COLS = (DUAL ? 32 : 64) * CW;
+    int tx, ct;
+    if (!tf_pg_tile((n_tok + 32 * TT - 1) / (32 * TT), (n_cols + COLS - 1) / COLS, tx, ct)) return;
+    tf_pg_body<FMT, TT, CW, KW, PRE, NBUF, DUAL>(
+        lds, w, w2, x, ximg, out + (size_t)blockIdx.z * (size_t)split_stride, n_cols, n_rows, n_cols,
+        col_bytes, n_tok, accumulate, n_split, tx * 32 * TT, ct);
+}
+
+// q, k and v of a prompt in one launch (their outputs side by side in rows of
+// ldo floats): the column tiles of the three matrices one after the other.
+__global__ __launch_bounds__(256, 2) void tf_pg_qkv_kernel(TfPgQkv m, const uint8_t* __restrict__ ximg,
+                                                           float* __restrict__ out, int ldo,
+                                                           int n_rows, int n_tok, int n_split,
+                                                           long long split_stride) {
+    __shared__ __align__(16) uint8_t lds[TF_PG_SLOT];
+    int tx, ct;
+    if (!tf_pg_tile((n_tok + 31) >> 5, m.ct[2], tx, ct)) return;
+    const int i = ct < m.ct[0] ? 0 : ct < m.ct[1] ? 1 : 2;
+    if (i) ct -= m.ct[i - 1];
+    float* o = out + (size_t)blockIdx.z * (size_t)split_stride + m.col[i];
+    auto go = [&](auto fmt) {
+        tf_pg_body<decltype(fmt)::value, 1, 4, 1, true, 1, false>(
+            lds, m.w[i], nullptr, nullptr, ximg, o, ldo, n_rows, m.n_cols[i], m.col_bytes[i], n_tok,
+            0, n_split, tx * 32, ct);
+    };
+    if (m.fmt[i] == TF_PG_W4) go(std::integral_constant<int, TF_PG_W4>{});
+    else if (m.fmt[i] == TF_PG_W6) go(std::integral_constant<int, TF_PG_W6>{});
+    else go(std::integral_constant<int, TF_PG_W6U>{});
 }
 
 // x[n_tok][n_rows] into images, [token tile of 32][super-block].
@@ -687,25 +738,125 @@ __global__ __launch_bounds__(256) void tf_pg_image_kernel(const float* __restric
     tf_pg_store_x<8, 4, true>(xr, img + ((size_t)blockIdx.y * gridDim.x + sb) * TF_PG_SLOT, st, ci);
 }
 
-// out[i] (+)= sum over z of part[z][i], z in order (split-K of the GEMM).
-__global__ __launch_bounds__(256) void tf_gemm_split_reduce_kernel(const float* __restrict__ part,
-                                                                   float* __restrict__ out,
-                                                                   long long n4, int n_split,
-                                                                   int accumulate) {
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+// x += the n_split slices of `part` (in order), then RMSNorm of the row and its
+// image: a workgroup per token, the row kept in LDS.  The sum of squares keeps
+// the reference's order (kernels/ops.cu:4-34: 256 strided fused sums, halving
+// tree).  Latency bound: a thread's loads are its n / 256 values of every
+// slice, all independent (a wave per token instead, four times the loads a
+// thread: 17 us at 20 tokens and 8 slices, 11.4 at 700 and 2).
+#define TF_PG_NORM_MAX 40448  // 158 KB of row
+__global__ __launch_bounds__(256) void tf_pg_norm_image_kernel(
+    float* __restrict__ x, const float* __restrict__ part, int n_split, long long split_stride,
+    const float* __restrict__ w, float eps, uint8_t* __restrict__ img, int n) {
+    extern __shared__ float row[];
+    __shared__ float red[1];
+    const int tid = threadIdx.x, t = blockIdx.x;
+    float* xr = x + (size_t)t * n;
+    const float* pr = part + (size_t)t * n;
+    float local = 0.f;
+#pragma unroll 4
+    for (int i = tid; i < n; i += 256) {
+        float v = xr[i];
+        if (n_split) {
+            float a = pr[i];
+#pragma unroll 4
+            for (int z = 1; z < n_split; z++) a += pr[(size_t)z * (size_t)split_stride + i];
+            v += a;
+            xr[i] = v;
+        }
+        row[i] = v;
+        local = fmaf(v, v, local);
+    }
+    // the halving tree over 256: 128 and 64 across the waves, the rest within one
+    __shared__ float buf[256];
+    buf[tid] = local;
+    __syncthreads();
+    if (tid < 64) {
+        float ss = (buf[tid] + buf[tid + 128]) + (buf[tid + 64] + buf[tid + 192]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) ss += __shfl_down(ss, o);
+        if (tid == 0) red[0] = 1.0f / sqrtf(ss / (float)n + eps);
+    }
+    __syncthreads();
+    const float scale = red[0];
+    const int ci = tid & 31, nb = n / 256;
+    for (int sb = tid >> 5; sb < nb; sb += 8) {  // uniform per half wave
+        const int k = 256 * sb + 8 * ci;
+        tf_pg_f4 v[1][2];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const tf_pg_f4 a = *reinterpret_cast<const tf_pg_f4*>(row + k + 4 * i);
+            const tf_pg_f4 g = *reinterpret_cast<const tf_pg_f4*>(w + k + 4 * i);
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[0][i][q] = a[q] * scale * g[q];
+        }
+        tf_pg_store_x<8, 1, true>(v, img + ((size_t)(t >> 5) * nb + sb) * TF_PG_SLOT, t & 31, ci);
+    }
+}
+
+// x[i] += sum over z of part[z][i], z in order.
+__global__ __launch_bounds__(256) void tf_pg_add_kernel(float* __restrict__ x,
+                                                        const float* __restrict__ part, int n4,
+                                                        int n_split, long long split_stride) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n4) return;
-    const float4* p = reinterpret_cast<const float4*>(part) + i;
-    float4 v = p[0];
+    float4 v = reinterpret_cast<const float4*>(part)[i];
+#pragma unroll 4
     for (int z = 1; z < n_split; z++) {
-        const float4 q = p[(size_t)z * (size_t)n4];
+        const float4 q = reinterpret_cast<const float4*>(part + (size_t)z * (size_t)split_stride)[i];
         v = make_float4(v.x + q.x, v.y + q.y, v.z + q.z, v.w + q.w);
     }
-    float4* o = reinterpret_cast<float4*>(out) + i;
-    if (accumulate) {
-        const float4 r = *o;
-        v = make_float4(r.x + v.x, r.y + v.y, r.z + v.z, r.w + v.w);
+    float4* o = reinterpret_cast<float4*>(x) + i;
+    const float4 r = *o;
+    *o = make_float4(r.x + v.x, r.y + v.y, r.z + v.z, r.w + v.w);
+}
+
+// q/k/v rows of token t (position pos0 + t) from the n_split slices of their
+// GEMM (columns q | k | v): the slices' sum and the bias, q and k rotated
+// (NeoX pairs (i, i + hd/2) by (pos0+t) theta^(-2i/hd)), q to q_out, k and v
+// to the f16 cache.  A workgroup per token; a thread keeps its pair index, and
+// with it the angle, over the heads it handles (hd / 2 divides 256).
+__global__ __launch_bounds__(256) void tf_pg_qkv_post_kernel(
+    const float* __restrict__ part, int n_split, long long split_stride,
+    const float* __restrict__ bq, const float* __restrict__ bk, const float* __restrict__ bv,
+    float* __restrict__ q_out, uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int n_head,
+    int n_kv, int hd, int pos0, float theta) {
+    const int t = blockIdx.x, pos = pos0 + t, half = hd / 2;
+    const int nq = n_head * hd, kvd = n_kv * hd, ld = nq + 2 * kvd;
+    const float* row = part + (size_t)t * ld;
+    const int i = threadIdx.x % half;
+    const float freq = powf(theta, -2.f * (float)i / (float)hd);
+    const float ang = (float)pos * freq;
+    float sn, cs;
+    sincosf(ang, &sn, &cs);
+    for (int hb = threadIdx.x / half; hb < n_head + 2 * n_kv; hb += 256 / half) {
+        const int c0 = hb * hd + i, c1 = c0 + half;
+        float x0 = row[c0], x1 = row[c1];
+#pragma unroll 4
+        for (int z = 1; z < n_split; z++) {
+            x0 += row[(size_t)z * (size_t)split_stride + c0];
+            x1 += row[(size_t)z * (size_t)split_stride + c1];
+        }
+        const float* b = hb < n_head ? bq : hb < n_head + n_kv ? bk : bv;
+        const int o = hb < n_head ? c0 : hb < n_head + n_kv ? c0 - nq : c0 - nq - kvd;
+        if (b) {
+            x0 += b[o];
+            x1 += b[o + half];
+        }
+        if (hb < n_head + n_kv) {
+            const float r0 = x0 * cs - x1 * sn, r1 = x0 * sn + x1 * cs;
+            x0 = r0;
+            x1 = r1;
+        }
+        if (hb < n_head) {
+            q_out[(size_t)t * nq + o] = x0;
+            q_out[(size_t)t * nq + o + half] = x1;
+        } else {
+            uint16_t* c = (hb < n_head + n_kv ? kc : vc) + (size_t)pos * kvd + o;
+            c[0] = tf_f2h_halfup(x0);
+            c[half] = tf_f2h_halfup(x1);
+        }
     }
-    *o = v;
 }
 
 // ------------------------------------------------------------------ launches
@@ -758,78 +909,188 @@ int tf_pg_check(bool q6, const uint8_t* w, const float* out, int n_rows, int n_c
     return 0;
 }
 
-// The GEMM on f32 rows: no memory besides the operands, so K is split only
-// inside a workgroup.  Three shapes of it (us at T tokens, Q4_K / Q6_K; each
-// line: waves as columns x K slices 1x4, 2x4 (Q6_K 2x2), 4x1):
-//   3584 x 3584 T 37     32 / -      33 / -      43 / -     (112 tiles of 64 columns)
-//   2048 x 5000 T 64      - / 21      - / 27      - / 35    (158)
-//   11008 x 2048 T 300    - / 175     - / 115     - / 176   (320; 80 of 256)
-//   11008 x 2048 T 512  168 / 188   102 / 137   133 / 176   (512; 128)
-//   2048 x 11008 T 256  111 / -      69 / -      48 / -     (1376; 344)
-//   2048 x 11008 T 512  219 / -     153 / -      71 / -     (2752; 688)
-// Four K slices need a CU's LDS, so 1x4 is taken while its tiles are at most
-// one a CU; 4x1 converts x once for 256 columns and is taken when its tiles
-// cover three quarters of the CUs; between the two, 128 columns and K split.
+// The GEMM on f32 rows.  There is no memory besides the operands, so K is
+// split only inside a workgroup: 256 columns a workgroup and K whole, or fewer
+// columns and K over two or four slices of its waves.  The first converts x
+// once for 256 columns and needs a third of a CU's LDS, the others (four
+// images) all of it.  A launch takes rounds x (a + b x super-blocks of a
+// slice), the rounds being the tiles over the CUs; a and b in us, fitted to
+// 256 CUs over 1..43 super-blocks, 77..11008 columns and 1..512 tokens:
+//                           Q4_K           Q6_K
+//   256 columns, K whole    2.8 + 3.0 n    4.4 + 3.7 n
+//   128 columns, K / 4      2.0 + 8.6 n    -
+//   128 columns, K / 2      -              6.5 + 4.9 n
+//   64 columns, K / 4       -              6.0 + 7.0 n
+// Measured at 300 tokens, 11008 -> 2048 (10 token tiles), Q6_K: 162, 113 and
+// 166 us in the order above; Q4_K 2048 -> 11008 at 512: 71 and 125; 1024 ->
+// 2048 at 100: 15.7 and 12.3.
 void tf_pg_f32(bool q6, const TfPgJob& j) {
     const size_t cus = (size_t)tf_device_cus();
-    if (q6 && ((uintptr_t)j.w & 2)) return tf_pg_go<TF_PG_W6U, 1, 2, 2, false, 2>(j);
-    if (tiles_of(j.n_tok, j.n_cols, 32, 64) <= cus) {
-        if (q6) tf_pg_go<TF_PG_W6, 1, 1, 4, false, 1>(j);
-        else tf_pg_go<TF_PG_W4, 1, 1, 4, false, 1>(j);
-    } else if (tiles_of(j.n_tok, j.n_cols, 32, 256) < cus * 3 / 4) {
-        if (q6) tf_pg_go<TF_PG_W6, 1, 2, 2, false, 2>(j);
-        else tf_pg_go<TF_PG_W4, 1, 2, 4, false, 1>(j);
+    const int nb = j.n_rows / 256;
+    auto cost = [&](int cols, int kw, float a, float b) {
+        const size_t rounds = (tiles_of(j.n_tok, j.n_cols, 32, cols) + cus - 1) / cus;
+        return (float)rounds * (a + b * (float)((nb + kw - 1) / kw));
+    };
+    if (!q6) {
+        if (cost(256, 1, 2.8f, 3.0f) <= cost(128, 4, 2.0f, 8.6f))
+            tf_pg_go<TF_PG_W4, 1, 4, 1, false, 1>(j);
+        else
+            tf_pg_go<TF_PG_W4, 1, 2, 4, false, 1>(j);
+        return;
+    }
+    const float whole = cost(256, 1, 4.4f, 3.7f), half = cost(128, 2, 6.5f, 4.9f),
+                quarter = cost(64, 4, 6.0f, 7.0f);
+    if ((uintptr_t)j.w & 2) {  // unaligned loads: the same order
+        if (whole <= half) tf_pg_go<TF_PG_W6U, 1, 4, 1, false, 1>(j);
+        else tf_pg_go<TF_PG_W6U, 1, 2, 2, false, 2>(j);
+    } else if (whole <= half && whole <= quarter) {
+        tf_pg_go<TF_PG_W6, 1, 4, 1, false, 1>(j);
+    } else if (half <= quarter) {
+        tf_pg_go<TF_PG_W6, 1, 2, 2, false, 2>(j);
     } else {
-        if (q6) tf_pg_go<TF_PG_W6, 1, 4, 1, false, 1>(j);
-        else tf_pg_go<TF_PG_W4, 1, 4, 1, false, 1>(j);
+        tf_pg_go<TF_PG_W6, 1, 1, 4, false, 1>(j);
     }
 }
 
 }  // namespace
 
-// (see prefill.hpp)
-int tf_gemm_kq(bool q6, const uint8_t* w, const float* x, float* out, int n_rows, int n_cols,
-               int col_bytes, int n_tok, int accumulate, tf_stream_t stream, float* ws,
-               size_t ws_floats) {
-    const int rc = tf_pg_check(q6, w, out, n_rows, n_cols, col_bytes, n_tok, q6 ? 210 : 144);
+size_t tf_pg_image_bytes(int n_rows, int n_tok) {
+    return (size_t)((n_tok + 31) / 32) * (size_t)(n_rows / 256) * TF_PG_SLOT;
+}
+
+int tf_pg_image(const float* x, uint8_t* img, int n_rows, int n_tok, tf_stream_t stream) {
+    TF_CHECK_ARG(x && img && n_rows >= 256 && n_tok > 0);
+    hipLaunchKernelGGL(tf_pg_image_kernel, dim3(n_rows / 256, (n_tok + 31) / 32), dim3(256), 0,
+                       tf_stream(stream), x, img, n_rows, n_tok);
+    return TF_LAUNCH_RESULT();
+}
+
+int tf_pg_norm_image(float* x, const TfPgPart* part, const float* w, float eps, uint8_t* img, int n,
+                     int n_tok, tf_stream_t stream) {
+    TF_CHECK_ARG(x && w && img && n >= 256 && n % 256 == 0 && n_tok > 0);
+    TF_CHECK_ARG(n <= TF_PG_NORM_MAX);
+    const int lds = n * (int)sizeof(float);
+    const int rc = tf_set_lds_limit((const void*)tf_pg_norm_image_kernel, lds);
     if (rc) return rc;
-    TF_CHECK_ARG(x && ((uintptr_t)x & 15) == 0);
-    TfPgJob j{w, nullptr, x, nullptr, out, n_rows, n_cols, col_bytes, n_tok, accumulate, 1,
+    hipLaunchKernelGGL(tf_pg_norm_image_kernel, dim3(n_tok), dim3(256), lds,
+                       tf_stream(stream), x, part ? part->p : nullptr, part ? part->n_split : 0,
+                       part ? part->stride : 0, w, eps, img, n);
+    return TF_LAUNCH_RESULT();
+}
+
+int tf_pg_add_row(float* x, const TfPgPart& part, int row, int n, tf_stream_t stream) {
+    TF_CHECK_ARG(x && part.p && part.n_split > 0 && n % 4 == 0);
+    hipLaunchKernelGGL(tf_pg_add_kernel, dim3((n / 4 + 255) / 256), dim3(256), 0, tf_stream(stream),
+                       x + (size_t)row * n, part.p + (size_t)row * n, n / 4, part.n_split,
+                       part.stride);
+    return TF_LAUNCH_RESULT();
+}
+
+// Slices of K for `tiles` output tiles: about 2.5 workgroups a CU in all, as
+// many as fit ws (a 700-token prompt of two 3B layers at 1, 1.5, 2, 2.5, 3, 4
+// a CU: 1190, 1096, 1137, 1095, 1096, 1104 us; 100 tokens: 524, 540, 541, 559,
+// 555, 563.  More slices shorten the GEMM and lengthen the kernel that adds
+// them; at 2, three slices of 176 tiles are one workgroup more than two a CU.)
+static int tf_pg_splits(size_t tiles, int nb, size_t slice, size_t ws_floats) {
+    const size_t target = 5 * (size_t)tf_device_cus() / 2;
+    int n = tiles >= target ? 1 : (int)((target + tiles / 2) / tiles);
+    n = std::max(1, std::min(n, std::min(nb, 16)));  // 16: what the adding kernel can hide
+    while (n > 1 && (size_t)n * slice > ws_floats) n--;
+    return n;
+}
+
+int tf_pg_gemm(const uint8_t* w, int block_bytes, const uint8_t* img, int n_rows, int n_cols,
+               int col_bytes, int n_tok, float* ws, size_t ws_floats, TfPgPart* part,
+               tf_stream_t stream) {
+    const bool q6 = block_bytes != 144;
+    const int rc = tf_pg_check(q6, w, ws, n_rows, n_cols, col_bytes, n_tok, block_bytes);
+    if (rc) return rc;
+    const size_t slice = (size_t)n_tok * n_cols;
+    TF_CHECK_ARG(img && slice <= ws_floats);
+    const int n_split = tf_pg_splits(tiles_of(n_tok, n_cols, 32, 256), n_rows / 256, slice, ws_floats);
+    *part = TfPgPart{ws, n_split, (long long)slice};
+    TfPgJob j{w, nullptr, nullptr, img, ws, n_rows, n_cols, col_bytes, n_tok, 0, n_split,
               tf_stream(stream)};
-    const size_t tiles = tiles_of(n_tok, n_cols, 32, 256), slice = (size_t)n_tok * n_cols;
-    const size_t target = 2 * (size_t)tf_device_cus();
-    if (!ws || tiles >= target * 3 / 4 || (n_cols & 3) || ((uintptr_t)ws & 15)) {
-        tf_pg_f32(q6, j);
-        return TF_LAUNCH_RESULT();
+    if (!q6) tf_pg_go<TF_PG_W4, 1, 4, 1, true, 1>(j);
+    else if (block_bytes == 212) tf_pg_go<TF_PG_W6C, 1, 4, 1, true, 1>(j);
+    else if ((uintptr_t)w & 2) tf_pg_go<TF_PG_W6U, 1, 4, 1, true, 1>(j);
+    else tf_pg_go<TF_PG_W6, 1, 4, 1, true, 1>(j);
+    return TF_LAUNCH_RESULT();
+}
+
+int tf_pg_qkv(const uint8_t* const w[3], const int block_bytes[3], const int n_cols[3],
+              const int col_bytes[3], const uint8_t* img, int n_rows, int n_tok, float* ws,
+              size_t ws_floats, TfPgPart* part, tf_stream_t stream) {
+    TfPgQkv m{};
+    int ct = 0, col = 0;
+    for (int i = 0; i < 3; i++) {
+        const bool q6 = block_bytes[i] != 144;
+        const int rc = tf_pg_check(q6, w[i], ws, n_rows, n_cols[i], col_bytes[i], n_tok, block_bytes[i]);
+        if (rc) return rc;
+        m.w[i] = w[i];
+        m.n_cols[i] = n_cols[i];
+        m.col_bytes[i] = col_bytes[i];
+        m.fmt[i] = !q6 ? TF_PG_W4 : (uintptr_t)w[i] & 2 ? TF_PG_W6U : TF_PG_W6;
+        m.col[i] = col;
+        col += n_cols[i];
+        m.ct[i] = ct += (n_cols[i] + 255) / 256;
     }
-    // Split-K when the tile grid leaves the chip short of workgroups: about two
-    // a CU in all, partial slices into ws, then a fixed-order sum.
-    j.n_split = (int)((target + tiles - 1) / tiles);
-    if (j.n_split > n_rows / 256) j.n_split = n_rows / 256;
-    while (j.n_split > 1 && (size_t)j.n_split * slice > ws_floats) j.n_split--;
-    if (j.n_split > 1) {
-        j.out = ws;
-        j.accumulate = 0;
-    }
-    if (!q6) tf_pg_go<TF_PG_W4, 1, 4, 1, false, 1>(j);
-    else if ((uintptr_t)w & 2) tf_pg_go<TF_PG_W6U, 1, 4, 1, false, 1>(j);
-    else tf_pg_go<TF_PG_W6, 1, 4, 1, false, 1>(j);
-    if (j.n_split > 1) {
-        const long long n4 = (long long)(slice / 4);
-        hipLaunchKernelGGL(tf_gemm_split_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)),
-                           dim3(256), 0, tf_stream(stream), ws, out, n4, j.n_split, accumulate);
-    }
+    const size_t slice = (size_t)n_tok * col, tiles = (size_t)((n_tok + 31) / 32) * ct;
+    TF_CHECK_ARG(img && slice <= ws_floats);
+    const int n_split = tf_pg_splits(tiles, n_rows / 256, slice, ws_floats);
+    *part = TfPgPart{ws, n_split, (long long)slice};
+    hipLaunchKernelGGL(tf_pg_qkv_kernel, dim3((unsigned)(8 * ((tiles + 7) / 8)), 1, n_split),
+                       dim3(256), 0, tf_stream(stream), m, img, ws, col, n_rows, n_tok, n_split,
+                       (long long)slice);
+    return TF_LAUNCH_RESULT();
+}
+
+int tf_pg_qkv_post(const TfPgPart& part, const float* bq, const float* bk, const float* bv,
+                   float* q_out, uint16_t* k_cache, uint16_t* v_cache, int n_head, int n_kv,
+                   int head_dim, int pos0, int n_tok, float theta, tf_stream_t stream) {
+    TF_CHECK_ARG(part.p && q_out && k_cache && v_cache && n_head > 0 && n_kv > 0 && n_tok > 0);
+    TF_CHECK_ARG(head_dim > 0 && head_dim % 2 == 0 && 256 % (head_dim / 2) == 0 && pos0 >= 0);
+    hipLaunchKernelGGL(tf_pg_qkv_post_kernel, dim3(n_tok), dim3(256), 0, tf_stream(stream), part.p,
+                       part.n_split, part.stride, bq, bk, bv, q_out, k_cache, v_cache, n_head, n_kv,
+                       head_dim, pos0, theta);
+    return TF_LAUNCH_RESULT();
+}
+
+int tf_pg_gate_up(const uint8_t* gate, const uint8_t* up, const uint8_t* img, float* out,
+                  int n_rows, int n_cols, int col_bytes, int n_tok, tf_stream_t stream) {
+    int rc = tf_pg_check(false, gate, out, n_rows, n_cols, col_bytes, n_tok, 144);
+    if (!rc) rc = tf_pg_check(false, up, out, n_rows, n_cols, col_bytes, n_tok, 144);
+    if (rc) return rc;
+    TF_CHECK_ARG(img);
+    const TfPgJob j{gate, up, nullptr, img, out, n_rows, n_cols, col_bytes, n_tok, 0, 1,
+                    tf_stream(stream)};
+    // a short prompt: half the columns a workgroup and K split over its waves
+    // (2048 -> 2 x 11008 at 20 tokens, 86 workgroups: 31 us)
+    if (tiles_of(n_tok, n_cols, 32, 128) < (size_t)tf_device_cus() * 3 / 4)
+        tf_pg_go<TF_PG_W4, 1, 2, 4, true, 1, true>(j);
+    else
+        tf_pg_go<TF_PG_W4, 1, 4, 1, true, 1, true>(j);
     return TF_LAUNCH_RESULT();
 }
 
 // ---------------------------------------------------------------- C ABI
 
+static int tf_gemm_f32(bool q6, const uint8_t* w, const float* x, float* out, int n_rows,
+                       int n_cols, int col_bytes, int n_tok, tf_stream_t stream) {
+    const int rc = tf_pg_check(q6, w, out, n_rows, n_cols, col_bytes, n_tok, q6 ? 210 : 144);
+    if (rc) return rc;
+    TF_CHECK_ARG(x && ((uintptr_t)x & 15) == 0);
+    tf_pg_f32(q6, TfPgJob{w, nullptr, x, nullptr, out, n_rows, n_cols, col_bytes, n_tok, 0, 1,
+                          tf_stream(stream)});
+    return TF_LAUNCH_RESULT();
+}
+
 extern "C" int tf_gemm_q4k_f32(const uint8_t* w, const float* x, float* out, int n_rows,
                                int n_cols, int col_bytes, int n_tok, tf_stream_t stream) {
-    return tf_gemm_kq(false, w, x, out, n_rows, n_cols, col_bytes, n_tok, 0, stream, nullptr, 0);
+    return tf_gemm_f32(false, w, x, out, n_rows, n_cols, col_bytes, n_tok, stream);
 }
 
 extern "C" int tf_gemm_q6k_f32(const uint8_t* w, const float* x, float* out, int n_rows,
                                int n_cols, int col_bytes, int n_tok, tf_stream_t stream) {
-    return tf_gemm_kq(true, w, x, out, n_rows, n_cols, col_bytes, n_tok, 0, stream, nullptr, 0);
+    return tf_gemm_f32(true, w, x, out, n_rows, n_cols, col_bytes, n_tok, stream);
 }

@@ -4,9 +4,10 @@ fp64 product with numpy-dequantized weights (tests/_util.gemm_ref), within the
 fp32 GEMV tolerance (1e-5 relative, floor 0.1 * sum |terms|): the split of x
 keeps 22 bits of each value, 2^-23 of a term, and the rest is fp32 summation.
 
-The token tile is 32, a wave's columns 64; the dispatch goes by the number of
-32 x 64 and 32 x 256 output tiles, the Q6_K loads by where a column starts
-modulo 4 (an odd number of 210-byte blocks makes it alternate).
+The token tile is 32, a wave's columns 64; the dispatch weighs 256 columns a
+workgroup with K whole against fewer columns with K split over its waves, by
+the number of output tiles and of super-blocks; the Q6_K loads go by where a
+column starts modulo 4 (an odd number of 210-byte blocks makes it alternate).
 """
 import numpy as np
 import pytest
@@ -38,13 +39,13 @@ def run(fmt, n_rows, n_cols, x, shift=0, seed=0):
 
 @pytest.mark.parametrize("fmt", ["q4k", "q6k"])
 @pytest.mark.parametrize("n_rows,n_cols,n_tok", [
-    (256, 1, 1),        # one value; most K slices empty
+    (256, 1, 1),        # one value
     (768, 63, 31),      # 3 super-blocks over 4 slices, one short of a tile each way
     (768, 65, 33),      # one past a tile
-    (1280, 129, 32),    # 5 super-blocks
-    (512, 4100, 130),   # 128 columns and K split: 325 tiles of 64 columns
-    (1792, 3200, 200),  # the same with 7 super-blocks
-    (256, 8200, 190),   # 256 columns: 198 tiles, ragged both ways
+    (1280, 129, 32),    # 5 super-blocks over 4 slices (Q6_K)
+    (512, 4100, 130),   # 128 columns, K over 2 slices (Q6_K)
+    (1792, 3200, 200),  # 7 super-blocks over 4 (Q4_K) and 2 (Q6_K) slices
+    (256, 8200, 190),   # 256 columns, ragged both ways
     (768, 6145, 260),
 ])
 def test_gemm_tiles(gpu, fmt, n_rows, n_cols, n_tok):
