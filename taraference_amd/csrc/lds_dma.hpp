@@ -27,6 +27,35 @@ __device__ __forceinline__ void tf_lds_dma16(const void* src, uint32_t lds_off) 
         : "memory");
 }
 
+// The same from a wave-uniform base plus a 32-bit offset of the lane; W = 4
+// moves 4 bytes a lane (256 a copy), for sources that are only 4-byte aligned.
+template <int W>
+__device__ __forceinline__ void tf_lds_dma_s(const void* base, uint32_t off, uint32_t lds_off) {
+    static_assert(W == 4 || W == 16, "bytes a lane");
+    const uint32_t la = __builtin_amdgcn_readfirstlane(lds_off);
+    uint32_t saved;
+    if constexpr (W == 16)
+        asm volatile(
+            "s_mov_b32 %0, m0\n\t"
+            "s_mov_b32 m0, %1\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %2, %3\n\t"
+            "s_mov_b32 m0, %0"
+            : "=&s"(saved)
+            : "s"(la), "v"(off), "s"(base)
+            : "memory");
+    else
+        asm volatile(
+            "s_mov_b32 %0, m0\n\t"
+            "s_mov_b32 m0, %1\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dword %2, %3\n\t"
+            "s_mov_b32 m0, %0"
+            : "=&s"(saved)
+            : "s"(la), "v"(off), "s"(base)
+            : "memory");
+}
+
 // LDS byte offset of a pointer into LDS.
 __device__ __forceinline__ uint32_t tf_lds_off(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;

@@ -3,6 +3,7 @@
 //
 // Replaces kernels/attn/fast_v2.cu attn_fast_v2 / attn_fast_v2_d (:12, :103).
 #include "dequant.hpp"
+#include "lds_dma.hpp"
 #include "prefill.hpp"
 #include "tf_common.hpp"
 #include "tf_host.hpp"
@@ -13,10 +14,10 @@ typedef _Float16 tf_h8 __attribute__((ext_vector_type(8)));
 // ---------------------------------------------------------------- attention
 //
 // Causal attention of n_q queries (positions pos0 .. pos0+n_q-1) over the
-// f16 cache, fp32 arithmetic.  A workgroup (256 threads) owns one head and
-// 16 consecutive queries; K/V tiles of T keys (64, 32, 16 for head_dim 64,
-// 128, 256: about 45 KB of LDS) are staged in LDS as f32 and shared by the
-// 16 queries.  Thread (query qi = tid / 16, m = tid % 16): scores of keys
+// f16 cache; head_dim 256 in fp32 vector arithmetic, 64 and 128 on the matrix
+// cores (below).  A workgroup (256 threads) owns one head and 16 consecutive
+// queries; K/V tiles of 16 keys (about 45 KB of LDS) are staged in LDS as f32
+// and shared by the 16 queries.  Thread (query qi = tid / 16, m = tid % 16): scores of keys
 // m, m+16, ... of the tile (a DPP row holds one query, so the row max and
 // sum are row reductions), then output dims DPT m .. DPT m + DPT-1 with
 // DPT = head_dim / 16.  Online softmax as
@@ -25,14 +26,14 @@ typedef _Float16 tf_h8 __attribute__((ext_vector_type(8)));
 
 #define TF_PA_Q 16
 
-template <int HD>
 __global__ __launch_bounds__(256) void tf_attn_prefill_kernel(
     const float* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     float* __restrict__ out, int n_head, int n_kv, int pos0_arg, const int* __restrict__ pos0_ptr,
     int n_q, float scale) {
-    constexpr int DPT = HD / 16;  // output dims per thread
-    constexpr int TF_PA_T = HD == 64 ? 64 : (HD == 128 ? 32 : 16);  // keys per tile
-    constexpr int NS = TF_PA_T / 16;                                // scores per thread
+    constexpr int HD = 256;
+    constexpr int DPT = HD / 16;      // output dims per thread
+    constexpr int TF_PA_T = 16;       // keys per tile
+    constexpr int NS = TF_PA_T / 16;  // scores per thread
     __shared__ __align__(16) float qs[TF_PA_Q * (HD + 4)];
     __shared__ __align__(16) float ks[TF_PA_T * (HD + 4)];
     __shared__ __align__(16) float vs[TF_PA_T * HD];
@@ -131,203 +132,316 @@ __global__ __launch_bounds__(256) void tf_attn_prefill_kernel(
     }
 }
 
-// Matrix-core form for head_dim 128.  A workgroup (4 waves) owns one head
-// and 16 queries; the waves split the 32-key tiles round-robin, each staging
-// its own tiles in LDS, and merge their (m, l, O) with the log-sum-exp rule
-// at the end (a wave with no keys for a query contributes e^(-1e30 - M) = 0).
-// Per tile, on v_mfma_f32_16x16x32_f16:
-//   S^T = K q^T: A = K rows (A row i of key block b is key
-//       8 (i / 4) + 4 b + i % 4, so the C values a lane holds, key rows
-//       4g .. 4g+3 of blocks 0 and 1, are the tile's keys 8g .. 8g+7), B =
-//       q^T, q split into two f16 parts after a power-of-two scale (2^-22
-//       relative per product; K is f16, the products are exact);
-//   O += P V: A = P (query l16, keys 8g .. 8g+7: the lane's own S values
-//       after the softmax, split into two f16 parts), B = V gathered from
-//       the row-major f16 tile (8 u16 reads per fragment).
-// Softmax per query: the lane's 8 values, then the 4 lanes of the query
-// (xor 16, 32).  Keys past the workgroup's last query are staged as zeros.
+// Matrix-core form for head_dim 64 and 128.  The rows of a kv head are its
+// (query, head) pairs, heads fastest: row r is query r / G, head r % G of the
+// group (G = n_head / n_kv).  A workgroup owns 32 rows, so each K/V byte it
+// reads serves 32 rows whatever the group or the prompt length, and its eight
+// waves share the 32-key tiles round-robin, each with its own LDS tile pair and
+// its own (m, l, O); the eight are merged with the log-sum-exp rule at the end.
+// Rows are split this finely because a prompt has few of them (512 tokens of 16
+// heads over 2 kv heads: 256 workgroups, one a CU); the waves take keys, not
+// rows, so that they never wait for each other while streaming.
+//
+// K and V move HBM / L2 -> LDS without registers (global_load_lds), one tile
+// ahead: the next K tile is requested when the scores of this one are formed
+// and arrives under the softmax and P V, the next V tile when P V is done and
+// arrives under the next scores.  Copies complete in issue order, so vmcnt(one
+// tile's copies) waits for exactly the older tile.
+//
+// Per tile, on v_mfma_f32_32x32x16_f16 (lane l, h = l / 32: A[l % 32][8h ..],
+// B[8h ..][l % 32], C[8 (i / 4) + 4 h + i % 4][l % 32]):
+//   S^T[key][row] = K q^T, q in two f16 parts after a power-of-two scale per
+//       row (2^-22 relative per product; K is f16, the products are exact);
+//   softmax over the lane's 16 keys and the other half's 16 (one exchange), in
+//       powers of two; O is rescaled only where a row's maximum moved;
+//   O^T[dim][row] += V^T P^T with P in two f16 parts (2^-22): k index i of half
+//       h in step s stands for key 16 s + 8 (i / 4) + 4 h + i % 4, which is how
+//       the scores already lie, so P needs no exchange; the V operand is two
+//       transposing LDS reads (ds_read_b64_tr_b16: four keys of a lane's dim).
+// LDS rows keep their 16-byte chunks xor-ed with the row, so that 16 K rows, or
+// the 4 rows x 64 bytes of a transposing read, fall on distinct banks.
+// What bounds it: the matrix cores, at two products per score and per P V term
+// (256 tokens of 28 heads at 8000: 30 GF, 60 GF of f16 products, 77 us), the
+// softmax's vector work beside them; the form before it (16 queries of one head,
+// keys staged through registers, V gathered two bytes at a time) took 234 us, and
+// 19.3 against 13.2 us for a fresh 512-token prompt of 16 heads.  Error against
+// 64 bits 5.6e-7 and 2.5e-7, before 6.8e-7 and 2.7e-7.
+#define TF_PM_WAVES 8
+#define TF_PM_T 32  // keys per tile, rows per workgroup
 
-#define TF_PM_T 32              // keys per tile
-#define TF_PM_KROW 272          // K tile row bytes (128 f16 + 16)
-#define TF_PM_VROW 264          // V tile row bytes (128 f16 + 8): 8-row gathers on distinct banks
-#define TF_PM_WAVE_BYTES (TF_PM_T * TF_PM_KROW + TF_PM_T * TF_PM_VROW)
+template <int HD>
+struct TfPmLds {
+    static constexpr int ROWB = 2 * HD;                // K / V row bytes
+    static constexpr int TILE = TF_PM_T * ROWB;        // a K or V tile
+    static constexpr int OROW = HD + 4;                // floats of a merge row
+    static constexpr int WAVE = TF_PM_T * OROW * 4;    // the K + V tiles, then the wave's O
+    static constexpr int ML = TF_PM_WAVES * WAVE;      // m, l: [2][waves][32]
+    static constexpr int BYTES = ML + 2 * TF_PM_WAVES * TF_PM_T * 4;
+    static_assert(2 * TILE <= WAVE, "the tiles fit where O goes");
+};
 
-__global__ __launch_bounds__(256) void tf_attn_prefill_mfma_kernel(
+typedef float tf_f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 tf_h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 tf_h4 __attribute__((ext_vector_type(4)));
+typedef short tf_s4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) uint8_t tf_lds_u8;
+
+template <int N>
+__device__ __forceinline__ void tf_wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// e = hi + lo in f16 parts, two values at a time
+__device__ __forceinline__ void tf_split2(float a, float b, tf_h2& hi, tf_h2& lo) {
+    hi = tf_h2{(_Float16)a, (_Float16)b};
+    lo = tf_h2{(_Float16)(a - (float)hi.x), (_Float16)(b - (float)hi.y)};
+}
+
+// r / d by the reciprocal m = ceil(2^32 / d) (0 for d = 1): the product is at
+// most one too large
+__device__ __forceinline__ uint32_t tf_div_by(uint32_t r, uint32_t d, uint32_t m) {
+    if (m == 0) return r;
+    const uint32_t t = __umulhi(r, m);
+    return t * d > r ? t - 1 : t;
+}
+
+// DW: bytes a lane copies (16; 4 where the caches are only 8-byte aligned)
+template <int HD, int DW>
+__global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kernel(
     const float* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     float* __restrict__ out, int n_head, int n_kv, int pos0_arg, const int* __restrict__ pos0_ptr,
-    int n_q, float scale) {
-    constexpr int HD = 128;
-    __shared__ __align__(16) uint8_t lds[4 * TF_PM_WAVE_BYTES];
-    __shared__ float ml[2][4][16];
+    int n_rows, int G, uint32_t g_inv, uint32_t kv_inv, float scale) {
+    using L = TfPmLds<HD>;
+    constexpr int ROWB = L::ROWB, ST = HD / 16, DB = HD / 32;
+    constexpr int NC = L::TILE / (64 * DW);  // copies of a tile
+    extern __shared__ __align__(16) uint8_t lds[];
     const int pos0 = pos0_ptr ? pos0_ptr[0] : pos0_arg;
-    const int h = blockIdx.y, q0 = blockIdx.x * 16;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 4, l16 = lane & 15;
-    const int kv_h = h / (n_head / n_kv), stride = n_kv * HD;
-    const int last_q = (q0 + 16 < n_q ? q0 + 16 : n_q) - 1;
-    const int kv_len = pos0 + last_q + 1;  // keys the workgroup reads
+    // kv heads fastest (workgroups of one kv head share few XCDs' L2), the
+    // rows with the most keys first
+    const int rb = tf_div_by(gridDim.x - 1 - blockIdx.x, n_kv, kv_inv);
+    const int kv_h = (gridDim.x - 1 - blockIdx.x) - rb * n_kv, r0 = rb * TF_PM_T;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, l32 = lane & 31;
+    const int rl = (r0 + TF_PM_T < n_rows ? r0 + TF_PM_T : n_rows) - 1;
+    const int kv_len = pos0 + (int)tf_div_by(rl, G, g_inv) + 1;  // keys the workgroup reads
+    const int first_pos = pos0 + (int)tf_div_by(r0, G, g_inv);   // every row sees keys up to here
     const int n_t = (kv_len + TF_PM_T - 1) / TF_PM_T;
-    uint8_t* kt = lds + wave * TF_PM_WAVE_BYTES;
-    uint8_t* vt = kt + TF_PM_T * TF_PM_KROW;
+    const uint32_t row_bytes = (uint32_t)n_kv * ROWB;
+    const uint8_t* kbase = reinterpret_cast<const uint8_t*>(kc) + (size_t)kv_h * ROWB;
+    const uint8_t* vbase = reinterpret_cast<const uint8_t*>(vc) + (size_t)kv_h * ROWB;
+    uint8_t* kt = lds + wave * L::WAVE;
+    uint8_t* vt = kt + L::TILE;
 
-    // q^T fragments: query l16, dims 32 st + 8 g .. +7, two f16 parts
-    const int my_q = q0 + l16 < n_q ? q0 + l16 : last_q;
-    const int qpos = pos0 + my_q;
-    float qv[32];
-    {
-        const float* qr = q + (size_t)my_q * n_head * HD + (size_t)h * HD;
+    // the row of this lane
+    const int row = r0 + l32 < n_rows ? r0 + l32 : rl;
+    const int qi = tf_div_by(row, G, g_inv);
+    const int qpos = pos0 + qi;
+
+    // copy i of a tile: byte p = 64 DW i + DW lane of it, row p / ROWB; rows past
+    // the last key repeat it (their scores are masked)
+    auto issue = [&](const uint8_t* base, uint8_t* dst, int t0, bool is_v) {
+        const uint8_t* tb = base + (size_t)t0 * row_bytes;
+        const uint32_t ldst = tf_lds_off(dst);
+        const int rmax = kv_len - 1 - t0;
+        auto off = [&](int i, int last) -> uint32_t {
+            const int p = 64 * DW * i + DW * lane, r = p / ROWB;
+            const int c = (p % ROWB) >> 4;
+            const int sw = is_v ? (HD == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1))
+                                : (HD == 128 ? r & 15 : (r >> 1) & 7);
+            return (uint32_t)(r < last ? r : last) * row_bytes + 16 * (c ^ sw) + (p & 15);
+        };
+        if (rmax >= TF_PM_T - 1) {
 #pragma unroll
-        for (int st = 0; st < 4; st++) {
-            const float4 a = *reinterpret_cast<const float4*>(qr + 32 * st + 8 * g);
-            const float4 b = *reinterpret_cast<const float4*>(qr + 32 * st + 8 * g + 4);
-            qv[8 * st] = a.x; qv[8 * st + 1] = a.y; qv[8 * st + 2] = a.z; qv[8 * st + 3] = a.w;
-            qv[8 * st + 4] = b.x; qv[8 * st + 5] = b.y; qv[8 * st + 6] = b.z; qv[8 * st + 7] = b.w;
+            for (int i = 0; i < NC; i++)
+                tf_lds_dma_s<DW>(tb, off(i, TF_PM_T), ldst + 64 * DW * i);
+        } else {
+#pragma unroll 1
+            for (int i = 0; i < NC; i++)
+                tf_lds_dma_s<DW>(tb, off(i, rmax), ldst + 64 * DW * i);
         }
+    };
+    float s2 = 0.f;  // score in powers of two = product * s2
+    tf_h8 qb[ST][2];
+    if (wave < n_t) {
+        const float* qr = q + ((size_t)qi * n_head + (size_t)kv_h * G + (row - qi * G)) * HD;
+        float qv[ST][8];
+#pragma unroll
+        for (int st = 0; st < ST; st++) {
+            const float4 a = *reinterpret_cast<const float4*>(qr + 16 * st + 8 * h);
+            const float4 b = *reinterpret_cast<const float4*>(qr + 16 * st + 8 * h + 4);
+            qv[st][0] = a.x; qv[st][1] = a.y; qv[st][2] = a.z; qv[st][3] = a.w;
+            qv[st][4] = b.x; qv[st][5] = b.y; qv[st][6] = b.z; qv[st][7] = b.w;
+        }
+        issue(kbase, kt, wave * TF_PM_T, false);
+        issue(vbase, vt, wave * TF_PM_T, true);
+
+        // q^T fragments: dims 16 st + 8 h .. +7 of the row in two f16 parts, after a
+        // power of two that takes the row's largest value to [2^14, 2^15) and with
+        // the sign of the scale, so that the largest score has the largest product
+        float amax = 0.f;
+#pragma unroll
+        for (int st = 0; st < ST; st++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(qv[st][i]));
+        amax = fmaxf(amax, __shfl_xor(amax, 32));
+        const int eb = (int)((__float_as_uint(amax) >> 23) & 0xff);
+        int fe = amax > 0.f ? 141 - eb : 0;
+        fe = fe > 126 ? 126 : fe;
+        const float f = copysignf(__uint_as_float((uint32_t)(fe + 127) << 23), scale);
+        s2 = fabsf(scale) * 1.44269504088896340736f * __uint_as_float((uint32_t)(127 - fe) << 23);
+#pragma unroll
+        for (int st = 0; st < ST; st++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float a = qv[st][i] * f;
+                const _Float16 hi = (_Float16)a;
+                qb[st][0][i] = hi;
+                qb[st][1][i] = (_Float16)(a - (float)hi);
+            }
     }
-    float amax = 0.f;
-#pragma unroll
-    for (int i = 0; i < 32; i++) amax = fmaxf(amax, fabsf(qv[i]));
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
-    const int eb = (int)((__float_as_uint(amax) >> 23) & 0xff);
-    int fe = amax > 0.f ? 141 - eb : 0;
-    fe = fe > 126 ? 126 : fe;
-    const float f = __uint_as_float((uint32_t)(fe + 127) << 23);
-    const float sscale = scale * __uint_as_float((uint32_t)(127 - fe) << 23);
-    tf_h8 qb[4][2];
-#pragma unroll
-    for (int st = 0; st < 4; st++)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float a = qv[8 * st + i] * f;
-            const _Float16 hi = (_Float16)a;
-            qb[st][0][i] = hi;
-            qb[st][1][i] = (_Float16)(a - (float)hi);
-        }
 
-    float mx = -1e30f, l = 0.f;
-    tf_f32x4 o[8];
+    float mx = -1e30f, l = 0.f;  // of the row; l is this half's share
+    tf_f32x16 o[DB];
 #pragma unroll
-    for (int nb = 0; nb < 8; nb++) o[nb] = tf_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[db][i] = 0.f;
+    const int ksw = HD == 128 ? l32 & 15 : (l32 >> 1) & 7;
+    // transposing read: lane 4 a + b of 16 fetches 8 bytes of key a, dims 4 b ..,
+    // and receives keys 0 .. 3 of dim 4 a + b; lanes 16 .. 31 take dims 16 ..
+    const int ta = (lane & 15) >> 2, tb4 = lane & 3;
+    const int vsw = HD == 128 ? ta : (ta >> 1);
+    const int vrow = (4 * h + ta) * ROWB + 16 * (2 * ((lane >> 4) & 1) + (tb4 >> 1)) + 8 * (tb4 & 1);
 
-    for (int ti = wave; ti < n_t; ti += 4) {
-        const int t0 = ti * TF_PM_T;
-        // stage K and V rows t0 .. t0+31 (zeros past kv_len)
+    for (int j = wave; j < n_t; j += TF_PM_WAVES) {
+        const int t0 = j * TF_PM_T;
+        const bool more = j + TF_PM_WAVES < n_t;
+        tf_wait_vm<NC>();  // K of tile j is there, V still on its way
+        tf_f32x16 sc;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int idx = lane + 64 * j, r = idx >> 4, c = idx & 15;
-            tf_u32x4 kb = {0, 0, 0, 0}, vb = {0, 0, 0, 0};
-            if (t0 + r < kv_len) {
-                const size_t off = (size_t)(t0 + r) * stride + (size_t)kv_h * HD + 8 * c;
-                kb = *reinterpret_cast<const tf_u32x4*>(kc + off);
-                vb = *reinterpret_cast<const tf_u32x4*>(vc + off);
-            }
-            *reinterpret_cast<tf_u32x4*>(kt + r * TF_PM_KROW + 16 * c) = kb;
-            uint32_t* vw = reinterpret_cast<uint32_t*>(vt + r * TF_PM_VROW + 16 * c);
-            vw[0] = vb.x; vw[1] = vb.y; vw[2] = vb.z; vw[3] = vb.w;  // 8-byte aligned rows
+        for (int i = 0; i < 16; i++) sc[i] = 0.f;
+#pragma unroll
+        for (int st = 0; st < ST; st++) {
+            const tf_h8 ka = *reinterpret_cast<const tf_h8*>(kt + l32 * ROWB + 16 * ((2 * st + h) ^ ksw));
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qb[st][0], sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qb[st][1], sc, 0, 0, 0);
         }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // LDS stores of the wave done (lgkmcnt 0)
-        __builtin_amdgcn_wave_barrier();
-        // S^T: two key blocks, 4 K steps, 2 parts
-        tf_f32x4 sc[2];
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const int key = 8 * (l16 >> 2) + 4 * b + (l16 & 3);
-            tf_f32x4 c = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int st = 0; st < 4; st++) {
-                const tf_h8 ka = *reinterpret_cast<const tf_h8*>(kt + key * TF_PM_KROW +
-                                                                 2 * (32 * st + 8 * g));
-                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qb[st][0], c, 0, 0, 0);
-                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qb[st][1], c, 0, 0, 0);
-            }
-            sc[b] = c;
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the K tile has been read
+            issue(kbase, kt, t0 + TF_PM_WAVES * TF_PM_T, false);
         }
-        // lane values: keys t0 + 8g + 4b + r of query my_q
-        float sv[8];
-        float tmax = -1e30f;
+        // the lane's keys: t0 + 8 (i / 4) + 4 h + i % 4
+        const bool edge = t0 + TF_PM_T - 1 > first_pos;
+        if (edge) {
 #pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int kp = t0 + 8 * g + 4 * b + r;
-                const float v = kp <= qpos ? sc[b][r] * sscale : -1e30f;
-                sv[4 * b + r] = v;
-                tmax = fmaxf(tmax, v);
+            for (int i = 0; i < 16; i++) {
+                const int kp = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
+                sc[i] = kp <= qpos ? sc[i] : -INFINITY;
             }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
+        }
+        float tmax = sc[0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) tmax = fmaxf(tmax, sc[i]);
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float m_new = fmaxf(mx, tmax);
-        const float alpha = __expf(mx - m_new);
+        const float m_new = fmaxf(mx, tmax * s2);
+        if (__ballot(m_new > mx)) {
+            const float alpha = __builtin_amdgcn_exp2f(mx - m_new);
+            l *= alpha;
+#pragma unroll
+            for (int db = 0; db < DB; db++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) o[db][i] *= alpha;
+            mx = m_new;
+        }
+        tf_h8 pa[2][2];
         float ls = 0.f;
-        tf_h8 pa[2];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float e = sv[i] > -1e29f ? __expf(sv[i] - m_new) : 0.f;
-            ls += e;
-            const _Float16 hi = (_Float16)e;
-            pa[0][i] = hi;
-            pa[1][i] = (_Float16)(e - (float)hi);
+        for (int i = 0; i < 16; i += 2) {
+            // a NaN score counts as no key
+            const float e0 = fmaxf(__builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], s2, -mx)), 0.f);
+            const float e1 = fmaxf(__builtin_amdgcn_exp2f(__builtin_fmaf(sc[i + 1], s2, -mx)), 0.f);
+            ls += e0 + e1;
+            tf_h2 hi, lo;
+            tf_split2(e0, e1, hi, lo);
+            pa[i >> 3][0][i & 7] = hi.x;
+            pa[i >> 3][0][(i & 7) + 1] = hi.y;
+            pa[i >> 3][1][i & 7] = lo.x;
+            pa[i >> 3][1][(i & 7) + 1] = lo.y;
         }
-        ls += __shfl_xor(ls, 16);
-        ls += __shfl_xor(ls, 32);
-        l = l * alpha + ls;
-        mx = m_new;
-        // O rows are queries 4g .. 4g+3: their alpha from lanes 4g + r
-        float al[4];
+        l += ls;
+        if (more) tf_wait_vm<NC>();  // V of tile j
+        else tf_wait_vm<0>();
 #pragma unroll
-        for (int r = 0; r < 4; r++) al[r] = __shfl(alpha, 4 * g + r);
+        for (int s = 0; s < 2; s++)
 #pragma unroll
-        for (int nb = 0; nb < 8; nb++) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) o[nb][r] *= al[r];
-            // V fragment: keys 8g .. 8g+7, dim 16 nb + l16
-            const uint8_t* vp = vt + (8 * g) * TF_PM_VROW + 2 * (16 * nb + l16);
-            tf_h8 vf;
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                vf[i] = __builtin_bit_cast(_Float16, *reinterpret_cast<const uint16_t*>(vp + i * TF_PM_VROW));
-            o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[0], vf, o[nb], 0, 0, 0);
-            o[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[1], vf, o[nb], 0, 0, 0);
+            for (int db = 0; db < DB; db++) {
+                const tf_lds_u8* vp = (const tf_lds_u8*)(vt + vrow + 16 * s * ROWB + 64 * (db ^ vsw));
+                const tf_h4 v0 = __builtin_bit_cast(
+                    tf_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                               (__attribute__((address_space(3))) tf_s4*)vp));
+                const tf_h4 v1 = __builtin_bit_cast(
+                    tf_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                               (__attribute__((address_space(3))) tf_s4*)(vp + 8 * ROWB)));
+                const tf_h8 vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pa[s][0], o[db], 0, 0, 0);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pa[s][1], o[db], 0, 0, 0);
+            }
+        if (more) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the V tile has been read
+            issue(vbase, vt, t0 + TF_PM_WAVES * TF_PM_T, true);
         }
-        __builtin_amdgcn_wave_barrier();  // tile reads done before the next staging
     }
-    // merge the 4 waves: (m, l) per query, O through LDS
-    if (g == 0) {
-        ml[0][wave][l16] = mx;
-        ml[1][wave][l16] = l;
-    }
-    __syncthreads();  // every wave's tiles consumed; ml visible
-    float* ow = reinterpret_cast<float*>(lds + wave * TF_PM_WAVE_BYTES);  // [16][128]
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int qi = 4 * g + r;
-        float mall = ml[0][0][qi];
-        for (int w = 1; w < 4; w++) mall = fmaxf(mall, ml[0][w][qi]);
-        const float sc_w = __expf(ml[0][wave][qi] - mall);
-#pragma unroll
-        for (int nb = 0; nb < 8; nb++) ow[qi * HD + 16 * nb + l16] = o[nb][r] * sc_w;
+
+    // merge the waves that had tiles
+    const int nw = n_t < TF_PM_WAVES ? n_t : TF_PM_WAVES;
+    float* ml = reinterpret_cast<float*>(lds + L::ML);
+    l += __shfl_xor(l, 32);
+    if (h == 0) {
+        ml[wave * TF_PM_T + l32] = mx;
+        ml[(TF_PM_WAVES + wave) * TF_PM_T + l32] = l;
     }
     __syncthreads();
-    {
-        const int qi = tid >> 4, d0 = 8 * (tid & 15);
-        if (q0 + qi < n_q) {
-            float mall = ml[0][0][qi];
-            for (int w = 1; w < 4; w++) mall = fmaxf(mall, ml[0][w][qi]);
-            float L = 0.f;
-            for (int w = 0; w < 4; w++) L += ml[1][w][qi] * __expf(ml[0][w][qi] - mall);
-            const float inv = 1.f / fmaxf(L, 1e-20f);
-            float acc[8];
-            for (int i = 0; i < 8; i++) acc[i] = 0.f;
-            for (int w = 0; w < 4; w++) {
-                const float* src = reinterpret_cast<const float*>(lds + w * TF_PM_WAVE_BYTES) + qi * HD + d0;
-                for (int i = 0; i < 8; i++) acc[i] += src[i];
-            }
-            float* dst = out + (size_t)(q0 + qi) * n_head * HD + (size_t)h * HD + d0;
-            *reinterpret_cast<float4*>(dst) = make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
-            *reinterpret_cast<float4*>(dst + 4) = make_float4(acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv);
+    if (wave < nw) {
+        float mall = ml[l32];
+        for (int w = 1; w < nw; w++) mall = fmaxf(mall, ml[w * TF_PM_T + l32]);
+        const float sw = __builtin_amdgcn_exp2f(mx - mall);
+        float* ow = reinterpret_cast<float*>(kt) + l32 * L::OROW + 4 * h;
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+                *reinterpret_cast<float4*>(ow + 32 * db + 8 * b) =
+                    make_float4(o[db][4 * b] * sw, o[db][4 * b + 1] * sw, o[db][4 * b + 2] * sw,
+                                o[db][4 * b + 3] * sw);
+    }
+    __syncthreads();
+    // 16 threads a row, HD / 16 dims each
+    const int mr = tid >> 4, r = r0 + mr;
+    if (r >= n_rows) return;
+    float mall = ml[mr];
+    for (int w = 1; w < nw; w++) mall = fmaxf(mall, ml[w * TF_PM_T + mr]);
+    float ltot = 0.f;
+    for (int w = 0; w < nw; w++)
+        ltot += ml[(TF_PM_WAVES + w) * TF_PM_T + mr] * __builtin_amdgcn_exp2f(ml[w * TF_PM_T + mr] - mall);
+    float inv = 1.f / fmaxf(ltot, 1e-20f);
+    if (mall < -1.4e29f) inv = 0.f;      // no score above the mask: nothing to attend to
+    if (mall == INFINITY) inv = NAN;     // an infinite score has no softmax
+    const int qo = tf_div_by(r, G, g_inv);
+    float* dst = out + ((size_t)qo * n_head + (size_t)kv_h * G + (r - qo * G)) * HD;
+#pragma unroll
+    for (int c = 0; c < HD / 64; c++) {
+        const int d0 = 4 * (tid & 15) + 64 * c;
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int w = 0; w < nw; w++) {
+            const float4 v = *reinterpret_cast<const float4*>(lds + w * L::WAVE + 4 * (mr * L::OROW + d0));
+            acc.x += v.x;
+            acc.y += v.y;
+            acc.z += v.z;
+            acc.w += v.w;
         }
+        *reinterpret_cast<float4*>(dst + d0) =
+            make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
     }
 }
 
@@ -392,18 +506,31 @@ int tf_attn_prefill_any(const float* q, const uint16_t* k_cache, const uint16_t*
     TF_CHECK_ARG(head_dim == 64 || head_dim == 128 || head_dim == 256);
     TF_CHECK_ARG(((uintptr_t)q & 15) == 0 && ((uintptr_t)out & 15) == 0);
     TF_CHECK_ARG(((uintptr_t)k_cache & 7) == 0 && ((uintptr_t)v_cache & 7) == 0);
-    const dim3 grid((n_q + TF_PA_Q - 1) / TF_PA_Q, n_head);
-    auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, dim3(256), 0, tf_stream(stream), q, k_cache, v_cache, out,
-                           n_head, n_kv, pos0, pos0_dev, n_q, scale);
+    if (head_dim == 256) {
+        hipLaunchKernelGGL(tf_attn_prefill_kernel, dim3((n_q + TF_PA_Q - 1) / TF_PA_Q, n_head),
+                           dim3(256), 0, tf_stream(stream), q, k_cache, v_cache, out, n_head, n_kv,
+                           pos0, pos0_dev, n_q, scale);
+        return TF_LAUNCH_RESULT();
+    }
+    const int G = n_head / n_kv;
+    const uint32_t g_inv = G > 1 ? (uint32_t)(((1ull << 32) + G - 1) / G) : 0;
+    const uint32_t kv_inv = n_kv > 1 ? (uint32_t)(((1ull << 32) + n_kv - 1) / n_kv) : 0;
+    const long long tiles = ((long long)n_q * G + TF_PM_T - 1) / TF_PM_T;
+    TF_CHECK_ARG(tiles * TF_PM_T <= INT32_MAX && tiles * n_kv <= INT32_MAX / (64 * TF_PM_WAVES));
+    auto go = [&](auto kern, int bytes) -> int {
+        const int rc = tf_set_lds_limit((const void*)kern, bytes);
+        if (rc) return rc;
+        hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * n_kv)), dim3(64 * TF_PM_WAVES), bytes,
+                           tf_stream(stream), q, k_cache, v_cache, out, n_head, n_kv, pos0, pos0_dev,
+                           n_q * G, G, g_inv, kv_inv, scale);
+        return TF_LAUNCH_RESULT();
     };
-    if (head_dim == 64) go(tf_attn_prefill_kernel<64>);
-    else if (head_dim == 128) {
-        const dim3 g16((n_q + 15) / 16, n_head);
-        hipLaunchKernelGGL(tf_attn_prefill_mfma_kernel, g16, dim3(256), 0, tf_stream(stream), q,
-                           k_cache, v_cache, out, n_head, n_kv, pos0, pos0_dev, n_q, scale);
-    } else go(tf_attn_prefill_kernel<256>);
-    return TF_LAUNCH_RESULT();
+    const bool a16 = (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
+    if (head_dim == 64)
+        return a16 ? go(tf_attn_prefill_mfma_kernel<64, 16>, TfPmLds<64>::BYTES)
+                   : go(tf_attn_prefill_mfma_kernel<64, 4>, TfPmLds<64>::BYTES);
+    return a16 ? go(tf_attn_prefill_mfma_kernel<128, 16>, TfPmLds<128>::BYTES)
+               : go(tf_attn_prefill_mfma_kernel<128, 4>, TfPmLds<128>::BYTES);
 }
 
 extern "C" int tf_attn_prefill(const float* q, const uint16_t* k_cache, const uint16_t* v_cache,

@@ -1,0 +1,65 @@
+"""tf_attn_prefill (kernels/attn/fast_v2.cu:12-192) on the matrix cores at the
+edges of its tiles: 32 (query, head) rows a workgroup, 32 keys a tile, eight
+waves that share the tiles.  Against the fp64 softmax attention of the oracle.
+
+Tolerance: q and the probabilities are held in two f16 parts (2^-22 of the
+row's largest q, of each p), K and V are f16 and the products exact.  A score
+is off by at most 2^-22 max|q| sum|k| scale (under 2e-5 here: 2^-22 * 4 * 128 *
+0.8 / 8) plus as much again from fp32 summation, and an output is a mean of V
+rows whose weights are off by that: 4e-5 max|V|.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from taraference_amd import synth
+from _gpu import P, S, call, dev, empty, host
+
+pytestmark = pytest.mark.gpu
+
+
+def run(n_head, n_kv, hd, pos0, n_q, shift=0, scale=None):
+    rng = np.random.default_rng(n_q * 5 + pos0 + hd)
+    L = pos0 + n_q
+    K = synth.kv_cache(rng, L + 33, n_kv, hd)
+    V = synth.kv_cache(rng, L + 33, n_kv, hd)
+    K[L:] = V[L:] = 0x7E00  # f16 NaN past the last query
+    q = np.clip(rng.standard_normal((n_q, n_head * hd)), -4, 4).astype(np.float32)
+    scale = float(np.float32(hd ** -0.5)) if scale is None else scale
+    pad = np.zeros(shift // 2, np.uint16)
+    kb = dev(np.concatenate([pad, K.reshape(-1).view(np.uint16)]).view(np.int16))
+    vb = dev(np.concatenate([pad, V.reshape(-1).view(np.uint16)]).view(np.int16))
+    out = empty(n_q * n_head * hd)
+    print(f"attn h={n_head} kv={n_kv} hd={hd} pos0={pos0} n_q={n_q} shift={shift}", flush=True)
+    call("tf_attn_prefill", P(dev(q)), P(kb) + shift, P(vb) + shift, P(out), n_head, n_kv, hd, pos0,
+         n_q, scale, S())
+    y = host(out).reshape(n_q, -1)
+    vmax = float(np.abs(V[:L].view(np.float16).astype(np.float32)).max())
+    for i in sorted({0, 1, n_q // 2, n_q - 2, n_q - 1} & set(range(n_q))):
+        ref = oracle.attn_f64(q[i], K, V, n_head, n_kv, hd, pos0 + i + 1, scale)
+        err = np.abs(y[i] - ref).max()
+        assert err <= 4e-5 * vmax, (i, err, vmax)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("n_head,n_kv,pos0,n_q", [
+    (4, 4, 0, 1),       # one row, one key
+    (4, 4, 0, 33),      # one row and one key past a tile
+    (14, 2, 31, 5),     # 35 rows of 7 heads: queries cut by a tile of rows
+    (16, 2, 0, 32),     # whole tiles
+    (28, 4, 255, 9),    # 8 tiles for most rows, 9 for the last
+    (40, 1, 511, 3),    # more heads in the group than rows in a tile
+    (8, 8, 257, 64),
+])
+def test_attn_tiles(gpu, hd, n_head, n_kv, pos0, n_q):
+    run(n_head, n_kv, hd, pos0, n_q)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attn_caches_8_byte_aligned(gpu, hd):
+    run(14, 2, hd, 300, 7, shift=8)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attn_negative_scale(gpu, hd):
+    run(8, 2, hd, 70, 12, scale=-0.1)
