@@ -10,6 +10,7 @@
 
 #include "argmax_key.hpp"
 #include "dequant.hpp"
+#include "gemv_b32.hpp"
 #include "tf_common.hpp"
 #include "tf_host.hpp"
 
@@ -157,6 +158,42 @@ __global__ __launch_bounds__(256) void tf_copy_kv_kernel(const float* __restrict
     if (i < stride) cache[(size_t)pos * stride + i] = tf_f2h_halfup(src[i]);
 }
 
+// tf_rope_neox of q and k and tf_copy_kv_f16 of k and v in one launch, a
+// workgroup a head (n_head of q, then n_kv of k, then n_kv of v); the same
+// arithmetic.  Four launches of 2-5 us each, one after the other, became one.
+__global__ __launch_bounds__(64) void tf_rope_append_kernel(
+    float* __restrict__ q, float* __restrict__ k, const float* __restrict__ v,
+    uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int n_head, int n_kv, int head_dim,
+    int pos, const int* __restrict__ pos_dev, float theta) {
+    if (pos_dev) pos = pos_dev[0];
+    int h = blockIdx.x;
+    const size_t row = (size_t)pos * n_kv * head_dim;
+    if (h >= n_head + n_kv) {
+        h -= n_head + n_kv;
+        for (int i = threadIdx.x; i < head_dim; i += 64)
+            vc[row + h * head_dim + i] = tf_f2h_halfup(v[h * head_dim + i]);
+        return;
+    }
+    const bool is_k = h >= n_head;
+    if (is_k) h -= n_head;
+    float* base = (is_k ? k : q) + (size_t)h * head_dim;
+    const int half = head_dim / 2;
+    for (int i = threadIdx.x; i < half; i += 64) {
+        const float freq = powf(theta, -2.f * (float)i / (float)head_dim);
+        const float ang = (float)pos * freq;
+        float s, c;
+        sincosf(ang, &s, &c);
+        const float x0 = base[i], x1 = base[i + half];
+        const float y0 = x0 * c - x1 * s, y1 = x0 * s + x1 * c;
+        base[i] = y0;
+        base[i + half] = y1;
+        if (is_k) {
+            kc[row + h * head_dim + i] = tf_f2h_halfup(y0);
+            kc[row + h * head_dim + i + half] = tf_f2h_halfup(y1);
+        }
+    }
+}
+
 // ------------------------------------------------------------ argmax
 
 // argmax_f32 (kernels/ops.cu:573-599): the reference's winner, ties and
@@ -201,6 +238,43 @@ __global__ __launch_bounds__(1024) void tf_argmax_kernel(const float* __restrict
         for (int w = 1; w < (int)(blockDim.x >> 6); w++) best = part[w] > best ? part[w] : best;
         out_idx[0] = tf_argmax_key_index(best);
     }
+}
+
+// The same winner by as many workgroups as the logits keep busy: workgroup b
+// leaves the largest key of its values in slot b, for tf_argmax_slots_take.
+// For callers that hold the slots; 151936 logits: 18 us by the one workgroup
+// above.
+#define TF_ARGMAX_WGS 128
+static_assert(TF_ARGMAX_WGS <= TF_ARGMAX_SLOTS, "a slot a workgroup");
+__global__ __launch_bounds__(256) void tf_argmax_keys_kernel(const float* __restrict__ x, int n,
+                                                             unsigned long long* __restrict__ slots) {
+    __shared__ unsigned long long part[4];
+    unsigned long long best = 0;
+    const int n4 = n >> 2, tid = blockIdx.x * 256 + threadIdx.x;
+    auto take = [&](float v, int i) {
+        const unsigned long long k = tf_argmax_key(v, i);
+        best = k > best ? k : best;
+    };
+    for (int i = tid; i < n4; i += TF_ARGMAX_WGS * 256) {
+        const tf_u32x4 v = tf_ld16_a4(x + 4 * (size_t)i);
+#pragma unroll
+        for (int k = 0; k < 4; k++) take(__uint_as_float(v[k]), 4 * i + k);
+    }
+    if (tid < n - 4 * n4) take(x[4 * n4 + tid], 4 * n4 + tid);
+    best = tf_wave_max_u64(best);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; w++) best = part[w] > best ? part[w] : best;
+        slots[blockIdx.x] = best;
+    }
+}
+
+int tf_argmax_keys(const float* x, int n, unsigned long long* slots, tf_stream_t stream) {
+    TF_CHECK_ARG(x && slots && n > 0);
+    hipLaunchKernelGGL(tf_argmax_keys_kernel, dim3(TF_ARGMAX_WGS), dim3(256), 0, tf_stream(stream),
+                       x, n, slots);
+    return TF_LAUNCH_RESULT();
 }
 
 // ---------------------------------------------------------------- C ABI
@@ -269,6 +343,17 @@ extern "C" int tf_copy_kv_f16(const float* src, uint16_t* cache, int pos, const 
     TF_CHECK_ARG(src && cache && stride > 0 && (pos_dev || pos >= 0));
     hipLaunchKernelGGL(tf_copy_kv_kernel, dim3((stride + 255) / 256), dim3(256), 0,
                        tf_stream(stream), src, cache, pos, pos_dev, stride);
+    return TF_LAUNCH_RESULT();
+}
+
+int tf_rope_append(float* q, float* k, const float* v, uint16_t* k_cache, uint16_t* v_cache,
+                   int n_head, int n_kv, int head_dim, int pos, const int* pos_dev, float theta,
+                   tf_stream_t stream) {
+    TF_CHECK_ARG(q && k && v && k_cache && v_cache && n_head > 0 && n_kv > 0 && head_dim > 0 &&
+                 head_dim % 2 == 0 && (pos_dev || pos >= 0));
+    hipLaunchKernelGGL(tf_rope_append_kernel, dim3(n_head + 2 * n_kv), dim3(64), 0,
+                       tf_stream(stream), q, k, v, k_cache, v_cache, n_head, n_kv, head_dim, pos,
+                       pos_dev, theta);
     return TF_LAUNCH_RESULT();
 }
 

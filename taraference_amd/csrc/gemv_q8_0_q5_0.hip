@@ -30,11 +30,14 @@
 //    reads.
 #include <type_traits>
 
+#include "gemv_b32.hpp"
 #include "tf_common.hpp"
 #include "tf_host.hpp"
 
 enum TfB32Fmt { TF_B32_Q8_PAIR = 0, TF_B32_Q8_GEN = 1, TF_B32_Q8_F32 = 2, TF_B32_Q5_F32 = 3 };
-enum TfB32Src { TF_B32_SRC_Q8 = 0, TF_B32_SRC_F32 = 1 };
+// TF_B32_SRC_NORM: an f32 row that the staging RMS-normalizes first;
+// TF_B32_SRC_FLASH: the (m, l, O) partials of a split-KV attention, merged by it
+enum TfB32Src { TF_B32_SRC_Q8 = 0, TF_B32_SRC_F32 = 1, TF_B32_SRC_NORM = 2, TF_B32_SRC_FLASH = 3 };
 
 // Up to three matrices with the same K (Q/K/V or Q/K) share one launch;
 // their columns are numbered one after the other.  With n_split >= 1 there
@@ -52,7 +55,12 @@ struct TfB32Job {
     const float* residual;
     const int8_t* xq;  // TF_B32_SRC_Q8
     const float* xd;
-    const float* x;  // TF_B32_SRC_F32
+    const float* x;  // TF_B32_SRC_F32, TF_B32_SRC_NORM
+    const float* norm_w;  // TF_B32_SRC_NORM
+    float eps;
+    const float* part;  // TF_B32_SRC_FLASH: [head][split](m, l, O[head_dim])
+    int parts, head_dim;
+    int paired;  // task 2j: column j of w[0], 2j + 1: of w[1]; out[0] = silu(.) * (.)
 };
 
 // ------------------------------------------------------------ LDS images
@@ -76,6 +84,75 @@ __device__ __forceinline__ int tf_b32_xperm(int fmt, int v) {
     return ((v & 15) >> 2) * 8 + (v >> 4) * 4 + (v & 3);
 }
 
+// The RMS scale of the row (n = 32 G values), in the summation order of
+// tf_rms_norm_kernel (256 strided sums, halving tree), so that the normalized
+// values are bit-identical to that launch's; the workgroup has at least 256
+// threads, buf 257 floats.
+__device__ __forceinline__ float tf_b32_rms_scale(const TfB32Job& jb, float* buf) {
+    const int n = 32 * jb.nb, tid = threadIdx.x;
+    if (tid < 256) {
+        float local = 0.f;
+        for (int i = tid; i < n; i += 256) {
+            const float v = jb.x[i];
+            local = fmaf(v, v, local);
+        }
+        buf[tid] = local;
+    }
+    __syncthreads();
+    if (tid < 128) buf[tid] += buf[tid + 128];
+    __syncthreads();
+    if (tid < 64) {
+        float v = buf[tid] + buf[tid + 64];
+        v += __shfl_down(v, 32, 64);
+        v += __shfl_down(v, 16, 64);
+        v += __shfl_down(v, 8, 64);
+        v += __shfl_down(v, 4, 64);
+        v += __shfl_down(v, 2, 64);
+        v += __shfl_down(v, 1, 64);
+        if (tid == 0) buf[256] = 1.0f / sqrtf(v / (float)n + jb.eps);
+    }
+    __syncthreads();
+    return buf[256];
+}
+
+// Four values of the attention output from its partials, as the reduce kernel
+// forms them (log-sum-exp weights, O / max(l, 1e-20)); eight partials in flight.
+__device__ __forceinline__ float4 tf_b32_merge4(const TfB32Job& jb, int e) {
+    const int hd = jb.head_dim, po = 2 + hd, h = e / hd;
+    const float* ph = jb.part + (size_t)h * jb.parts * po;
+    const int d = 2 + e - h * hd;
+    float m = -1e30f, l = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 0; s0 < jb.parts; s0 += 8) {  // parts % 8 == 0
+        float2 ml[8], a[8], b[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float* p = ph + (size_t)(s0 + k) * po;  // 8-byte aligned: po is even
+            ml[k] = *reinterpret_cast<const float2*>(p);
+            a[k] = *reinterpret_cast<const float2*>(p + d);
+            b[k] = *reinterpret_cast<const float2*>(p + d + 2);
+        }
+        float mm = m;
+#pragma unroll
+        for (int k = 0; k < 8; k++) mm = fmaxf(mm, ml[k].x);
+        const float f = __expf(m - mm);
+        m = mm;
+        l *= f;
+        acc = make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float w = __expf(ml[k].x - mm);
+            l += w * ml[k].y;
+            acc.x += w * a[k].x;
+            acc.y += w * a[k].y;
+            acc.z += w * b[k].x;
+            acc.w += w * b[k].y;
+        }
+    }
+    const float inv = 1.f / fmaxf(l, 1e-20f);
+    return make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+}
+
 // Build the activation image; all threads of the workgroup; ends with a
 // barrier.  Quantization (f32 source, Q8 formats) is the reference's
 // (kernels/gemv.cu:16-40), bit-identical to tf_quantize_q8: a 16-lane DPP
@@ -83,10 +160,19 @@ __device__ __forceinline__ int tf_b32_xperm(int fmt, int v) {
 template <int FMT, int SK>
 __device__ __forceinline__ void tf_b32_stage(const TfB32Job& jb, uint8_t* lds) {
     const int G = jb.nb;
+    [[maybe_unused]] float scale = 1.f;
     if constexpr (FMT >= TF_B32_Q8_F32) {
         float* xs = reinterpret_cast<float*>(lds);
+        if constexpr (SK == TF_B32_SRC_NORM) scale = tf_b32_rms_scale(jb, xs + 32 * G);
         for (int i = threadIdx.x; i < G * 8; i += blockDim.x) {
-            const float4 v = *reinterpret_cast<const float4*>(jb.x + 4 * i);
+            float4 v;
+            if constexpr (SK == TF_B32_SRC_FLASH) v = tf_b32_merge4(jb, 4 * i);
+            else v = *reinterpret_cast<const float4*>(jb.x + 4 * i);
+            if constexpr (SK == TF_B32_SRC_NORM) {
+                const float4 w = *reinterpret_cast<const float4*>(jb.norm_w + 4 * i);
+                v = make_float4(v.x * scale * w.x, v.y * scale * w.y, v.z * scale * w.z,
+                                v.w * scale * w.w);
+            }
             const int g = i >> 3, v0 = 4 * (i & 7);
             *reinterpret_cast<float4*>(xs + 32 * g + tf_b32_xperm(FMT, v0)) = v;
         }
@@ -106,12 +192,18 @@ __device__ __forceinline__ void tf_b32_stage(const TfB32Job& jb, uint8_t* lds) {
                 d8[g] = tf_gld(jb.xd + g);
             }
         } else {
+            if constexpr (SK == TF_B32_SRC_NORM) scale = tf_b32_rms_scale(jb, d8 + G);
             const int m = threadIdx.x & 15, rows = blockDim.x >> 4;
             for (int g0 = 0; g0 < G; g0 += rows) {  // workgroup-uniform trip count
                 const int g = g0 + (threadIdx.x >> 4);
                 const bool ok = g < G;
-                const float2 v = ok ? *reinterpret_cast<const float2*>(jb.x + 32 * g + 2 * m)
-                                    : make_float2(0.f, 0.f);
+                float2 v = ok ? *reinterpret_cast<const float2*>(jb.x + 32 * g + 2 * m)
+                              : make_float2(0.f, 0.f);
+                if constexpr (SK == TF_B32_SRC_NORM) {
+                    const float2 w = ok ? *reinterpret_cast<const float2*>(jb.norm_w + 32 * g + 2 * m)
+                                        : make_float2(0.f, 0.f);
+                    v = make_float2(v.x * scale * w.x, v.y * scale * w.y);
+                }
                 const TfQ8Pair r = tf_q8_pair<false>(v.x, v.y);
                 if (ok) {
                     uint16_t* dst = reinterpret_cast<uint16_t*>(q8 + tf_b32_q8_off(FMT, g));
@@ -132,8 +224,10 @@ __device__ __forceinline__ void tf_b32_stage(const TfB32Job& jb, uint8_t* lds) {
 __device__ __forceinline__ uint32_t tf_b32_u16(const uint8_t* p) {
     return *(const TF_GAS uint16_t*)p;
 }
+// four bytes at a 2-byte aligned address: one load (gfx950 takes any alignment)
+typedef uint32_t tf_u32_a2 __attribute__((aligned(2)));
 __device__ __forceinline__ uint32_t tf_b32_u32_a2(const uint8_t* p) {
-    return tf_b32_u16(p) | (tf_b32_u16(p + 2) << 16);
+    return *(const TF_GAS tf_u32_a2*)p;
 }
 
 // Weights of one quad-step of a row, loaded before any of them is used.
@@ -225,12 +319,14 @@ __device__ __forceinline__ float tf_b32_step(const TfB32Regs& r, int k, int p, i
             s += (float)(int8_t)(v >> 16) * xb.z;
             s += (float)(int8_t)(v >> 24) * xb.w;
         } else {
-            // codes of values 4p+i (low nibbles) and 16+4p+i (high nibbles)
-            const uint32_t q = r.a.x, hl = r.e >> (4 * p), hh = r.e >> (16 + 4 * p);
+            // codes of values 4p+i (low nibbles) and 16+4p+i (high nibbles), four
+            // to a word: the product spreads four bits of qh to the words' bytes
+            const uint32_t M = 0x0f0f0f0fu, B = 0x01010101u;
+            const uint32_t hl = (r.e >> (4 * p)) & 15u, hh = (r.e >> (16 + 4 * p)) & 15u;
+            const uint32_t cl = (r.a.x & M) | (((hl * 0x00204081u) & B) << 4);
+            const uint32_t ch = ((r.a.x >> 4) & M) | (((hh * 0x00204081u) & B) << 4);
             auto code = [&](int i, bool high) -> float {
-                const uint32_t nib = high ? (q >> (8 * i + 4)) & 15u : (q >> (8 * i)) & 15u;
-                const uint32_t hb = ((high ? hh : hl) >> i) & 1u;
-                return (float)((int)(nib | (hb << 4)) - 16);
+                return (float)(((high ? ch : cl) >> (8 * i)) & 0xffu) - 16.f;
             };
             s = code(0, false) * xa.x;
             s += code(1, false) * xa.y;
@@ -267,6 +363,13 @@ __device__ __forceinline__ TfB32Task tf_b32_task(const TfB32Job& jb, int t) {
         r.j = j;
         r.b0 = (jb.nb * s) / jb.n_split;
         r.b1 = (jb.nb * (s + 1)) / jb.n_split;
+    } else if (jb.paired) {
+        r.col = ((tt & 1) ? jb.w[1] : jb.w[0]) + (size_t)(tt >> 1) * jb.col_bytes;
+        r.out = jb.out[0];
+        r.bias = nullptr;
+        r.j = tt >> 1;
+        r.b0 = 0;
+        r.b1 = jb.nb;
     } else {
         const int m = tt < jb.n[0] ? 0 : (tt < jb.n[0] + jb.n[1] ? 1 : 2);
         const int j = tt - (m > 0 ? jb.n[0] : 0) - (m > 1 ? jb.n[1] : 0);
@@ -285,14 +388,16 @@ __device__ __forceinline__ TfB32Task tf_b32_task(const TfB32Job& jb, int t) {
 // SPR quads per row (4, 8 or 16).  ITERS > 0: every quad has at most ITERS
 // units of work per row, all loaded up front, and the next task's loads are
 // issued before this task is computed; ITERS == 0: a plain loop.
-template <int FMT, int SK, int SPR, int ITERS>
-__global__ __launch_bounds__(512) void tf_b32_kernel(TfB32Job jb) {
-    extern __shared__ __align__(16) uint8_t lds[];
+//
+// PAIRED (SPR <= 8): the even units of a wave hold gate rows, the odd ones the
+// up rows of the same output, which leaves as silu(gate) * up.
+template <int FMT, int SK, int SPR, int ITERS, bool PAIRED = false>
+__device__ __forceinline__ void tf_b32_body(const TfB32Job& jb, uint8_t* lds, int wave,
+                                            int nwaves) {
     constexpr int UNITS = 16 / SPR;
+    static_assert(!PAIRED || UNITS % 2 == 0, "gate and up rows of one wave");
     const int lane = threadIdx.x & 63;
     const int p = lane & 3, slot = lane >> 2, unit = slot / SPR, sir = slot % SPR;
-    const int wave = tf_wave_id();
-    const int nwaves = (gridDim.x * blockDim.x) >> 6;
     const int n_tasks = (jb.n_tot + UNITS - 1) / UNITS;
     const int G = jb.nb;
     constexpr bool PAIR = FMT == TF_B32_Q8_PAIR;
@@ -302,6 +407,12 @@ __global__ __launch_bounds__(512) void tf_b32_kernel(TfB32Job jb) {
 
     auto finish = [&](const TfB32Task& t, float acc) {
         acc = tf_group_sum<4 * SPR>(acc);
+        if constexpr (PAIRED) {
+            const float up = __shfl(acc, (lane + 4 * SPR) & 63, 64);
+            if (t.valid && (unit & 1) == 0 && (lane & (4 * SPR - 1)) == 0)
+                t.out[t.j] = (acc / (1.f + __expf(-acc))) * up;
+            return;
+        }
         if (t.valid && (lane & (4 * SPR - 1)) == 0) {
             if (jb.n_split == 0) {
                 if (jb.use_res == 1) acc += jb.residual[t.j];
@@ -357,6 +468,31 @@ __global__ __launch_bounds__(512) void tf_b32_kernel(TfB32Job jb) {
             finish(t, acc);
         }
     }
+}
+
+template <int FMT, int SK, int SPR, int ITERS, bool PAIRED = false>
+__global__ __launch_bounds__(512) void tf_b32_kernel(TfB32Job jb) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    tf_b32_body<FMT, SK, SPR, ITERS, PAIRED>(jb, lds, tf_wave_id(),
+                                             (gridDim.x * blockDim.x) >> 6);
+}
+
+// Q5_0 q and k and a Q8_0 v of the same row in one launch, each workgroup
+// normalizing the row for itself: the first `blocks5` workgroups take q and k,
+// the others v.
+template <int ITERS>
+__global__ __launch_bounds__(512) void tf_b32_norm_qkv_kernel(TfB32Job j5, TfB32Job j8,
+                                                              int blocks5) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    const int wpb = blockDim.x >> 6, w = threadIdx.x >> 6, b = blockIdx.x;
+    const int blocks8 = gridDim.x - blocks5;
+    // waves numbered within their part, block-major as tf_wave_id
+    if (b < blocks5)
+        tf_b32_body<TF_B32_Q5_F32, TF_B32_SRC_NORM, 16, ITERS>(j5, lds, w * blocks5 + b,
+                                                               blocks5 * wpb);
+    else
+        tf_b32_body<TF_B32_Q8_PAIR, TF_B32_SRC_NORM, 8, ITERS>(j8, lds, w * blocks8 + b - blocks5,
+                                                               blocks8 * wpb);
 }
 
 // ---------------------------------------------------------------- dispatch
@@ -416,8 +552,13 @@ static int tf_b32_launch(TfB32Job jb, tf_stream_t stream) {
             else go(tf_icb<16>{}, tf_icb<0>{});
         }
     } else {
-        if (len <= 4) go(tf_icb<4>{}, tf_icb<0>{});
-        else if (len <= 8) go(tf_icb<8>{}, tf_icb<0>{});
+        // up to four blocks a quad: loaded ahead of the staging
+        const int i16 = (len + 15) / 16;
+        if (len <= 4) go(tf_icb<4>{}, tf_icb<1>{});
+        else if (len <= 8) go(tf_icb<8>{}, tf_icb<1>{});
+        else if (i16 == 1) go(tf_icb<16>{}, tf_icb<1>{});
+        else if (i16 == 2) go(tf_icb<16>{}, tf_icb<2>{});
+        else if (i16 <= 4) go(tf_icb<16>{}, tf_icb<4>{});
         else go(tf_icb<16>{}, tf_icb<0>{});
     }
     return rc;
@@ -539,6 +680,111 @@ static int tf_b32_multi(int fmt, int nw, const uint8_t* const* w, float* const* 
     TF_CHECK_ARG(tf_b32_f32_src_ok(x, fmt));
     jb.x = x;
     return tf_b32_run(fmt, TF_B32_SRC_F32, jb, stream);
+}
+
+// ------------------------------------------------- the decode step's fusions
+
+bool tf_b32_norm_fits(int n_rows) { return n_rows > 0 && n_rows % 64 == 0 && n_rows <= 2048; }
+
+int tf_b32_norm_qkv(const float* x, const float* norm_w, float eps, const uint8_t* wq,
+                    const uint8_t* wk, const uint8_t* wv, float* q, float* k, float* v,
+                    const float* bq, const float* bk, const float* bv, int n_rows, int n_q, int n_k,
+                    int n_v, int cb_qk, int cb_v, tf_stream_t stream) {
+    TF_CHECK_ARG(x && norm_w && (((uintptr_t)x | (uintptr_t)norm_w) & 15) == 0);
+    TF_CHECK_ARG(tf_b32_norm_fits(n_rows) && (!bq) == (!bk));
+    TfB32Job j5 = tf_b32_job(wq, q, n_rows, n_q, cb_qk);
+    j5.w[1] = wk;
+    j5.out[1] = k;
+    j5.n[1] = n_k;
+    j5.n_tot = n_q + n_k;
+    j5.bias[0] = bq;
+    j5.bias[1] = bk;
+    TfB32Job j8 = tf_b32_job(wv, v, n_rows, n_v, cb_v);
+    j8.bias[0] = bv;
+    TF_CHECK_ARG(tf_b32_common_ok(j5, 2, n_rows, 22) && tf_b32_common_ok(j8, 1, n_rows, 34));
+    TF_CHECK_ARG(tf_q8_0_pair_ok(j8.w, 1, j8.nb, cb_v));
+    j5.x = j8.x = x;
+    j5.norm_w = j8.norm_w = norm_w;
+    j5.eps = j8.eps = eps;
+    const int lds = tf_b32_lds_bytes(TF_B32_Q5_F32, j5.nb) + 257 * 4;  // the larger image
+    const int its = (j5.nb + 15) / 16;  // blocks over 16 quads, pairs over 8
+    int rc = 0;
+    auto go = [&](auto it) {
+        auto fn = tf_b32_norm_qkv_kernel<decltype(it)::value>;
+        const int t8 = (n_v + 1) / 2;
+        const int BT = tf_block_threads(512, j5.n_tot + t8);
+        const int b5 = tf_persistent_blocks((const void*)fn, BT, lds, j5.n_tot);
+        const int b8 = tf_persistent_blocks((const void*)fn, BT, lds, t8);
+        hipLaunchKernelGGL(fn, dim3(b5 + b8), dim3(BT), lds, tf_stream(stream), j5, j8, b5);
+        rc = TF_LAUNCH_RESULT();
+    };
+    if (its == 1) go(tf_icb<1>{});
+    else if (its == 2) go(tf_icb<2>{});
+    else go(tf_icb<4>{});
+    return rc;
+}
+
+bool tf_b32_flash_out_fits(int n_head, int head_dim, int parts) {
+    return n_head > 0 && head_dim > 0 && head_dim % 32 == 0 && n_head * head_dim <= 2048 &&
+           (parts == 8 || parts == 16);
+}
+
+int tf_b32_flash_out(const uint8_t* w, const float* partial, int n_head, int head_dim, int parts,
+                     float* x, int n_cols, int col_bytes, tf_stream_t stream) {
+    TF_CHECK_ARG(partial && ((uintptr_t)partial & 7) == 0);
+    TF_CHECK_ARG(tf_b32_flash_out_fits(n_head, head_dim, parts));
+    const int n_rows = n_head * head_dim;
+    TfB32Job jb = tf_b32_job(w, x, n_rows, n_cols, col_bytes);
+    TF_CHECK_ARG(tf_b32_common_ok(jb, 1, n_rows, 22));
+    jb.part = partial;
+    jb.parts = parts;
+    jb.head_dim = head_dim;
+    jb.use_res = 2;
+    const int lds = tf_b32_lds_bytes(TF_B32_Q5_F32, jb.nb);
+    const int its = (jb.nb + 15) / 16;
+    int rc = 0;
+    auto go = [&](auto it) {
+        auto fn = tf_b32_kernel<TF_B32_Q5_F32, TF_B32_SRC_FLASH, 16, decltype(it)::value>;
+        const int BT = tf_block_threads(512, n_cols);
+        const int blocks = tf_persistent_blocks((const void*)fn, BT, lds, n_cols);
+        hipLaunchKernelGGL(fn, dim3(blocks), dim3(BT), lds, tf_stream(stream), jb);
+        rc = TF_LAUNCH_RESULT();
+    };
+    if (its == 1) go(tf_icb<1>{});
+    else if (its == 2) go(tf_icb<2>{});
+    else go(tf_icb<4>{});
+    return rc;
+}
+
+int tf_b32_norm_gate_up(const float* x, const float* norm_w, float eps, const uint8_t* gate,
+                        const uint8_t* up, float* h, int n_rows, int n_cols, int col_bytes,
+                        tf_stream_t stream) {
+    TF_CHECK_ARG(x && norm_w && (((uintptr_t)x | (uintptr_t)norm_w) & 15) == 0);
+    TF_CHECK_ARG(tf_b32_norm_fits(n_rows) && n_cols < (1 << 30));
+    TfB32Job jb = tf_b32_job(gate, h, n_rows, n_cols, col_bytes);
+    jb.w[1] = up;
+    jb.out[1] = h;
+    jb.n[1] = n_cols;
+    jb.n_tot = 2 * n_cols;
+    jb.paired = 1;
+    TF_CHECK_ARG(tf_b32_common_ok(jb, 2, n_rows, 22));
+    jb.x = x;
+    jb.norm_w = norm_w;
+    jb.eps = eps;
+    const int lds = tf_b32_lds_bytes(TF_B32_Q5_F32, jb.nb) + 257 * 4;
+    const int its = (jb.nb + 7) / 8;
+    int rc = 0;
+    auto go = [&](auto it) {
+        auto fn = tf_b32_kernel<TF_B32_Q5_F32, TF_B32_SRC_NORM, 8, decltype(it)::value, true>;
+        const int BT = tf_block_threads(512, n_cols);
+        const int blocks = tf_persistent_blocks((const void*)fn, BT, lds, n_cols);
+        hipLaunchKernelGGL(fn, dim3(blocks), dim3(BT), lds, tf_stream(stream), jb);
+        rc = TF_LAUNCH_RESULT();
+    };
+    if (its <= 2) go(tf_icb<2>{});
+    else if (its <= 4) go(tf_icb<4>{});
+    else go(tf_icb<8>{});
+    return rc;
 }
 
 // ---------------------------------------------------------------- C ABI

@@ -30,6 +30,7 @@
 
 #include "argmax_key.hpp"
 #include "decode_persistent.hpp"
+#include "gemv_b32.hpp"
 #include "op_api.hpp"
 #include "prefill.hpp"
 #include "taraference_hip.h"
@@ -165,6 +166,29 @@ struct tf_model {
         for (void* p : allocs) (void)hipFree(p);
     }
 
+    // Layers whose norm, GEMVs and (gate / up) SiLU run as one launch in step():
+    // Q5_0 q and k beside a Q8_0 v, a Q5_0 gate and up; and a Q5_0 wo that
+    // merges the attention's few partials.
+    bool b32_qkv_ok(const Layer& L) const {
+        return L.wq.wtype == tf::WType::Q5_0 && L.wk.wtype == tf::WType::Q5_0 &&
+               L.wv.wtype == tf::WType::Q8_0 && (int)L.wq.n_rows == cfg.n_embd &&
+               (int)L.wk.n_rows == cfg.n_embd && (int)L.wv.n_rows == cfg.n_embd &&
+               L.wq.col_bytes == L.wk.col_bytes && L.wv.col_bytes % 4 == 0 && (!L.bq) == (!L.bk) &&
+               ((uintptr_t)L.wv.data & 3) == 0 && ((uintptr_t)L.attn_norm & 15) == 0 &&
+               tf_b32_norm_fits(cfg.n_embd);
+    }
+    bool b32_wo_ok(const Layer& L) const {
+        return L.wo.wtype == tf::WType::Q5_0 && (int)L.wo.n_rows == fd.n_head * fd.head_dim &&
+               tf_b32_flash_out_fits(fd.n_head, fd.head_dim, fd.n_split);
+    }
+    bool b32_gate_up_ok(const Layer& L) const {
+        return L.gate.wtype == tf::WType::Q5_0 && L.up.wtype == tf::WType::Q5_0 &&
+               (int)L.gate.n_rows == cfg.n_embd && (int)L.up.n_rows == cfg.n_embd &&
+               (int)L.gate.n_cols == cfg.n_ff && (int)L.up.n_cols == cfg.n_ff &&
+               L.gate.col_bytes == L.up.col_bytes && ((uintptr_t)L.ffn_norm & 15) == 0 &&
+               tf_b32_norm_fits(cfg.n_embd);
+    }
+
     // One decode step.  pos_dev == nullptr: host position `pos` and host
     // token `token`; otherwise both are read from device memory.
     void step(hipStream_t s, int token, int pos, bool device_state) {
@@ -174,12 +198,20 @@ struct tf_model {
         tf::check(tf_embed_row(token_embd.data, embd_block_bytes, x, token, tok_dev, c.n_embd,
                                (int)token_embd.col_bytes, s),
                   "embed");
-        const int stride = c.n_kv * c.head_dim;
         for (size_t li = 0; li < layers.size(); li++) {
             const Layer& L = layers[li];
             // ---- attention block
-            tf::check(tf_rms_norm(x, L.attn_norm, xb, c.n_embd, c.rms_eps, s), "rms_norm");
-            if (!tf::try_gemv_qkv(s, L.wq, L.wk, L.wv, xb, q, k, v, L.bq, L.bk, L.bv, q8_x, q8_d)) {
+            const bool fused_qkv = b32_qkv_ok(L);
+            if (fused_qkv)
+                tf::check(tf_b32_norm_qkv(x, L.attn_norm, c.rms_eps, L.wq.data, L.wk.data, L.wv.data,
+                                          q, k, v, L.bq, L.bk, L.bv, c.n_embd, (int)L.wq.n_cols,
+                                          (int)L.wk.n_cols, (int)L.wv.n_cols, (int)L.wq.col_bytes,
+                                          (int)L.wv.col_bytes, s),
+                          "norm+qkv");
+            else
+                tf::check(tf_rms_norm(x, L.attn_norm, xb, c.n_embd, c.rms_eps, s), "rms_norm");
+            if (!fused_qkv &&
+                !tf::try_gemv_qkv(s, L.wq, L.wk, L.wv, xb, q, k, v, L.bq, L.bk, L.bv, q8_x, q8_d)) {
                 if (tf::try_gemv_pair(s, L.wq, L.wk, xb, q, k, L.bq, L.bk, q8_x, q8_d) ||
                     tf::try_gemv_q5_dual(s, L.wq, L.wk, xb, q, k, L.bq, L.bk)) {
                     tf::gemv(s, L.wv, xb, v, L.bv, GemvResidual::none(), gemv_partial,
@@ -190,18 +222,36 @@ struct tf_model {
                     tf::gemv(s, L.wv, xb, v, L.bv, GemvResidual::none(), gemv_partial, partial_stride);
                 }
             }
-            tf::check(tf_rope_neox(q, c.n_head, c.head_dim, pos, pos_dev, c.rope_theta, s), "rope q");
-            tf::check(tf_rope_neox(k, c.n_kv, c.head_dim, pos, pos_dev, c.rope_theta, s), "rope k");
-            tf::check(tf_copy_kv_f16(k, kc[li], pos, pos_dev, stride, s), "copy k");
-            tf::check(tf_copy_kv_f16(v, vc[li], pos, pos_dev, stride, s), "copy v");
-            tf::launch_attn_flash(s, fd, q, kc[li], vc[li], flash_partial, xb, pos, pos_dev);
-            if (!tf::try_gemv_global_q8(s, L.wo, xb, x, nullptr, GemvResidual::in_place(), q8_x,
-                                        q8_d, gemv_partial, partial_stride))
-                tf::gemv(s, L.wo, xb, x, nullptr, GemvResidual::in_place(), gemv_partial,
-                         partial_stride);
+            tf::check(tf_rope_append(q, k, v, kc[li], vc[li], c.n_head, c.n_kv, c.head_dim, pos,
+                                     pos_dev, c.rope_theta, s),
+                      "rope + append");
+            if (b32_wo_ok(L)) {  // wo merges the attention's partials itself
+                tf::check(pos_dev ? tf_flash_decode_partial_d(q, kc[li], vc[li], flash_partial,
+                                                              fd.n_head, fd.n_kv, fd.head_dim,
+                                                              pos_dev, 1, fd.n_split, fd.scale, s)
+                                  : tf_flash_decode_partial(q, kc[li], vc[li], flash_partial,
+                                                            fd.n_head, fd.n_kv, fd.head_dim, pos,
+                                                            1, fd.n_split, fd.scale, s),
+                          "flash partial");
+                tf::check(tf_b32_flash_out(L.wo.data, flash_partial, fd.n_head, fd.head_dim,
+                                           fd.n_split, x, (int)L.wo.n_cols, (int)L.wo.col_bytes, s),
+                          "merge+wo");
+            } else {
+                tf::launch_attn_flash(s, fd, q, kc[li], vc[li], flash_partial, xb, pos, pos_dev);
+                if (!tf::try_gemv_global_q8(s, L.wo, xb, x, nullptr, GemvResidual::in_place(), q8_x,
+                                            q8_d, gemv_partial, partial_stride))
+                    tf::gemv(s, L.wo, xb, x, nullptr, GemvResidual::in_place(), gemv_partial,
+                             partial_stride);
+            }
             // ---- FFN block
-            tf::check(tf_rms_norm(x, L.ffn_norm, xb, c.n_embd, c.rms_eps, s), "rms_norm");
-            if (!tf::try_gemv_q4_ffn(s, L.gate, L.up, xb, hb, q8_x, q8_d)) {
+            const bool fused_ffn = b32_gate_up_ok(L);
+            if (fused_ffn)
+                tf::check(tf_b32_norm_gate_up(x, L.ffn_norm, c.rms_eps, L.gate.data, L.up.data, hb,
+                                              c.n_embd, c.n_ff, (int)L.gate.col_bytes, s),
+                          "norm+gate+up");
+            else
+                tf::check(tf_rms_norm(x, L.ffn_norm, xb, c.n_embd, c.rms_eps, s), "rms_norm");
+            if (!fused_ffn && !tf::try_gemv_q4_ffn(s, L.gate, L.up, xb, hb, q8_x, q8_d)) {
                 // layer.rs:1267-1390: gate and up (one dual launch when both
                 // are Q5_0), then silu_mul
                 if (!tf::try_gemv_q5_dual(s, L.gate, L.up, xb, hb, hb2, nullptr, nullptr)) {
@@ -219,17 +269,32 @@ struct tf_model {
                          partial_stride);
         }
         // ---- logits + argmax
-        tf::check(tf_rms_norm(x, output_norm, xb, c.n_embd, c.rms_eps, s), "rms_norm");
-        if (!tf::try_gemv_global_q8(s, output, xb, logits, nullptr, GemvResidual::none(), q8_x,
-                                    q8_d, gemv_partial, partial_stride))
-            tf::gemv(s, output, xb, logits, nullptr, GemvResidual::none(), gemv_partial,
-                     partial_stride);
-        tf::check(tf_argmax(logits, c.n_vocab, d_argmax, s), "argmax");
-        if (device_state) {
+        head(s, x);
+        if (!device_state)
+            tf::check(tf_argmax_key_finalize(d_amax_key, d_argmax, s), "argmax");
+        else {
             hipLaunchKernelGGL(tf_decode_advance_kernel, dim3(1), dim3(256), 0, s, d_pos, d_step,
-                               d_token, d_argmax, nullptr, d_forced, d_nforced, d_log);
+                               d_token, d_argmax, d_amax_key, d_forced, d_nforced, d_log);
             tf::check((int)hipGetLastError(), "advance");
         }
+    }
+
+    // Logits of one hidden row and the keys of their argmax (d_amax_key).
+    void head(hipStream_t s, const float* row) {
+        const tf_model_config& c = cfg;
+        if (tf::global_q8_ok(output) && (int)output.n_rows == c.n_embd && c.n_embd % 128 == 0 &&
+            c.n_embd <= 8192) {  // the rows that tf_norm_quant takes
+            tf::check(tf_norm_quant(row, output_norm, c.rms_eps, xb, q8_x, q8_d, c.n_embd, s),
+                      "norm_quant");
+            tf::gemv_global_q8(s, output, logits, nullptr, GemvResidual::none(), q8_x, q8_d);
+        } else {
+            tf::check(tf_rms_norm(row, output_norm, xb, c.n_embd, c.rms_eps, s), "rms_norm");
+            if (!tf::try_gemv_global_q8(s, output, xb, logits, nullptr, GemvResidual::none(), q8_x,
+                                        q8_d, gemv_partial, partial_stride))
+                tf::gemv(s, output, xb, logits, nullptr, GemvResidual::none(), gemv_partial,
+                         partial_stride);
+        }
+        tf::check(tf_argmax_keys(logits, c.n_vocab, d_amax_key, s), "argmax");
     }
 
     // The same step with fused kernels: each activation is normalized and
@@ -750,13 +815,8 @@ struct tf_model {
             if (off + CH >= n) tf::check(tf_pg_add_row(pf_x, part, last, E, ts), "add");
         }
         // logits of the last prompt token (the decode step's head)
-        const float* xl = pf_x + (size_t)last * E;
-        tf::check(tf_rms_norm(xl, output_norm, xb, E, c.rms_eps, s), "rms_norm");
-        if (!tf::try_gemv_global_q8(s, output, xb, logits, nullptr, GemvResidual::none(), q8_x,
-                                    q8_d, gemv_partial, partial_stride))
-            tf::gemv(s, output, xb, logits, nullptr, GemvResidual::none(), gemv_partial,
-                     partial_stride);
-        tf::check(tf_argmax(logits, c.n_vocab, d_argmax, s), "argmax");
+        head(s, pf_x + (size_t)last * E);
+        tf::check(tf_argmax_key_finalize(d_amax_key, d_argmax, s), "argmax");
     }
 
     void dump_trace() {

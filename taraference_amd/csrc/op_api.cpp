@@ -50,21 +50,31 @@ void gemv(hipStream_t s, const GpuMat& w, const float* x, float* y, const float*
 bool try_gemv_global_q8(hipStream_t s, const GpuMat& w, const float* x, float* y,
                         const float* bias, GemvResidual res, int8_t* q8_x, float* q8_d,
                         float* /*partial*/, size_t /*partial_stride*/) {
-    if (w.wtype == WType::Q6K && !w.compact_data) return false;
-    if (w.wtype == WType::Q5_0) return false;  // no global-Q8 Q5_0 kernel (matmul.rs:160-176)
-    const int use_bias = bias ? 1 : 0;
+    if (!global_q8_ok(w)) return false;
     quantize_q8(s, x, q8_x, q8_d, I(w.n_rows));
+    gemv_global_q8(s, w, y, bias, res, q8_x, q8_d);
+    return true;
+}
+
+bool global_q8_ok(const GpuMat& w) {
+    if (w.wtype == WType::Q6K && !w.compact_data) return false;
+    return w.wtype != WType::Q5_0;  // no global-Q8 Q5_0 kernel (matmul.rs:160-176)
+}
+
+void gemv_global_q8(hipStream_t s, const GpuMat& w, float* y, const float* bias, GemvResidual res,
+                    const int8_t* q8_x, const float* q8_d) {
+    const int use_bias = bias ? 1 : 0;
     if (w.wtype == WType::Q8_0) {
         check(tf_gemv_q8_0_q8(w.data, q8_x, q8_d, y, I(w.n_rows), I(w.n_cols), I(w.col_bytes),
                               use_bias, bias, res.use_res(), res.add, S(s)),
               "gemv_q8_0_global");
-        return true;
+        return;
     }
     if (w.wtype == WType::Q4K) {
         check(tf_gemv_q4k_q8(w.data, q8_x, q8_d, y, I(w.n_rows), I(w.n_cols), I(w.col_bytes),
                              use_bias, bias, res.use_res(), res.add, S(s)),
               "gemv_q4_k_global");
-        return true;
+        return;
     }
     // Q6_K compact: the reference picks the 8/4-way in-block split-K kernel
     // for tall rows (matmul.rs:196-223) and the single-pass kernel otherwise.
@@ -79,7 +89,6 @@ bool try_gemv_global_q8(hipStream_t s, const GpuMat& w, const float* x, float* y
                                      res.add, S(s)),
               "gemv_q6_k_compact_global");
     }
-    return true;
 }
 
 bool try_gemv_pair(hipStream_t s, const GpuMat& wa, const GpuMat& wb, const float* x,

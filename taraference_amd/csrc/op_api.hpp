@@ -67,6 +67,10 @@ void gemv(hipStream_t s, const GpuMat& w, const float* x, float* y, const float*
 bool try_gemv_global_q8(hipStream_t s, const GpuMat& w, const float* x, float* y,
                         const float* bias, GemvResidual res, int8_t* q8_x, float* q8_d,
                         float* partial, size_t partial_stride);
+// Its second half, for an activation already in q8_x / q8_d.
+bool global_q8_ok(const GpuMat& w);
+void gemv_global_q8(hipStream_t s, const GpuMat& w, float* y, const float* bias, GemvResidual res,
+                    const int8_t* q8_x, const float* q8_d);
 
 // matmul.rs:509 try_gemv_pair (Q4_K branch :727-784)
 bool try_gemv_pair(hipStream_t s, const GpuMat& wa, const GpuMat& wb, const float* x,
