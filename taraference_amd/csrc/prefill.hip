@@ -160,12 +160,17 @@ __global__ __launch_bounds__(256) void tf_attn_prefill_kernel(
 //       transposing LDS reads (ds_read_b64_tr_b16: four keys of a lane's dim).
 // LDS rows keep their 16-byte chunks xor-ed with the row, so that 16 K rows, or
 // the 4 rows x 64 bytes of a transposing read, fall on distinct banks.
-// What bounds it: the matrix cores, at two products per score and per P V term
-// (256 tokens of 28 heads at 8000: 30 GF, 60 GF of f16 products, 77 us), the
-// softmax's vector work beside them; the form before it (16 queries of one head,
-// keys staged through registers, V gathered two bytes at a time) took 234 us, and
-// 19.3 against 13.2 us for a fresh 512-token prompt of 16 heads.  Error against
-// 64 bits 5.6e-7 and 2.5e-7, before 6.8e-7 and 2.7e-7.
+// What bounds it: long contexts, the matrix cores (two products per score and per
+// P V term) and LDS bandwidth about equally, 27 us each of the 77 us that 256
+// tokens of 28 heads at position 8000 take, with the softmax between them (a raised
+// wave priority for either half changed nothing); short ones, the chain of copy,
+// scores, P V and merge of one tile.  The form before it (16 queries of one head,
+// keys staged through registers, V gathered two bytes at a time; head_dim 64 on the
+// vector ALU) took 234 us there, 16.5 where this takes 11.0 for a fresh 512-token
+// prompt of 16 heads, 33 against 7.7 for 400 tokens of 14 heads of 64, 5.1 and 5.1
+// for 5 tokens (q split by each wave for itself instead of once: 13.4, 9.1 and 5.1
+// us for these three).  Error against 64 bits 5.5e-7 at 8000 and
+// 2.5e-7 at 512, before 6.7e-7 and 2.7e-7.
 #define TF_PM_WAVES 8
 #define TF_PM_T 32  // keys per tile, rows per workgroup
 
@@ -176,7 +181,9 @@ struct TfPmLds {
     static constexpr int OROW = HD + 4;                // floats of a merge row
     static constexpr int WAVE = TF_PM_T * OROW * 4;    // the K + V tiles, then the wave's O
     static constexpr int ML = TF_PM_WAVES * WAVE;      // m, l: [2][waves][32]
-    static constexpr int BYTES = ML + 2 * TF_PM_WAVES * TF_PM_T * 4;
+    static constexpr int Q = ML + 2 * TF_PM_WAVES * TF_PM_T * 4;  // q fragments, two parts
+    static constexpr int S2 = Q + 2 * TILE;                       // a factor per row
+    static constexpr int BYTES = S2 + TF_PM_T * 4;
     static_assert(2 * TILE <= WAVE, "the tiles fit where O goes");
 };
 
@@ -233,10 +240,8 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
     uint8_t* kt = lds + wave * L::WAVE;
     uint8_t* vt = kt + L::TILE;
 
-    // the row of this lane
-    const int row = r0 + l32 < n_rows ? r0 + l32 : rl;
-    const int qi = tf_div_by(row, G, g_inv);
-    const int qpos = pos0 + qi;
+    // the query of this lane's row
+    const int qpos = pos0 + (int)tf_div_by(r0 + l32 < n_rows ? r0 + l32 : rl, G, g_inv);
 
     // copy i of a tile: byte p = 64 DW i + DW lane of it, row p / ROWB; rows past
     // the last key repeat it (their scores are masked)
@@ -261,44 +266,75 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
                 tf_lds_dma_s<DW>(tb, off(i, rmax), ldst + 64 * DW * i);
         }
     };
-    float s2 = 0.f;  // score in powers of two = product * s2
+    // q^T fragments: dims 16 st + 8 h .. +7 of a row in two f16 parts, after a
+    // power of two that takes the row's largest value to [2^14, 2^15) and with the
+    // sign of the scale, so that the largest score has the largest product.  Made
+    // once for the workgroup: wave w copies rows 4 w .. + 3 (where its V tile will
+    // go, K right behind them), a thread splits eight dims; chunk c = 2 st + h of
+    // row r at 16-byte slot 32 c + (r ^ c) of a part.
+    float s2;  // score in powers of two = product * s2
     tf_h8 qb[ST][2];
-    if (wave < n_t) {
-        const float* qr = q + ((size_t)qi * n_head + (size_t)kv_h * G + (row - qi * G)) * HD;
-        float qv[ST][8];
+    {
+        constexpr int QC = 4 * HD * 4 / 1024;  // copies of a wave's q rows
+        const bool tiles = wave < n_t;
 #pragma unroll
-        for (int st = 0; st < ST; st++) {
-            const float4 a = *reinterpret_cast<const float4*>(qr + 16 * st + 8 * h);
-            const float4 b = *reinterpret_cast<const float4*>(qr + 16 * st + 8 * h + 4);
-            qv[st][0] = a.x; qv[st][1] = a.y; qv[st][2] = a.z; qv[st][3] = a.w;
-            qv[st][4] = b.x; qv[st][5] = b.y; qv[st][6] = b.z; qv[st][7] = b.w;
+        for (int i = 0; i < QC; i++) {
+            const int p = 1024 * i + 16 * lane, rq = r0 + 4 * wave + p / (4 * HD);
+            const int r = rq < n_rows ? rq : rl;
+            const int ri = tf_div_by(r, G, g_inv);
+            tf_lds_dma16(reinterpret_cast<const uint8_t*>(
+                             q + ((size_t)ri * n_head + (size_t)kv_h * G + (r - ri * G)) * HD) +
+                             p % (4 * HD),
+                         tf_lds_off(vt) + 1024 * i);
         }
-        issue(kbase, kt, wave * TF_PM_T, false);
-        issue(vbase, vt, wave * TF_PM_T, true);
-
-        // q^T fragments: dims 16 st + 8 h .. +7 of the row in two f16 parts, after a
-        // power of two that takes the row's largest value to [2^14, 2^15) and with
-        // the sign of the scale, so that the largest score has the largest product
-        float amax = 0.f;
+        if (tiles) {
+            issue(kbase, kt, wave * TF_PM_T, false);
+            tf_wait_vm<NC>();
+        } else {
+            tf_wait_vm<0>();
+        }
+        const int c = lane & (HD / 8 - 1), rw = lane / (HD / 8);
+        if (rw < 4) {
+            const float4 a = *reinterpret_cast<const float4*>(vt + rw * 4 * HD + 32 * c);
+            const float4 b = *reinterpret_cast<const float4*>(vt + rw * 4 * HD + 32 * c + 16);
+            const float qv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            float amax = 0.f;
 #pragma unroll
-        for (int st = 0; st < ST; st++)
+            for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(qv[i]));
 #pragma unroll
-            for (int i = 0; i < 8; i++) amax = fmaxf(amax, fabsf(qv[st][i]));
-        amax = fmaxf(amax, __shfl_xor(amax, 32));
-        const int eb = (int)((__float_as_uint(amax) >> 23) & 0xff);
-        int fe = amax > 0.f ? 141 - eb : 0;
-        fe = fe > 126 ? 126 : fe;
-        const float f = copysignf(__uint_as_float((uint32_t)(fe + 127) << 23), scale);
-        s2 = fabsf(scale) * 1.44269504088896340736f * __uint_as_float((uint32_t)(127 - fe) << 23);
-#pragma unroll
-        for (int st = 0; st < ST; st++)
+            for (int x = 1; x < HD / 8; x <<= 1) amax = fmaxf(amax, __shfl_xor(amax, x));
+            const int eb = (int)((__float_as_uint(amax) >> 23) & 0xff);
+            int fe = amax > 0.f ? 141 - eb : 0;
+            fe = fe > 126 ? 126 : fe;
+            const float f = copysignf(__uint_as_float((uint32_t)(fe + 127) << 23), scale);
+            tf_h8 q0, q1;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const float a = qv[st][i] * f;
-                const _Float16 hi = (_Float16)a;
-                qb[st][0][i] = hi;
-                qb[st][1][i] = (_Float16)(a - (float)hi);
+                const float v = qv[i] * f;
+                const _Float16 hi = (_Float16)v;
+                q0[i] = hi;
+                q1[i] = (_Float16)(v - (float)hi);
             }
+            const int r = 4 * wave + rw;
+            tf_h8* slot = reinterpret_cast<tf_h8*>(lds + L::Q) + 32 * c + (r ^ c);
+            slot[0] = q0;
+            slot[L::TILE / 16] = q1;
+            if (c == 0)
+                reinterpret_cast<float*>(lds + L::S2)[r] =
+                    fabsf(scale) * 1.44269504088896340736f *
+                    __uint_as_float((uint32_t)(127 - fe) << 23);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // q read, fragments written
+        if (tiles) issue(vbase, vt, wave * TF_PM_T, true);
+        __builtin_amdgcn_s_barrier();  // the copies stay in flight over it
+        asm volatile("" ::: "memory");
+        s2 = reinterpret_cast<const float*>(lds + L::S2)[l32];
+#pragma unroll
+        for (int st = 0; st < ST; st++)
+#pragma unroll
+            for (int pl = 0; pl < 2; pl++)
+                qb[st][pl] = reinterpret_cast<const tf_h8*>(
+                    lds + L::Q)[pl * (L::TILE / 16) + 32 * (2 * st + h) + (l32 ^ (2 * st + h))];
     }
 
     float mx = -1e30f, l = 0.f;  // of the row; l is this half's share
