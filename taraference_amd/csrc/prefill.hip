@@ -204,6 +204,17 @@ __device__ __forceinline__ void tf_split2(float a, float b, tf_h2& hi, tf_h2& lo
     lo = tf_h2{(_Float16)(a - (float)hi.x), (_Float16)(b - (float)hi.y)};
 }
 
+// v *= f, each product rounded (not fused into what uses it)
+__device__ __forceinline__ void tf_scores_pow2(tf_f32x16& v, float f) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        float t = v[i] * f;
+        asm("" : "+v"(t));
+        v[i] = t;
+    }
+}
+
 // r / d by the reciprocal m = ceil(2^32 / d) (0 for d = 1): the product is at
 // most one too large
 __device__ __forceinline__ uint32_t tf_div_by(uint32_t r, uint32_t d, uint32_t m) {
@@ -376,11 +387,15 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
                 sc[i] = kp <= qpos ? sc[i] : -INFINITY;
             }
         }
+        // rounded before the maximum is subtracted: a fused step would leave the
+        // maximum itself above 0 by 2^-24 of a score, past f16's range for scores
+        // of 2^28 and more
+        tf_scores_pow2(sc, s2);
         float tmax = sc[0];
 #pragma unroll
         for (int i = 1; i < 16; i++) tmax = fmaxf(tmax, sc[i]);
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float m_new = fmaxf(mx, tmax * s2);
+        const float m_new = fmaxf(mx, tmax);
         if (__ballot(m_new > mx)) {
             const float alpha = __builtin_amdgcn_exp2f(mx - m_new);
             l *= alpha;
@@ -395,8 +410,8 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
             // a NaN score counts as no key
-            const float e0 = fmaxf(__builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], s2, -mx)), 0.f);
-            const float e1 = fmaxf(__builtin_amdgcn_exp2f(__builtin_fmaf(sc[i + 1], s2, -mx)), 0.f);
+            const float e0 = fmaxf(__builtin_amdgcn_exp2f(sc[i] - mx), 0.f);
+            const float e1 = fmaxf(__builtin_amdgcn_exp2f(sc[i + 1] - mx), 0.f);
             ls += e0 + e1;
             tf_h2 hi, lo;
             tf_split2(e0, e1, hi, lo);
@@ -552,7 +567,7 @@ int tf_attn_prefill_any(const float* q, const uint16_t* k_cache, const uint16_t*
     const uint32_t g_inv = G > 1 ? (uint32_t)(((1ull << 32) + G - 1) / G) : 0;
     const uint32_t kv_inv = n_kv > 1 ? (uint32_t)(((1ull << 32) + n_kv - 1) / n_kv) : 0;
     const long long tiles = ((long long)n_q * G + TF_PM_T - 1) / TF_PM_T;
-    TF_CHECK_ARG(tiles * TF_PM_T <= INT32_MAX && tiles * n_kv <= INT32_MAX / (64 * TF_PM_WAVES));
+    TF_CHECK_ARG(tiles * TF_PM_T <= INT32_MAX && tiles * n_kv <= UINT32_MAX / (64 * TF_PM_WAVES));
     auto go = [&](auto kern, int bytes) -> int {
         const int rc = tf_set_lds_limit((const void*)kern, bytes);
         if (rc) return rc;

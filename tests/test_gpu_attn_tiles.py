@@ -63,3 +63,24 @@ def test_attn_caches_8_byte_aligned(gpu, hd):
 @pytest.mark.parametrize("hd", [64, 128])
 def test_attn_negative_scale(gpu, hd):
     run(8, 2, hd, 70, 12, scale=-0.1)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("mag", [1e4, 1e9, 1e25])
+def test_attn_large_scores(gpu, hd, mag):
+    """Scores far beyond 2^24: every weight still lies in [0, 1], so an output is
+    finite and within its V column's range (2^-22 for the two parts of P)."""
+    rng = np.random.default_rng(hd)
+    n_head, n_kv, pos0, n_q = 14, 2, 290, 20
+    L = pos0 + n_q
+    K, V = synth.kv_cache(rng, L, n_kv, hd), synth.kv_cache(rng, L, n_kv, hd)
+    q = (rng.standard_normal((n_q, n_head * hd)) * mag).astype(np.float32)
+    out = empty(n_q * n_head * hd)
+    print(f"attn large scores hd={hd} mag={mag}", flush=True)
+    call("tf_attn_prefill", P(dev(q)), P(dev(K)), P(dev(V)), P(out), n_head, n_kv, hd, pos0, n_q,
+         float(np.float32(hd ** -0.5)), S())
+    y = host(out).reshape(n_q, n_head, hd)
+    v = V.view(np.float16).astype(np.float32).reshape(L, n_kv, hd)
+    for h in range(n_head):
+        g = v[:, h // (n_head // n_kv)]
+        assert np.all(y[:, h] <= g.max(0) + 1e-5) and np.all(y[:, h] >= g.min(0) - 1e-5)
