@@ -479,7 +479,13 @@ __global__ __launch_bounds__(512) void tf_b32_kernel(TfB32Job jb) {
 
 // Q5_0 q and k and a Q8_0 v of the same row in one launch, each workgroup
 // normalizing the row for itself: the first `blocks5` workgroups take q and k,
-// the others v.
+// the others v.  At K = 896 a launch costs 3 to 5 us whatever it does (0.7 MB of
+// weights here), so what counts is their number: with the norm, SiLU, RoPE and the
+// merge of the attention in the launches around them a layer has seven instead of
+// fifteen, and 16 steps of six layers take 3.6 instead of 5.5 ms.  Measured beside
+// it and not taken: gate and up on 256, 304 or 512 workgroups instead of all that
+// are resident (3.57, 3.62, 3.53 against 3.50 ms); down quantizing its f32 row
+// itself (4864 -> 896: 6.8 us, 5.1 with the Q8 launch before it).
 template <int ITERS>
 __global__ __launch_bounds__(512) void tf_b32_norm_qkv_kernel(TfB32Job j5, TfB32Job j8,
                                                               int blocks5) {

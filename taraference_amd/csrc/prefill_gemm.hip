@@ -741,32 +741,41 @@ __global__ __launch_bounds__(256) void tf_pg_image_kernel(const float* __restric
 // x += the n_split slices of `part` (in order), then RMSNorm of the row and its
 // image: a workgroup per token, the row kept in LDS.  The sum of squares keeps
 // the reference's order (kernels/ops.cu:4-34: 256 strided fused sums, halving
-// tree).  Latency bound: a thread's loads are its n / 256 values of every
+// tree).  Latency bound: a thread's loads are n / 1024 times 16 bytes of every
 // slice, all independent (a wave per token instead, four times the loads a
-// thread: 17 us at 20 tokens and 8 slices, 11.4 at 700 and 2).
+// thread: 17 us at 20 tokens and 8 slices).  At 700 tokens of 2048 and four
+// slices 11.2 us, 15.2 with 4-byte loads and the parts of an image line written
+// from eight XCDs.
 #define TF_PG_NORM_MAX 40448  // 158 KB of row
 __global__ __launch_bounds__(256) void tf_pg_norm_image_kernel(
     float* __restrict__ x, const float* __restrict__ part, int n_split, long long split_stride,
     const float* __restrict__ w, float eps, uint8_t* __restrict__ img, int n) {
-    extern __shared__ float row[];
+    extern __shared__ __align__(16) float row[];
     __shared__ float red[1];
-    const int tid = threadIdx.x, t = blockIdx.x;
+    const int tid = threadIdx.x;
+    // Workgroup b runs on XCD b mod 8; eight consecutive tokens share the
+    // image's 128-byte lines (16 bytes each), so within a whole group of 64 they
+    // go to one XCD, whose L2 then holds whole lines to write back.
+    int t = blockIdx.x;
+    if ((t | 63) < (int)gridDim.x) t = (t & ~63) | ((t & 7) << 3) | ((t >> 3) & 7);
     float* xr = x + (size_t)t * n;
     const float* pr = part + (size_t)t * n;
-    float local = 0.f;
-#pragma unroll 4
-    for (int i = tid; i < n; i += 256) {
-        float v = xr[i];
+#pragma unroll 2
+    for (int i = 4 * tid; i < n; i += 1024) {
+        tf_pg_f4 v = *reinterpret_cast<const tf_pg_f4*>(xr + i);
         if (n_split) {
-            float a = pr[i];
+            tf_pg_f4 a = *reinterpret_cast<const tf_pg_f4*>(pr + i);
 #pragma unroll 4
-            for (int z = 1; z < n_split; z++) a += pr[(size_t)z * (size_t)split_stride + i];
+            for (int z = 1; z < n_split; z++)
+                a += *reinterpret_cast<const tf_pg_f4*>(pr + (size_t)z * (size_t)split_stride + i);
             v += a;
-            xr[i] = v;
+            *reinterpret_cast<tf_pg_f4*>(xr + i) = v;
         }
-        row[i] = v;
-        local = fmaf(v, v, local);
+        *reinterpret_cast<tf_pg_f4*>(row + i) = v;
     }
+    __syncthreads();
+    float local = 0.f;
+    for (int i = tid; i < n; i += 256) local = fmaf(row[i], row[i], local);
     // the halving tree over 256: 128 and 64 across the waves, the rest within one
     __shared__ float buf[256];
     buf[tid] = local;
@@ -814,8 +823,11 @@ __global__ __launch_bounds__(256) void tf_pg_add_kernel(float* __restrict__ x,
 // q/k/v rows of token t (position pos0 + t) from the n_split slices of their
 // GEMM (columns q | k | v): the slices' sum and the bias, q and k rotated
 // (NeoX pairs (i, i + hd/2) by (pos0+t) theta^(-2i/hd)), q to q_out, k and v
-// to the f16 cache.  A workgroup per token; a thread keeps its pair index, and
-// with it the angle, over the heads it handles (hd / 2 divides 256).
+// to the f16 cache.  A workgroup per token and 512 / hd heads (hd / 2 divides
+// 256), one round of loads a thread; the angles of the hd / 2 pairs are formed
+// once for all of its heads while the loads arrive (powf and sincosf by every
+// thread bounded it: 9 us at 700 tokens of 20 heads and three slices; all heads
+// of a token in one workgroup, a round after the other: 10 us).
 __global__ __launch_bounds__(256) void tf_pg_qkv_post_kernel(
     const float* __restrict__ part, int n_split, long long split_stride,
     const float* __restrict__ bq, const float* __restrict__ bk, const float* __restrict__ bv,
@@ -825,18 +837,28 @@ __global__ __launch_bounds__(256) void tf_pg_qkv_post_kernel(
     const int nq = n_head * hd, kvd = n_kv * hd, ld = nq + 2 * kvd;
     const float* row = part + (size_t)t * ld;
     const int i = threadIdx.x % half;
-    const float freq = powf(theta, -2.f * (float)i / (float)hd);
-    const float ang = (float)pos * freq;
-    float sn, cs;
-    sincosf(ang, &sn, &cs);
-    for (int hb = threadIdx.x / half; hb < n_head + 2 * n_kv; hb += 256 / half) {
-        const int c0 = hb * hd + i, c1 = c0 + half;
-        float x0 = row[c0], x1 = row[c1];
+    __shared__ float2 rot[256];  // cos, sin of pair i
+    const int hb = blockIdx.y * (256 / half) + threadIdx.x / half;
+    const int c0 = hb * hd + i, c1 = c0 + half;
+    float x0 = 0.f, x1 = 0.f;
+    if (hb < n_head + 2 * n_kv) {
+        x0 = row[c0];
+        x1 = row[c1];
 #pragma unroll 4
         for (int z = 1; z < n_split; z++) {
             x0 += row[(size_t)z * (size_t)split_stride + c0];
             x1 += row[(size_t)z * (size_t)split_stride + c1];
         }
+    }
+    if ((int)threadIdx.x < half) {
+        const float freq = powf(theta, -2.f * (float)i / (float)hd);
+        const float ang = (float)pos * freq;
+        float sn, cs;
+        sincosf(ang, &sn, &cs);
+        rot[i] = make_float2(cs, sn);
+    }
+    __syncthreads();
+    if (hb < n_head + 2 * n_kv) {
         const float* b = hb < n_head ? bq : hb < n_head + n_kv ? bk : bv;
         const int o = hb < n_head ? c0 : hb < n_head + n_kv ? c0 - nq : c0 - nq - kvd;
         if (b) {
@@ -844,6 +866,7 @@ __global__ __launch_bounds__(256) void tf_pg_qkv_post_kernel(
             x1 += b[o + half];
         }
         if (hb < n_head + n_kv) {
+            const float cs = rot[i].x, sn = rot[i].y;
             const float r0 = x0 * cs - x1 * sn, r1 = x0 * sn + x1 * cs;
             x0 = r0;
             x1 = r1;
@@ -1050,7 +1073,9 @@ int tf_pg_qkv_post(const TfPgPart& part, const float* bq, const float* bk, const
                    int head_dim, int pos0, int n_tok, float theta, tf_stream_t stream) {
     TF_CHECK_ARG(part.p && q_out && k_cache && v_cache && n_head > 0 && n_kv > 0 && n_tok > 0);
     TF_CHECK_ARG(head_dim > 0 && head_dim % 2 == 0 && 256 % (head_dim / 2) == 0 && pos0 >= 0);
-    hipLaunchKernelGGL(tf_pg_qkv_post_kernel, dim3(n_tok), dim3(256), 0, tf_stream(stream), part.p,
+    const int per = 512 / head_dim;  // heads of a workgroup
+    const dim3 grid(n_tok, (n_head + 2 * n_kv + per - 1) / per);
+    hipLaunchKernelGGL(tf_pg_qkv_post_kernel, grid, dim3(256), 0, tf_stream(stream), part.p,
                        part.n_split, part.stride, bq, bk, bv, q_out, k_cache, v_cache, n_head, n_kv,
                        head_dim, pos0, theta);
     return TF_LAUNCH_RESULT();
