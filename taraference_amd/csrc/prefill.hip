@@ -161,7 +161,7 @@ __global__ __launch_bounds__(256) void tf_attn_prefill_kernel(
 // LDS rows keep their 16-byte chunks xor-ed with the row, so that 16 K rows, or
 // the 4 rows x 64 bytes of a transposing read, fall on distinct banks.
 // What bounds it: long contexts, the matrix cores (two products per score and per
-// P V term) and LDS bandwidth about equally, 27 us each of the 77 us that 256
+// P V term) and LDS bandwidth about equally, 27 us each of the 74 us that 256
 // tokens of 28 heads at position 8000 take, with the softmax between them (a raised
 // wave priority for either half changed nothing); short ones, the chain of copy,
 // scores, P V and merge of one tile.  The form before it (16 queries of one head,

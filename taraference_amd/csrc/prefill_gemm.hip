@@ -825,9 +825,10 @@ __global__ __launch_bounds__(256) void tf_pg_add_kernel(float* __restrict__ x,
 // (NeoX pairs (i, i + hd/2) by (pos0+t) theta^(-2i/hd)), q to q_out, k and v
 // to the f16 cache.  A workgroup per token and 512 / hd heads (hd / 2 divides
 // 256), one round of loads a thread; the angles of the hd / 2 pairs are formed
-// once for all of its heads while the loads arrive (powf and sincosf by every
-// thread bounded it: 9 us at 700 tokens of 20 heads and three slices; all heads
-// of a token in one workgroup, a round after the other: 10 us).
+// once for all of its heads while the loads arrive.  Bound by its bytes: 700
+// tokens of 20 heads and three slices are 30 MB, 6.3 us at the rate of a large
+// copy, and take 8.6 us (9.1 with powf and sincosf in every thread, 9.8 with all
+// heads of a token in one workgroup, a round after the other).
 __global__ __launch_bounds__(256) void tf_pg_qkv_post_kernel(
     const float* __restrict__ part, int n_split, long long split_stride,
     const float* __restrict__ bq, const float* __restrict__ bk, const float* __restrict__ bv,
