@@ -59,7 +59,7 @@ struct TfB32Job {
     const float* norm_w;  // TF_B32_SRC_NORM
     float eps;
     const float* part;  // TF_B32_SRC_FLASH: [head][split](m, l, O[head_dim])
-    int parts, head_dim;
+    int parts, head_dim;  // parts: 8 or 16
     int paired;  // task 2j: column j of w[0], 2j + 1: of w[1]; out[0] = silu(.) * (.)
 };
 
@@ -115,42 +115,46 @@ __device__ __forceinline__ float tf_b32_rms_scale(const TfB32Job& jb, float* buf
     return buf[256];
 }
 
-// Four values of the attention output from its partials, as the reduce kernel
-// forms them (log-sum-exp weights, O / max(l, 1e-20)); eight partials in flight.
+// Four values of the attention output from its 8 R partials, bit-identical to
+// tf_flash_reduce_kernel's: the maximum of all; partials i, i + 8 (weights
+// e^(m - max)) fused into one sum, the eight sums in order; O / max(l, 1e-20).
+// All loads are independent and in flight together.
+template <int R>
 __device__ __forceinline__ float4 tf_b32_merge4(const TfB32Job& jb, int e) {
     const int hd = jb.head_dim, po = 2 + hd, h = e / hd;
-    const float* ph = jb.part + (size_t)h * jb.parts * po;
+    const float* ph = jb.part + (size_t)h * (8 * R) * po;  // 8-byte aligned: po is even
     const int d = 2 + e - h * hd;
-    float m = -1e30f, l = 0.f;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s0 = 0; s0 < jb.parts; s0 += 8) {  // parts % 8 == 0
-        float2 ml[8], a[8], b[8];
+    float2 ml[8 * R], a[8 * R], b[8 * R];
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const float* p = ph + (size_t)(s0 + k) * po;  // 8-byte aligned: po is even
-            ml[k] = *reinterpret_cast<const float2*>(p);
-            a[k] = *reinterpret_cast<const float2*>(p + d);
-            b[k] = *reinterpret_cast<const float2*>(p + d + 2);
-        }
-        float mm = m;
-#pragma unroll
-        for (int k = 0; k < 8; k++) mm = fmaxf(mm, ml[k].x);
-        const float f = __expf(m - mm);
-        m = mm;
-        l *= f;
-        acc = make_float4(acc.x * f, acc.y * f, acc.z * f, acc.w * f);
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const float w = __expf(ml[k].x - mm);
-            l += w * ml[k].y;
-            acc.x += w * a[k].x;
-            acc.y += w * a[k].y;
-            acc.z += w * b[k].x;
-            acc.w += w * b[k].y;
-        }
+    for (int k = 0; k < 8 * R; k++) {
+        const float* p = ph + (size_t)k * po;
+        ml[k] = *reinterpret_cast<const float2*>(p);
+        a[k] = *reinterpret_cast<const float2*>(p + d);
+        b[k] = *reinterpret_cast<const float2*>(p + d + 2);
     }
-    const float inv = 1.f / fmaxf(l, 1e-20f);
-    return make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    float m = ml[0].x;
+#pragma unroll
+    for (int k = 1; k < 8 * R; k++) m = fmaxf(m, ml[k].x);
+    float l = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        float ls = 0.f;
+        float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int k = i; k < 8 * R; k += 8) {
+            const float w = __expf(ml[k].x - m);
+            ls = fmaf(w, ml[k].y, ls);
+            t.x = fmaf(w, a[k].x, t.x);
+            t.y = fmaf(w, a[k].y, t.y);
+            t.z = fmaf(w, b[k].x, t.z);
+            t.w = fmaf(w, b[k].y, t.w);
+        }
+        l += ls;
+        acc = make_float4(acc.x + t.x, acc.y + t.y, acc.z + t.z, acc.w + t.w);
+    }
+    l = fmaxf(l, 1e-20f);
+    return make_float4(acc.x / l, acc.y / l, acc.z / l, acc.w / l);
 }
 
 // Build the activation image; all threads of the workgroup; ends with a
@@ -166,7 +170,8 @@ __device__ __forceinline__ void tf_b32_stage(const TfB32Job& jb, uint8_t* lds) {
         if constexpr (SK == TF_B32_SRC_NORM) scale = tf_b32_rms_scale(jb, xs + 32 * G);
         for (int i = threadIdx.x; i < G * 8; i += blockDim.x) {
             float4 v;
-            if constexpr (SK == TF_B32_SRC_FLASH) v = tf_b32_merge4(jb, 4 * i);
+            if constexpr (SK == TF_B32_SRC_FLASH)
+                v = jb.parts == 8 ? tf_b32_merge4<1>(jb, 4 * i) : tf_b32_merge4<2>(jb, 4 * i);
             else v = *reinterpret_cast<const float4*>(jb.x + 4 * i);
             if constexpr (SK == TF_B32_SRC_NORM) {
                 const float4 w = *reinterpret_cast<const float4*>(jb.norm_w + 4 * i);
@@ -389,13 +394,16 @@ __device__ __forceinline__ TfB32Task tf_b32_task(const TfB32Job& jb, int t) {
 // units of work per row, all loaded up front, and the next task's loads are
 // issued before this task is computed; ITERS == 0: a plain loop.
 //
-// PAIRED (SPR <= 8): the even units of a wave hold gate rows, the odd ones the
-// up rows of the same output, which leaves as silu(gate) * up.
+// PAIRED (SPR == 8): the even units of a wave hold gate rows, the odd ones the
+// up rows of the same output, which leaves as silu(gate) * up.  A quad keeps two
+// sums, of its blocks sir + 16 i and sir + 8 + 16 i: those of the quads of a
+// 16-quad row, added as tf_group_sum<64> adds them, so that gate and up are
+// bit-identical to their own launches'.
 template <int FMT, int SK, int SPR, int ITERS, bool PAIRED = false>
 __device__ __forceinline__ void tf_b32_body(const TfB32Job& jb, uint8_t* lds, int wave,
                                             int nwaves) {
     constexpr int UNITS = 16 / SPR;
-    static_assert(!PAIRED || UNITS % 2 == 0, "gate and up rows of one wave");
+    static_assert(!PAIRED || SPR == 8, "gate and up rows of one wave, two sums a quad");
     const int lane = threadIdx.x & 63;
     const int p = lane & 3, slot = lane >> 2, unit = slot / SPR, sir = slot % SPR;
     const int n_tasks = (jb.n_tot + UNITS - 1) / UNITS;
@@ -405,9 +413,10 @@ __device__ __forceinline__ void tf_b32_body(const TfB32Job& jb, uint8_t* lds, in
     auto u_lo = [&](const TfB32Task& t) { return PAIR ? (t.b0 >> 1) : t.b0; };
     auto u_hi = [&](const TfB32Task& t) { return PAIR ? ((t.b1 + 1) >> 1) : t.b1; };
 
-    auto finish = [&](const TfB32Task& t, float acc) {
+    auto finish = [&](const TfB32Task& t, float acc, [[maybe_unused]] float acc2) {
         acc = tf_group_sum<4 * SPR>(acc);
         if constexpr (PAIRED) {
+            acc += tf_group_sum<4 * SPR>(acc2);
             const float up = __shfl(acc, (lane + 4 * SPR) & 63, 64);
             if (t.valid && (unit & 1) == 0 && (lane & (4 * SPR - 1)) == 0)
                 t.out[t.j] = (acc / (1.f + __expf(-acc))) * up;
@@ -441,15 +450,19 @@ __device__ __forceinline__ void tf_b32_body(const TfB32Job& jb, uint8_t* lds, in
             const int nt = task + nwaves;
             const TfB32Task tn = tf_b32_task(jb, nt * UNITS + unit);
             if (nt < n_tasks) load_all(tn, nxt);
-            float acc = 0.f;
+            float acc = 0.f, acc2 = 0.f;
             const int lo = u_lo(tc), hi = u_hi(tc);
 #pragma unroll
             for (int i = 0; i < ITERS; i++) {
                 const int k = lo + sir + i * SPR;
                 const float c = tf_b32_step<FMT>(cur[i], k < hi ? k : lo, p, tc.b0, tc.b1, lds, G);
-                if (k < hi) acc += c;
+                if (PAIRED && (i & 1)) {
+                    if (k < hi) acc2 += c;
+                } else if (k < hi) {
+                    acc += c;
+                }
             }
-            finish(tc, acc);
+            finish(tc, acc, acc2);
 #pragma unroll
             for (int i = 0; i < ITERS; i++) cur[i] = nxt[i];
             tc = tn;
@@ -465,7 +478,7 @@ __device__ __forceinline__ void tf_b32_body(const TfB32Job& jb, uint8_t* lds, in
                 tf_b32_load<FMT>(t.col, k, p, r);
                 acc += tf_b32_step<FMT>(r, k, p, t.b0, t.b1, lds, G);
             }
-            finish(t, acc);
+            finish(t, acc, 0.f);
         }
     }
 }
