@@ -283,7 +283,7 @@ struct tf_model {
     void head(hipStream_t s, const float* row) {
         const tf_model_config& c = cfg;
         if (tf::global_q8_ok(output) && (int)output.n_rows == c.n_embd && c.n_embd % 128 == 0 &&
-            c.n_embd <= 8192) {  // the rows that tf_norm_quant takes
+            c.n_embd <= 8192 && ((uintptr_t)output_norm & 7) == 0) {  // what tf_norm_quant takes
             tf::check(tf_norm_quant(row, output_norm, c.rms_eps, xb, q8_x, q8_d, c.n_embd, s),
                       "norm_quant");
             tf::gemv_global_q8(s, output, logits, nullptr, GemvResidual::none(), q8_x, q8_d);

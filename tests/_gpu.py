@@ -39,3 +39,23 @@ def S():
 def call(name, *args):
     print(f"[gpu] {name}", flush=True)
     capi.call(name, *args)
+
+
+class Unaligned(np.ndarray):
+    """A vector (a.view(Unaligned)) that model_class() places 4 bytes past a
+    16-byte boundary."""
+
+
+def model_class():
+    from taraference_amd.model import DecodeModel
+
+    class Model(DecodeModel):
+        def _f32(self, a):
+            if not isinstance(a, Unaligned):
+                return super()._f32(a)
+            t = torch.zeros(a.size + 4, device="cuda")
+            t[1:1 + a.size] = torch.from_numpy(np.array(a, np.float32))
+            self._keep.append(t)
+            return t.data_ptr() + 4
+
+    return Model

@@ -23,7 +23,7 @@ import torch
 
 import oracle
 from taraference_amd import synth
-from _gpu import P, S, call, dev, empty, host
+from _gpu import P, S, Unaligned, call, dev, empty, host, model_class
 from _model_ref import RefModelMixed
 from _util import q8_0_dequant
 from test_gpu_q05_model import f16, write_model
@@ -92,30 +92,16 @@ def test_fused_layers(gpu, tmp_path, heads, kv, ff, vocab, max_seq):
 def make(cfg, layers, emb, max_seq, shift=()):
     """A DecodeModel; the vectors named in `shift` (attn_norm, ffn_norm or
     output_norm) lie 4 bytes past a 16-byte boundary."""
-    from taraference_amd.model import DecodeModel
-
-    class Shifted(np.ndarray):
-        pass
-
-    class Model(DecodeModel):
-        def _f32(self, a):
-            if not isinstance(a, Shifted):
-                return super()._f32(a)
-            t = torch.zeros(a.size + 4, device="cuda")
-            t[1:1 + a.size] = torch.from_numpy(np.array(a, np.float32))
-            self._keep.append(t)
-            return t.data_ptr() + 4
-
     rng = np.random.default_rng(9)
 
     def norm(name, v):
         v = np.asarray(v * rng.uniform(0.8, 1.2, v.size), np.float32)
-        return v.view(Shifted) if name in shift else v
+        return v.view(Unaligned) if name in shift else v
 
     layers = [dict(L, attn_norm=norm("attn_norm", L["attn_norm"]),
                    ffn_norm=norm("ffn_norm", L["ffn_norm"])) for L in layers]
     onorm = norm("output_norm", np.ones(cfg["n_embd"], np.float32))
-    return Model(dict(cfg, max_seq=max_seq), layers, emb, output_norm=onorm), layers, onorm
+    return model_class()(dict(cfg, max_seq=max_seq), layers, emb, output_norm=onorm), layers, onorm
 
 
 @pytest.mark.parametrize("heads,kv", [(2, 1), (4, 2), (5, 5), (14, 2), (32, 4)])
@@ -181,3 +167,18 @@ def test_merge_wo_as_separate_launches(gpu, heads, kv, max_seq):
     call("tf_gemv_q8_0_q8", E, P(xq), P(xd), P(lg), e, vocab, ecb, 0, None, 0, None, S())
     np.testing.assert_array_equal(m.logits(), host(lg))
     m.close()
+
+
+def test_output_norm_4_byte_aligned(gpu):
+    """The head's fused norm + Q8 takes 8-byte aligned norms; others go through
+    tf_rms_norm and tf_quantize_q8, with the same bits."""
+    cfg = dict(n_layer=1, n_embd=896, n_ff=256, n_head=14, n_kv=2, head_dim=64, n_vocab=130,
+               rope_theta=1e6, rms_eps=1e-6)
+    rng = np.random.default_rng(1)
+    layers, emb = [synth.qwen05_layer(rng, cfg, 0)], synth.qwen05_embedding(rng, cfg)
+    a, _, _ = make(cfg, layers, emb, 40)
+    b, _, _ = make(cfg, layers, emb, 40, ("output_norm",))
+    assert a.forward(5, 0) == b.forward(5, 0)
+    np.testing.assert_array_equal(a.logits(), b.logits())
+    a.close()
+    b.close()

@@ -19,6 +19,8 @@ starts with prefill's token and runs on the decode path.
 import numpy as np
 import pytest
 
+from taraference_amd import synth
+from _gpu import Unaligned, model_class
 from test_gpu_model import TINY, build
 
 pytestmark = pytest.mark.gpu
@@ -67,6 +69,29 @@ def test_prefill_matches_reference(gpu, ci, n_prompt, n_more):
         check_kv(gm, rm, cfg["n_layer"], slice(0, n_prompt + n_more))
         check_logits(gm, rl2, rt2, tok2)
     gm.close()
+
+
+@pytest.mark.parametrize("name", ["output_norm"])
+def test_prefill_norms_4_byte_aligned(gpu, name):
+    """A norm vector that starts 4 bytes past a 16-byte boundary: the same bits."""
+    cfg = TINY[0]
+    rng = np.random.default_rng(77)
+    layers = [synth.qwen_layer(rng, cfg, li) for li in range(cfg["n_layer"])]
+    emb = synth.qwen_embedding(rng, cfg)
+    vec = {n: rng.uniform(0.8, 1.2, cfg["n_embd"]).astype(np.float32)
+           for n in ("attn_norm", "ffn_norm", "output_norm")}
+    prompt = rng.integers(0, cfg["n_vocab"], 20).tolist()
+    out = []
+    for u in (False, True):
+        v = dict(vec, **({name: vec[name].view(Unaligned)} if u else {}))
+        m = model_class()(dict(cfg, max_seq=40),
+                          [dict(L, attn_norm=v["attn_norm"], ffn_norm=v["ffn_norm"])
+                           for L in layers], emb, output_norm=v["output_norm"])
+        print(f"prefill {name} unaligned={u}", flush=True)
+        out.append((m.prefill(prompt, 0), m.logits()))
+        m.close()
+    assert out[0][0] == out[1][0]
+    np.testing.assert_array_equal(out[0][1], out[1][1])
 
 
 def test_generate_after_prefill(gpu):
