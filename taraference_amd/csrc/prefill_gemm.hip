@@ -795,7 +795,9 @@ __global__ __launch_bounds__(256) void tf_pg_norm_image_kernel(
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const tf_pg_f4 a = *reinterpret_cast<const tf_pg_f4*>(row + k + 4 * i);
-            const tf_pg_f4 g = *reinterpret_cast<const tf_pg_f4*>(w + k + 4 * i);
+            // the caller's vector, at any multiple of 4 bytes
+            const tf_pg_f4 g = __builtin_bit_cast(
+                tf_pg_f4, tf_pg_ld16(reinterpret_cast<const uint8_t*>(w), 4 * (k + 4 * i)));
 #pragma unroll
             for (int q = 0; q < 4; q++) v[0][i][q] = a[q] * scale * g[q];
         }
@@ -983,7 +985,8 @@ size_t tf_pg_image_bytes(int n_rows, int n_tok) {
 }
 
 int tf_pg_image(const float* x, uint8_t* img, int n_rows, int n_tok, tf_stream_t stream) {
-    TF_CHECK_ARG(x && img && n_rows >= 256 && n_tok > 0);
+    TF_CHECK_ARG(x && img && n_rows >= 256 && n_rows % 4 == 0 && n_tok > 0);
+    TF_CHECK_ARG((((uintptr_t)x | (uintptr_t)img) & 15) == 0);
     hipLaunchKernelGGL(tf_pg_image_kernel, dim3(n_rows / 256, (n_tok + 31) / 32), dim3(256), 0,
                        tf_stream(stream), x, img, n_rows, n_tok);
     return TF_LAUNCH_RESULT();
@@ -993,6 +996,8 @@ int tf_pg_norm_image(float* x, const TfPgPart* part, const float* w, float eps, 
                      int n_tok, tf_stream_t stream) {
     TF_CHECK_ARG(x && w && img && n >= 256 && n % 256 == 0 && n_tok > 0);
     TF_CHECK_ARG(n <= TF_PG_NORM_MAX);
+    TF_CHECK_ARG((((uintptr_t)x | (uintptr_t)img) & 15) == 0);
+    TF_CHECK_ARG(!part || (((uintptr_t)part->p & 15) == 0 && part->stride % 4 == 0));
     const int lds = n * (int)sizeof(float);
     const int rc = tf_set_lds_limit((const void*)tf_pg_norm_image_kernel, lds);
     if (rc) return rc;
@@ -1003,7 +1008,8 @@ int tf_pg_norm_image(float* x, const TfPgPart* part, const float* w, float eps, 
 }
 
 int tf_pg_add_row(float* x, const TfPgPart& part, int row, int n, tf_stream_t stream) {
-    TF_CHECK_ARG(x && part.p && part.n_split > 0 && n % 4 == 0);
+    TF_CHECK_ARG(x && part.p && part.n_split > 0 && n % 4 == 0 && part.stride % 4 == 0);
+    TF_CHECK_ARG((((uintptr_t)x | (uintptr_t)part.p) & 15) == 0);
     hipLaunchKernelGGL(tf_pg_add_kernel, dim3((n / 4 + 255) / 256), dim3(256), 0, tf_stream(stream),
                        x + (size_t)row * n, part.p + (size_t)row * n, n / 4, part.n_split,
                        part.stride);

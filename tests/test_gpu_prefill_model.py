@@ -71,7 +71,7 @@ def test_prefill_matches_reference(gpu, ci, n_prompt, n_more):
     gm.close()
 
 
-@pytest.mark.parametrize("name", ["output_norm"])
+@pytest.mark.parametrize("name", ["attn_norm", "ffn_norm", "output_norm"])
 def test_prefill_norms_4_byte_aligned(gpu, name):
     """A norm vector that starts 4 bytes past a 16-byte boundary: the same bits."""
     cfg = TINY[0]
