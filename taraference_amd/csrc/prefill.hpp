@@ -21,7 +21,7 @@ struct TfPgPart {
 };
 
 // x[t] += part[t] (part may be null), then img = rmsnorm(x) * w.
-// n % 256 == 0, n <= 40448.
+// n % 256 == 0; w at any multiple of 4 bytes.
 int tf_pg_norm_image(float* x, const TfPgPart* part, const float* w, float eps, uint8_t* img, int n,
                      int n_tok, tf_stream_t stream);
 // x[row] += part[row], rows of n.

@@ -746,11 +746,14 @@ __global__ __launch_bounds__(256) void tf_pg_image_kernel(const float* __restric
 // thread: 17 us at 20 tokens and 8 slices).  At 700 tokens of 2048 and four
 // slices 11.2 us, 15.2 with 4-byte loads and the parts of an image line written
 // from eight XCDs.
+// Rows wider than TF_PG_NORM_MAX values do not fit the LDS (ROW false): the sums go
+// to x as ever and the row is read back from there.
 #define TF_PG_NORM_MAX 40448  // 158 KB of row
+template <bool ROW>
 __global__ __launch_bounds__(256) void tf_pg_norm_image_kernel(
     float* __restrict__ x, const float* __restrict__ part, int n_split, long long split_stride,
     const float* __restrict__ w, float eps, uint8_t* __restrict__ img, int n) {
-    extern __shared__ __align__(16) float row[];
+    extern __shared__ __align__(16) float row_lds[];
     __shared__ float red[1];
     const int tid = threadIdx.x;
     // Workgroup b runs on XCD b mod 8; eight consecutive tokens share the
@@ -759,6 +762,7 @@ __global__ __launch_bounds__(256) void tf_pg_norm_image_kernel(
     int t = blockIdx.x;
     if ((t | 63) < (int)gridDim.x) t = (t & ~63) | ((t & 7) << 3) | ((t >> 3) & 7);
     float* xr = x + (size_t)t * n;
+    float* const row = ROW ? row_lds : xr;
     const float* pr = part + (size_t)t * n;
 #pragma unroll 2
     for (int i = 4 * tid; i < n; i += 1024) {
@@ -771,7 +775,7 @@ __global__ __launch_bounds__(256) void tf_pg_norm_image_kernel(
             v += a;
             *reinterpret_cast<tf_pg_f4*>(xr + i) = v;
         }
-        *reinterpret_cast<tf_pg_f4*>(row + i) = v;
+        if constexpr (ROW) *reinterpret_cast<tf_pg_f4*>(row + i) = v;
     }
     __syncthreads();
     float local = 0.f;
@@ -995,16 +999,18 @@ int tf_pg_image(const float* x, uint8_t* img, int n_rows, int n_tok, tf_stream_t
 int tf_pg_norm_image(float* x, const TfPgPart* part, const float* w, float eps, uint8_t* img, int n,
                      int n_tok, tf_stream_t stream) {
     TF_CHECK_ARG(x && w && img && n >= 256 && n % 256 == 0 && n_tok > 0);
-    TF_CHECK_ARG(n <= TF_PG_NORM_MAX);
     TF_CHECK_ARG((((uintptr_t)x | (uintptr_t)img) & 15) == 0);
     TF_CHECK_ARG(!part || (((uintptr_t)part->p & 15) == 0 && part->stride % 4 == 0));
-    const int lds = n * (int)sizeof(float);
-    const int rc = tf_set_lds_limit((const void*)tf_pg_norm_image_kernel, lds);
-    if (rc) return rc;
-    hipLaunchKernelGGL(tf_pg_norm_image_kernel, dim3(n_tok), dim3(256), lds,
-                       tf_stream(stream), x, part ? part->p : nullptr, part ? part->n_split : 0,
-                       part ? part->stride : 0, w, eps, img, n);
-    return TF_LAUNCH_RESULT();
+    auto go = [&](auto kern, int lds) -> int {
+        const int rc = tf_set_lds_limit((const void*)kern, lds);
+        if (rc) return rc;
+        hipLaunchKernelGGL(kern, dim3(n_tok), dim3(256), lds, tf_stream(stream), x,
+                           part ? part->p : nullptr, part ? part->n_split : 0,
+                           part ? part->stride : 0, w, eps, img, n);
+        return TF_LAUNCH_RESULT();
+    };
+    if (n <= TF_PG_NORM_MAX) return go(tf_pg_norm_image_kernel<true>, n * (int)sizeof(float));
+    return go(tf_pg_norm_image_kernel<false>, 0);
 }
 
 int tf_pg_add_row(float* x, const TfPgPart& part, int row, int n, tf_stream_t stream) {
