@@ -154,8 +154,11 @@ __global__ __launch_bounds__(256) void tf_attn_prefill_kernel(
 //       row (2^-22 relative per product; K is f16, the products are exact);
 //   softmax over the lane's 16 keys and the other half's 16 (one exchange), in
 //       powers of two; O is rescaled only where a row's maximum moved;
-//   O^T[dim][row] += V^T P^T with P in two f16 parts (2^-22): k index i of half
-//       h in step s stands for key 16 s + 8 (i / 4) + 4 h + i % 4, which is how
+//   O^T[dim][row] += V^T P^T with 2^14 P in two f16 parts: 2^-22 of a weight, and
+//       2^-39 of the row's largest where a weight is below 2^-17 of it (unscaled the
+//       parts end at 2^-24: 8000 keys e^-17 below a sink lost half their share).
+//       l stays unscaled; the merge takes 2^14 out again.  k index i of half h in
+//       step s stands for key 16 s + 8 (i / 4) + 4 h + i % 4, which is how
 //       the scores already lie, so P needs no exchange; the V operand is two
 //       transposing LDS reads (ds_read_b64_tr_b16: four keys of a lane's dim).
 // LDS rows keep their 16-byte chunks xor-ed with the row, so that 16 K rows, or
@@ -169,7 +172,7 @@ __global__ __launch_bounds__(256) void tf_attn_prefill_kernel(
 // vector ALU) took 234 us there, 16.5 where this takes 11.0 for a fresh 512-token
 // prompt of 16 heads, 33 against 7.7 for 400 tokens of 14 heads of 64, 5.1 and 5.1
 // for 5 tokens (q split by each wave for itself instead of once: 13.4, 9.1 and 5.1
-// us for these three).  Error against 64 bits 5.5e-7 at 8000 and
+// us for these three).  Error against 64 bits 5.1e-7 at 8000 and
 // 2.5e-7 at 512, before 6.7e-7 and 2.7e-7.
 #define TF_PM_WAVES 8
 #define TF_PM_T 32  // keys per tile, rows per workgroup
@@ -198,9 +201,14 @@ __device__ __forceinline__ void tf_wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// e = hi + lo in f16 parts, two values at a time
+// 2^14 e = hi + lo in f16 parts, two values at a time.  hi is opaque to the compiler,
+// which would otherwise convert each value a second time for lo's difference.
 __device__ __forceinline__ void tf_split2(float a, float b, tf_h2& hi, tf_h2& lo) {
-    hi = tf_h2{(_Float16)a, (_Float16)b};
+    a *= 0x1p14f;
+    b *= 0x1p14f;
+    uint32_t h = __builtin_bit_cast(uint32_t, tf_h2{(_Float16)a, (_Float16)b});
+    asm("" : "+v"(h));
+    hi = __builtin_bit_cast(tf_h2, h);
     lo = tf_h2{(_Float16)(a - (float)hi.x), (_Float16)(b - (float)hi.y)};
 }
 
@@ -409,9 +417,11 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
         float ls = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
-            // a NaN score counts as no key
-            const float e0 = fmaxf(__builtin_amdgcn_exp2f(sc[i] - mx), 0.f);
-            const float e1 = fmaxf(__builtin_amdgcn_exp2f(sc[i + 1] - mx), 0.f);
+            // a NaN score counts as no key (one instruction: med3 with 0 and 1 is the
+            // exponential's own clamp)
+            const float e0 = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(sc[i] - mx), 0.f, 1.f);
+            const float e1 =
+                __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(sc[i + 1] - mx), 0.f, 1.f);
             ls += e0 + e1;
             tf_h2 hi, lo;
             tf_split2(e0, e1, hi, lo);
@@ -475,7 +485,7 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
     float ltot = 0.f;
     for (int w = 0; w < nw; w++)
         ltot += ml[(TF_PM_WAVES + w) * TF_PM_T + mr] * __builtin_amdgcn_exp2f(ml[w * TF_PM_T + mr] - mall);
-    float inv = 1.f / fmaxf(ltot, 1e-20f);
+    float inv = 0x1p-14f / fmaxf(ltot, 1e-20f);  // O carries 2^14 P
     if (mall < -1.4e29f) inv = 0.f;      // no score above the mask: nothing to attend to
     if (mall == INFINITY) inv = NAN;     // an infinite score has no softmax
     const int qo = tf_div_by(r, G, g_inv);

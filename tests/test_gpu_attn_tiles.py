@@ -2,11 +2,12 @@
 edges of its tiles: 32 (query, head) rows a workgroup, 32 keys a tile, eight
 waves that share the tiles.  Against the fp64 softmax attention of the oracle.
 
-Tolerance: q and the probabilities are held in two f16 parts (2^-22 of the
-row's largest q, of each p), K and V are f16 and the products exact.  A score
-is off by at most 2^-22 max|q| sum|k| scale (under 2e-5 here: 2^-22 * 4 * 128 *
-0.8 / 8) plus as much again from fp32 summation, and an output is a mean of V
-rows whose weights are off by that: 4e-5 max|V|.
+Tolerance: q and 2^14 p are held in two f16 parts (2^-22 of the row's largest q;
+2^-22 of each weight p, and of p below 2^-17 2^-39, the largest being 1), K and V
+are f16 and the products exact.  A score is off by at most 2^-22 max|q| sum|k| scale
+(under 2e-5 here: 2^-22 * 4 * 128 * 0.8 / 8) plus as much again from fp32
+summation, and an output is a mean of V rows whose weights are off by that: 4e-5
+max|V|, and n 2^-39 max|V| for n keys (6e-8 at 32768).
 """
 import numpy as np
 import pytest
@@ -84,3 +85,32 @@ def test_attn_large_scores(gpu, hd, mag):
     for h in range(n_head):
         g = v[:, h // (n_head // n_kv)]
         assert np.all(y[:, h] <= g.max(0) + 1e-5) and np.all(y[:, h] >= g.min(0) - 1e-5)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attn_sinks(gpu, hd):
+    """Eight keys, one in each wave's first tile, 17 above 8000 others and with V = 0:
+    the others' weights are e^-17 (below 2^-24), their share of the output 4e-5 max|V|
+    of which 4e-5 may be off by the scores, and 1e-7 by the 2^-39 steps (8000 2^-39 =
+    1.5e-8) and fp32."""
+    rng = np.random.default_rng(hd)
+    n_head, n_kv, pos0, n_q = 4, 2, 7990, 18
+    L, scale = pos0 + n_q, float(np.float32(hd ** -0.5))
+    q = np.zeros((n_q, n_head, hd), np.float32)
+    q[..., 0] = np.float32(17 / 16 / scale)
+    q[..., 1] = rng.uniform(-1, 1, (n_q, n_head)) / scale
+    K = np.zeros((L, n_kv, hd), np.float16)
+    V = rng.uniform(0.5, 1, (L, n_kv, hd)).astype(np.float16)
+    K[..., 1] = rng.uniform(-0.5, 0.5, (L, n_kv))
+    sinks = 32 * np.arange(8)
+    K[sinks, :, 0], V[sinks] = 16, 0
+    Kb, Vb = K.view(np.uint16).reshape(L, -1), V.view(np.uint16).reshape(L, -1)
+    out = empty(n_q * n_head * hd)
+    print(f"attn sinks hd={hd}", flush=True)
+    call("tf_attn_prefill", P(dev(q)), P(dev(Kb)), P(dev(Vb)), P(out), n_head, n_kv, hd, pos0, n_q,
+         scale, S())
+    y = host(out).reshape(n_q, -1)
+    for i in (0, n_q - 1):
+        ref = oracle.attn_f64(q[i].reshape(-1), Kb, Vb, n_head, n_kv, hd, pos0 + i + 1, scale)
+        assert 2e-5 < np.abs(ref).min()
+        assert np.abs(y[i] - ref).max() <= 4e-5 * np.abs(ref).max() + 1e-7
