@@ -276,7 +276,7 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
             return (uint32_t)(r < last ? r : last) * row_bytes + 16 * (c ^ sw) + (p & 15);
         };
         if (rmax >= TF_PM_T - 1) {
-#pragma unroll
+#pragma unroll(NC > 16 ? 16 : NC)  // 32 copies at once do not fit the registers
             for (int i = 0; i < NC; i++)
                 tf_lds_dma_s<DW>(tb, off(i, TF_PM_T), ldst + 64 * DW * i);
         } else {
