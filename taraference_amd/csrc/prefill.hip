@@ -231,6 +231,37 @@ __device__ __forceinline__ uint32_t tf_div_by(uint32_t r, uint32_t d, uint32_t m
     return t * d > r ? t - 1 : t;
 }
 
+// A head_dim 64 row in which something is not finite, in fp32 as the vector form
+// takes it (an infinity in q, K or V times one f16 part of the other operand is NaN
+// where the product is not): a NaN or -inf score is no key, a +inf one makes the row
+// NaN.  The row's 16 threads take four dims each, one key after the other.
+__device__ __noinline__ float4 tf_attn_row64(const float* q, const uint8_t* kbase,
+                                             const uint8_t* vbase, uint32_t row_bytes, int n_keys,
+                                             float scale) {
+    const int m = threadIdx.x & 15;
+    const float4 a = *reinterpret_cast<const float4*>(q + 4 * m);
+    float mx = -1e30f, l = 0.f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int t = 0; t < n_keys; t++) {
+        const size_t off = (size_t)t * row_bytes + 8 * m;
+        const uint2 k = *reinterpret_cast<const uint2*>(kbase + off);
+        const uint2 v = *reinterpret_cast<const uint2*>(vbase + off);
+        const float s = scale * tf_row16_sum(a.x * tf_h2f(k.x) + a.y * tf_h2f(k.x >> 16) +
+                                             a.z * tf_h2f(k.y) + a.w * tf_h2f(k.y >> 16));
+        const float m_new = fmaxf(mx, s);
+        const float alpha = __expf(mx - m_new);
+        const float e = s > -1e29f ? __expf(s - m_new) : 0.f;
+        mx = m_new;
+        l = l * alpha + e;
+        acc.x = acc.x * alpha + e * tf_h2f(v.x);
+        acc.y = acc.y * alpha + e * tf_h2f(v.x >> 16);
+        acc.z = acc.z * alpha + e * tf_h2f(v.y);
+        acc.w = acc.w * alpha + e * tf_h2f(v.y >> 16);
+    }
+    const float inv = 1.f / fmaxf(l, 1e-20f);
+    return make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+}
+
 // DW: bytes a lane copies (16; 4 where the caches are only 8-byte aligned)
 template <int HD, int DW>
 __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kernel(
@@ -357,6 +388,7 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
     }
 
     float mx = -1e30f, l = 0.f;  // of the row; l is this half's share
+    [[maybe_unused]] bool nan_row = false;
     tf_f32x16 o[DB];
 #pragma unroll
     for (int db = 0; db < DB; db++)
@@ -400,8 +432,16 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
         // of 2^28 and more
         tf_scores_pow2(sc, s2);
         float tmax = sc[0];
+        if constexpr (HD == 64) {  // the largest of the lane's scores, or NaN if it has one
 #pragma unroll
-        for (int i = 1; i < 16; i++) tmax = fmaxf(tmax, sc[i]);
+            for (int i = 1; i < 16; i++) tmax = __builtin_elementwise_maximum(tmax, sc[i]);
+            nan_row |= tmax != tmax;
+        }
+        if (HD == 128 || __ballot(tmax != tmax)) {
+            tmax = sc[0];
+#pragma unroll
+            for (int i = 1; i < 16; i++) tmax = fmaxf(tmax, sc[i]);
+        }
         tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
         const float m_new = fmaxf(mx, tmax);
         if (__ballot(m_new > mx)) {
@@ -457,6 +497,7 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
     // merge the waves that had tiles
     const int nw = n_t < TF_PM_WAVES ? n_t : TF_PM_WAVES;
     float* ml = reinterpret_cast<float*>(lds + L::ML);
+    if (HD == 64 && nan_row) l = NAN;
     l += __shfl_xor(l, 32);
     if (h == 0) {
         ml[wave * TF_PM_T + l32] = mx;
@@ -489,7 +530,8 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
     if (mall < -1.4e29f) inv = 0.f;      // no score above the mask: nothing to attend to
     if (mall == INFINITY) inv = NAN;     // an infinite score has no softmax
     const int qo = tf_div_by(r, G, g_inv);
-    float* dst = out + ((size_t)qo * n_head + (size_t)kv_h * G + (r - qo * G)) * HD;
+    const size_t row = ((size_t)qo * n_head + (size_t)kv_h * G + (r - qo * G)) * HD;
+    float* dst = out + row;
 #pragma unroll
     for (int c = 0; c < HD / 64; c++) {
         const int d0 = 4 * (tid & 15) + 64 * c;
@@ -501,8 +543,13 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
             acc.z += v.z;
             acc.w += v.w;
         }
-        *reinterpret_cast<float4*>(dst + d0) =
-            make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+        acc = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+        if constexpr (HD == 64) {
+            const float sum = (acc.x + acc.y) + (acc.z + acc.w);
+            if (tf_row16_max(ltot != ltot || sum != sum ? 1.f : 0.f) > 0.f)
+                acc = tf_attn_row64(q + row, kbase, vbase, row_bytes, pos0 + qo + 1, scale);
+        }
+        *reinterpret_cast<float4*>(dst + d0) = acc;
     }
 }
 

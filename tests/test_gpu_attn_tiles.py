@@ -114,3 +114,44 @@ def test_attn_sinks(gpu, hd):
         ref = oracle.attn_f64(q[i].reshape(-1), Kb, Vb, n_head, n_kv, hd, pos0 + i + 1, scale)
         assert 2e-5 < np.abs(ref).min()
         assert np.abs(y[i] - ref).max() <= 4e-5 * np.abs(ref).max() + 1e-7
+
+
+def rows64(q, K, V, n_head, n_kv, hd, pos0, scale):
+    """The outputs in 64 bits where something is infinite or NaN: a NaN or -inf score
+    is no key, a +inf one makes the row NaN, and weight 0 times an infinite V is NaN."""
+    out = np.empty((len(q), n_head, hd))
+    with np.errstate(all="ignore"):
+        for i in range(len(q)):
+            for h in range(n_head):
+                g = h // (n_head // n_kv)
+                k, v = K[:pos0 + i + 1, g], V[:pos0 + i + 1, g]
+                s = (q[i, h] * k).sum(1) * scale
+                e = np.where(s > -1e29, np.exp(s - s[s > -1e29].max(initial=-1e30)), 0)
+                out[i, h] = (e[:, None] * v).sum(0) / max(e.sum(), 1e-20)
+    return out
+
+
+def test_attn_hd64_not_finite(gpu):
+    """Infinities and NaN at head_dim 64, which takes them as fp32 arithmetic does: in
+    a query (alone and beside others of its tile), in a key and in values."""
+    rng = np.random.default_rng(64)
+    n_head, n_kv, hd, pos0, n_q = 6, 2, 64, 50, 70
+    L, scale = pos0 + n_q, 0.125
+    q = rng.standard_normal((n_q, n_head, hd)).astype(np.float32)
+    K = rng.standard_normal((L, n_kv, hd)).astype(np.float16)
+    V = rng.standard_normal((L, n_kv, hd)).astype(np.float16)
+    q[2, 0, 5], q[5, 1, 7], q[7, 2, 9] = np.inf, -np.inf, np.nan
+    q[30, 4, 1], q[31, 4, 1:3] = np.inf, (np.inf, -np.inf)
+    K[95, 0, 3], K[60, 1, 4] = np.inf, -np.inf
+    V[100, 0, 9], V[52, 1, 20], V[57, 1, 21] = np.inf, -np.inf, np.nan
+    ref = rows64(q.astype(np.float64), K.astype(np.float64), V.astype(np.float64), n_head, n_kv,
+                 hd, pos0, scale)
+    out = empty(q.size)
+    print("attn hd=64 not finite", flush=True)
+    call("tf_attn_prefill", P(dev(q)), P(dev(K.view(np.int16))), P(dev(V.view(np.int16))), P(out),
+         n_head, n_kv, hd, pos0, n_q, scale, S())
+    y = host(out).reshape(ref.shape).astype(np.float64)
+    fin = np.isfinite(ref)
+    assert 0.3 < fin.mean() < 0.9 and np.isinf(ref).any()
+    np.testing.assert_array_equal(np.where(fin, 0, y), np.where(fin, 0, ref))
+    assert np.abs(y[fin] - ref[fin]).max() <= 4e-5 * 5
