@@ -124,10 +124,13 @@ def ptr(t) -> int | None:
 
 def stream_ptr(stream=None) -> int | None:
     if stream is None:
-        if torch.cuda.is_initialized():
-            # the handle alone: current_stream() builds a Stream object, 3 us of a
-            # call whose launch takes as long
-            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()) or None
+        # the handle alone: current_stream() builds a Stream object, 3 us of a call
+        # whose launch takes as long.  Both names are private to torch: without them
+        # the Stream object serves.
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        device = getattr(torch._C, "_cuda_getDevice", None)
+        if raw and device and torch.cuda.is_initialized():
+            return raw(device()) or None
         stream = torch.cuda.current_stream()
     return stream.cuda_stream or None
 

@@ -97,3 +97,20 @@ def test_argtypes_match_header_arity(capi):
     counts = header_param_counts()
     for name, args in capi.SIGNATURES.items():
         assert counts[name] == len(args), (name, counts[name], len(args))
+
+
+@pytest.mark.parametrize("gone", ["_cuda_getCurrentRawStream", "_cuda_getDevice"])
+def test_stream_ptr_without_torchs_private_names(monkeypatch, gone):
+    """capi.stream_ptr falls back on the public current_stream()."""
+    import types
+
+    import torch
+
+    from taraference_amd import capi
+
+    handle = types.SimpleNamespace(cuda_stream=4096)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: handle)
+    monkeypatch.delattr(torch._C, gone, raising=False)
+    assert capi.stream_ptr() == 4096
+    assert capi.stream_ptr(types.SimpleNamespace(cuda_stream=0)) is None
