@@ -39,6 +39,7 @@
 // h supplies values 32 s + 16 h + 8 b + {0, 2, 1, 3, 4, 6, 5, 7} (the order in
 // which nibbles come out of a dword), for x and W alike.
 #include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #include "lds_dma.hpp"
@@ -226,7 +227,7 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
                                            const float* __restrict__ x,
                                            const uint8_t* __restrict__ ximg,
                                            float* __restrict__ out, int ldo, int n_rows, int n_cols,
-                                           int col_bytes, int n_tok, int accumulate, int n_split,
+                                           int col_bytes, int n_tok, int n_split,
                                            int t0, int ctile) {
     constexpr int CPW = DUAL ? 32 : 64;  // output columns of a wave
     constexpr bool Q6 = FMT != TF_PG_W4;
@@ -660,9 +661,7 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
             for (int i = 0; i < 16; i++) {
                 const int t = t0 + 32 * tt + 8 * (i >> 2) + 4 * h + (i & 3);
                 if (t >= n_tok) continue;
-                float* o = out + (size_t)t * ldo + c;
-                // accumulate: out += W x (the residual stream), one rounding
-                *o = accumulate ? *o + acc[ct][tt][i] : acc[ct][tt][i];
+                out[(size_t)t * ldo + c] = acc[ct][tt][i];
             }
     }
 }
@@ -689,14 +688,14 @@ __global__ __launch_bounds__(64 * CW * KW, KW * NBUF * TT >= 4 ? CW * KW / 4
 tf_gemm_kq_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
                   const float* __restrict__ x, const uint8_t* __restrict__ ximg,
                   float* __restrict__ out, int n_rows, int n_cols, int col_bytes, int n_tok,
-                  int accumulate, int n_split, long long split_stride) {
+                  int n_split, int ldo, long long split_stride) {
     __shared__ __align__(16) uint8_t lds[KW * NBUF * TT * TF_PG_SLOT];
     constexpr int COLS = (DUAL ? 32 : 64) * CW;
     int tx, ct;
     if (!tf_pg_tile((n_tok + 32 * TT - 1) / (32 * TT), (n_cols + COLS - 1) / COLS, tx, ct)) return;
     tf_pg_body<FMT, TT, CW, KW, PRE, NBUF, DUAL>(
-        lds, w, w2, x, ximg, out + (size_t)blockIdx.z * (size_t)split_stride, n_cols, n_rows, n_cols,
-        col_bytes, n_tok, accumulate, n_split, tx * 32 * TT, ct);
+        lds, w, w2, x, ximg, out + (size_t)blockIdx.z * (size_t)split_stride, ldo, n_rows, n_cols,
+        col_bytes, n_tok, n_split, tx * 32 * TT, ct);
 }
 
 // q, k and v of a prompt in one launch (their outputs side by side in rows of
@@ -714,7 +713,7 @@ __global__ __launch_bounds__(256, 2) void tf_pg_qkv_kernel(TfPgQkv m, const uint
     auto go = [&](auto fmt) {
         tf_pg_body<decltype(fmt)::value, 1, 4, 1, true, 1, false>(
             lds, m.w[i], nullptr, nullptr, ximg, o, ldo, n_rows, m.n_cols[i], m.col_bytes[i], n_tok,
-            0, n_split, tx * 32, ct);
+            n_split, tx * 32, ct);
     };
     if (m.fmt[i] == TF_PG_W4) go(std::integral_constant<int, TF_PG_W4>{});
     else if (m.fmt[i] == TF_PG_W6) go(std::integral_constant<int, TF_PG_W6>{});
@@ -898,7 +897,7 @@ struct TfPgJob {
     const float* x;
     const uint8_t* img;
     float* out;
-    int n_rows, n_cols, col_bytes, n_tok, accumulate, n_split;
+    int n_rows, n_cols, col_bytes, n_tok, n_split, ldo;  // ldo: floats of an output row
     hipStream_t stream;
 };
 
@@ -912,7 +911,7 @@ void tf_pg_go(const TfPgJob& j) {
     const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, j.n_split);
     hipLaunchKernelGGL((tf_gemm_kq_kernel<FMT, TT, CW, KW, PRE, NBUF, DUAL>), grid,
                        dim3(64 * CW * KW), 0, j.stream, j.w, j.w2, j.x, j.img, j.out, j.n_rows,
-                       j.n_cols, j.col_bytes, j.n_tok, j.accumulate, j.n_split,
+                       j.n_cols, j.col_bytes, j.n_tok, j.n_split, j.ldo,
                        (long long)j.n_tok * j.n_cols);
 }
 
@@ -1045,7 +1044,7 @@ int tf_pg_gemm(const uint8_t* w, int block_bytes, const uint8_t* img, int n_rows
     TF_CHECK_ARG(img && slice <= ws_floats);
     const int n_split = tf_pg_splits(tiles_of(n_tok, n_cols, 32, 256), n_rows / 256, slice, ws_floats);
     *part = TfPgPart{ws, n_split, (long long)slice};
-    TfPgJob j{w, nullptr, nullptr, img, ws, n_rows, n_cols, col_bytes, n_tok, 0, n_split,
+    TfPgJob j{w, nullptr, nullptr, img, ws, n_rows, n_cols, col_bytes, n_tok, n_split, n_cols,
               tf_stream(stream)};
     if (!q6) tf_pg_go<TF_PG_W4, 1, 4, 1, true, 1>(j);
     else if (block_bytes == 212) tf_pg_go<TF_PG_W6C, 1, 4, 1, true, 1>(j);
@@ -1100,7 +1099,7 @@ int tf_pg_gate_up(const uint8_t* gate, const uint8_t* up, const uint8_t* img, fl
     if (!rc) rc = tf_pg_check(false, up, out, n_rows, n_cols, col_bytes, n_tok, 144);
     if (rc) return rc;
     TF_CHECK_ARG(img);
-    const TfPgJob j{gate, up, nullptr, img, out, n_rows, n_cols, col_bytes, n_tok, 0, 1,
+    const TfPgJob j{gate, up, nullptr, img, out, n_rows, n_cols, col_bytes, n_tok, 1, n_cols,
                     tf_stream(stream)};
     // a short prompt: half the columns a workgroup and K split over its waves
     // (2048 -> 2 x 11008 at 20 tokens, 86 workgroups: 31 us)
@@ -1113,13 +1112,24 @@ int tf_pg_gate_up(const uint8_t* gate, const uint8_t* up, const uint8_t* img, fl
 
 // ---------------------------------------------------------------- C ABI
 
+// Columns and rows so long that a launch's 32-bit offsets cannot take 64 and 32 of
+// them (above 2^26 bytes and 2^25 values) go in groups that they can.
 static int tf_gemm_f32(bool q6, const uint8_t* w, const float* x, float* out, int n_rows,
                        int n_cols, int col_bytes, int n_tok, tf_stream_t stream) {
-    const int rc = tf_pg_check(q6, w, out, n_rows, n_cols, col_bytes, n_tok, q6 ? 210 : 144);
-    if (rc) return rc;
-    TF_CHECK_ARG(x && ((uintptr_t)x & 15) == 0);
-    tf_pg_f32(q6, TfPgJob{w, nullptr, x, nullptr, out, n_rows, n_cols, col_bytes, n_tok, 0, 1,
-                          tf_stream(stream)});
+    const int blk = q6 ? 210 : 144;
+    TF_CHECK_ARG(x && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0);
+    const int max_c = col_bytes < (1 << 26) ? n_cols : (int)(((1ll << 32) - 1) / col_bytes);
+    const int max_t = n_rows < (1 << 25) ? n_tok : (int)(((1ll << 30) - 1) / n_rows);
+    for (int t0 = 0; t0 == 0 || t0 < n_tok; t0 += max_t)
+        for (int c0 = 0; c0 == 0 || c0 < n_cols; c0 += max_c) {
+            const int nt = std::min(n_tok - t0, max_t), nc = std::min(n_cols - c0, max_c);
+            const uint8_t* wc = w + (size_t)c0 * col_bytes;
+            const int rc = tf_pg_check(q6, wc, out, n_rows, nc, col_bytes, nt, blk);
+            if (rc) return rc;
+            tf_pg_f32(q6, TfPgJob{wc, nullptr, x + (size_t)t0 * n_rows, nullptr,
+                                  out + (size_t)t0 * n_cols + c0, n_rows, nc, col_bytes, nt, 1,
+                                  n_cols, tf_stream(stream)});
+        }
     return TF_LAUNCH_RESULT();
 }
 

@@ -11,9 +11,10 @@ column starts modulo 4 (an odd number of 210-byte blocks makes it alternate).
 """
 import numpy as np
 import pytest
+import torch
 
 from taraference_amd import synth
-from _gpu import P, S, call, dev, empty, host
+from _gpu import KEEP, P, S, call, dev, empty, host
 from _util import assert_gemv_close, gemm_ref
 
 pytestmark = pytest.mark.gpu
@@ -76,3 +77,37 @@ def test_gemm_scales_of_x(gpu, fmt):
     x[7] = np.float32(1e-38)  # subnormal products with the block scales still count
     x[8] = 1
     run(fmt, 768, 200, x)
+
+
+@pytest.mark.parametrize("fmt,n_rows,n_cols,n_tok", [
+    ("q4k", 1 << 27, 64, 1),           # 64 columns of 72 MB: more than 4 GB
+    ("q6k", 1 << 27, 64, 1),
+    ("q4k", (1 << 25) + 256, 3, 33),   # 32 rows of 128 MB
+])
+def test_gemm_past_32_bit_offsets(gpu, fmt, n_rows, n_cols, n_tok):
+    """Everything 0 but a few super-blocks of the first, the last and the columns and
+    rows on either side of 4 GB."""
+    rng = np.random.default_rng(n_cols)
+    nb, bb = n_rows // 256, 144 if fmt == "q4k" else 210
+    make = synth.q4k_blocks if fmt == "q4k" else synth.q6k_blocks
+    w = torch.zeros((n_cols, nb, bb), dtype=torch.uint8, device="cuda")
+    x = torch.zeros((n_tok, nb, 256), device="cuda")
+    KEEP.extend((w, x))
+    sbs = [0, 1, nb // 2 + 3, nb - 1]
+    cols = sorted({0, n_cols // 2, n_cols - 9, n_cols - 2, n_cols - 1} & set(range(n_cols)))
+    cols += [c for c in (36, 37, 55, 56, 57) if c < n_cols and c not in cols]
+    wb = np.zeros((n_cols, len(sbs), bb), np.uint8)
+    wb[cols] = make(rng, len(cols) * len(sbs)).reshape(len(cols), len(sbs), bb)
+    xb = rng.standard_normal((n_tok, len(sbs), 256)).astype(np.float32)
+    w[:, sbs] = torch.from_numpy(wb).cuda()
+    x[:, sbs] = torch.from_numpy(xb).cuda()
+    out = empty(n_tok * n_cols)
+    print(f"gemm {fmt} {n_rows}x{n_cols} tok={n_tok}", flush=True)
+    call(f"tf_gemm_{fmt}_f32", P(w), P(x), P(out), n_rows, n_cols, nb * bb, n_tok, S())
+    y = host(out).reshape(n_tok, n_cols)
+    ref, absn = gemm_ref(fmt, wb.reshape(n_cols, -1), 256 * len(sbs), xb.reshape(n_tok, -1))
+    for t in range(n_tok):
+        assert_gemv_close(y[t], ref[t], absn[t], f"{fmt} t={t}")
+    KEEP.clear()
+    del w, x
+    torch.cuda.empty_cache()
