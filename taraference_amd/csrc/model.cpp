@@ -768,7 +768,8 @@ struct tf_model {
             TfPgPart part{nullptr, 0, 0};
             // x += W a for the image of a; the add is the next kernel's
             auto gemm_add = [&](const GpuMat& w) {
-                const bool compact = w.wtype == tf::WType::Q6K && w.compact_data;
+                const bool compact = w.wtype == tf::WType::Q6K && w.compact_data &&
+                                     (((uintptr_t)w.compact_data | w.compact_col_bytes) & 3) == 0;
                 tf::check(tf_pg_gemm(compact ? w.compact_data : w.data, compact ? 212 : blk(w),
                                      pf_img, (int)w.n_rows, (int)w.n_cols,
                                      (int)(compact ? w.compact_col_bytes : w.col_bytes), nt, pf_ws,

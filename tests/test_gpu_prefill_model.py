@@ -18,6 +18,7 @@ starts with prefill's token and runs on the decode path.
 """
 import numpy as np
 import pytest
+import torch
 
 from taraference_amd import synth
 from _gpu import Unaligned, model_class
@@ -88,6 +89,39 @@ def test_prefill_norms_4_byte_aligned(gpu, name):
                           [dict(L, attn_norm=v["attn_norm"], ffn_norm=v["ffn_norm"])
                            for L in layers], emb, output_norm=v["output_norm"])
         print(f"prefill {name} unaligned={u}", flush=True)
+        out.append((m.prefill(prompt, 0), m.logits()))
+        m.close()
+    assert out[0][0] == out[1][0]
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+
+
+def test_prefill_compact_down_2_byte_aligned(gpu):
+    """A compact copy of a Q6_K down that the GEMM cannot load in dwords: the prompt
+    reads the raw blocks, with the same bits."""
+    from taraference_amd.model import DecodeModel
+
+    class Shifted(DecodeModel):
+        def _q6(self, wm, n_rows, compact):
+            m = super()._q6(wm, n_rows, compact)
+            if n_rows == self.cfg["n_ff"]:
+                old = self._keep[-1]
+                new = torch.zeros(old.numel() + 16, dtype=torch.uint8, device="cuda")
+                new[2:2 + old.numel()] = old
+                self._keep.append(new)
+                m.compact = new.data_ptr() + 2
+            return m
+
+    cfg = TINY[0]
+    rng = np.random.default_rng(78)
+    layers = [synth.qwen_layer(rng, cfg, li) for li in range(cfg["n_layer"])]
+    for L in layers:
+        L["down"], L["down_q6k"] = synth.q6k_matrix(rng, cfg["n_ff"], cfg["n_embd"]), True
+    emb = synth.qwen_embedding(rng, cfg)
+    prompt = rng.integers(0, cfg["n_vocab"], 20).tolist()
+    out = []
+    for cls in (DecodeModel, Shifted):
+        m = cls(dict(cfg, max_seq=40), layers, emb)
+        print(f"prefill {cls.__name__}", flush=True)
         out.append((m.prefill(prompt, 0), m.logits()))
         m.close()
     assert out[0][0] == out[1][0]
