@@ -271,6 +271,7 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
     using L = TfPmLds<HD>;
     constexpr int ROWB = L::ROWB, ST = HD / 16, DB = HD / 32;
     constexpr int NC = L::TILE / (64 * DW);  // copies of a tile
+    constexpr int NCU = NC > 16 ? 16 : NC;   // 32 at once do not fit the registers
     extern __shared__ __align__(16) uint8_t lds[];
     const int pos0 = pos0_ptr ? pos0_ptr[0] : pos0_arg;
     // kv heads fastest (workgroups of one kv head share few XCDs' L2), the
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
             return (uint32_t)(r < last ? r : last) * row_bytes + 16 * (c ^ sw) + (p & 15);
         };
         if (rmax >= TF_PM_T - 1) {
-#pragma unroll(NC > 16 ? 16 : NC)  // 32 copies at once do not fit the registers
+#pragma unroll NCU
             for (int i = 0; i < NC; i++)
                 tf_lds_dma_s<DW>(tb, off(i, TF_PM_T), ldst + 64 * DW * i);
         } else {
