@@ -215,13 +215,12 @@ __device__ __forceinline__ void tf_pg_store_x(const tf_pg_f4 (&xr)[NP][2], uint8
     }
 }
 
-// The wide kernel: a workgroup (4 waves) owns 256 columns x 32 TT tokens, a
-// wave 64 columns x 32 TT tokens.  PRE: x is already in images (ximg,
-// [token tile of 32][super-block], TF_PG_SLOT bytes each) and is copied into
-// LDS; otherwise the workgroup converts x itself.
-// One workgroup's tile: tokens t0 .., columns c0 .. of this wave's 64 (DUAL:
-// 32 of w and 32 of w2), slice z of n_split.  out has rows of ldo floats.
-template <int FMT, int TT, int CW, int KW, bool PRE, int NBUF, bool DUAL>
+// One workgroup's tile: CW x KW waves, KW slices of K of CW column groups of 64
+// (DUAL: 32 of w and 32 of w2), times the 32 tokens from t0; slice z of n_split.
+// PRE: x is already in images (ximg, [token tile of 32][super-block], TF_PG_SLOT
+// bytes each) and is copied into LDS; otherwise the workgroup converts x itself,
+// into one image a slice or, NBUF 2, two in turn.  out has rows of ldo floats.
+template <int FMT, int CW, int KW, bool PRE, int NBUF, bool DUAL>
 __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint8_t* __restrict__ w,
                                            const uint8_t* __restrict__ w2,
                                            const float* __restrict__ x,
@@ -229,15 +228,16 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
                                            float* __restrict__ out, int ldo, int n_rows, int n_cols,
                                            int col_bytes, int n_tok, int n_split,
                                            int t0, int ctile) {
+    static_assert(!PRE || NBUF == 1, "one image a slice is copied");
     constexpr int CPW = DUAL ? 32 : 64;  // output columns of a wave
     constexpr bool Q6 = FMT != TF_PG_W4;
     constexpr int BLK = FMT == TF_PG_W4 ? 144 : FMT == TF_PG_W6C ? 212 : 210;
-    constexpr int RP = 2 * CW, NP = 32 * TT / RP;  // tokens staged per pass, passes
+    constexpr int RP = 2 * CW, NP = 32 / RP;  // tokens staged per pass, passes
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cw = wave % CW, kw = wave / CW;
     const int h = lane >> 5, l32 = lane & 31;
-    uint8_t* const img0 = lds + kw * NBUF * TT * TF_PG_SLOT;
+    uint8_t* const img0 = lds + kw * NBUF * TF_PG_SLOT;
 
     const int c0 = ctile * (CPW * CW) + CPW * cw;
     const int nb = n_rows / 256;
@@ -278,35 +278,22 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
         }
     };
     auto store_x = [&](uint8_t* slot) {
-        if constexpr (!PRE) {
-#pragma unroll
-            for (int tt = 0; tt < TT; tt++)
-                tf_pg_store_x<RP, NP / TT, !Q6>(
-                    reinterpret_cast<const tf_pg_f4(&)[NP / TT][2]>(xr[NP / TT * tt]),
-                    slot + tt * TF_PG_SLOT, st, ci);
-        }
+        if constexpr (!PRE) tf_pg_store_x<RP, NP, !Q6>(xr, slot, st, ci);
     };
     auto dma_x = [&](int sb, uint8_t* slot) {
         if constexpr (PRE) {
             const uint32_t l0 = tf_lds_off(slot);
-#pragma unroll
-            for (int tt = 0; tt < TT; tt++) {
-                int tb = (t0 >> 5) + tt;
-                if (TT > 1 && tt && t0 + 32 * tt >= n_tok) tb -= tt;  // no such tokens: any image
-                const uint8_t* src = ximg + ((size_t)tb * nb + sb) * TF_PG_SLOT + 16 * lane;
-                for (int i = cw; i < TF_PG_SLOT / 1024; i += CW)
-                    tf_lds_dma16(src + 1024 * i, l0 + tt * TF_PG_SLOT + 1024 * i);
-            }
+            const uint8_t* src = ximg + ((size_t)(t0 >> 5) * nb + sb) * TF_PG_SLOT + 16 * lane;
+            for (int i = cw; i < TF_PG_SLOT / 1024; i += CW)
+                tf_lds_dma16(src + 1024 * i, l0 + 1024 * i);
         }
     };
 
-    tf_pg_f16v acc[2][TT];
+    tf_pg_f16v acc[2];
 #pragma unroll
     for (int ct = 0; ct < 2; ct++)
 #pragma unroll
-        for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[ct][tt][i] = 0.f;
+        for (int i = 0; i < 16; i++) acc[ct][i] = 0.f;
 
     uint32_t m_lo = 0x000F000Fu, m_hi = 0x00F000F0u;
     asm("" : "+v"(m_lo), "+v"(m_hi));  // the masks in VGPRs (see tf_pg_and_or)
@@ -338,25 +325,21 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
     }
     if (NBUF == 2) {
         store_x(img0);
-        dma_x(round_sb(0), img0);
         load_x(round_sb(1));
     }
     for (int it = 0; it < n_it; it++) {
         const int n1 = round_sb(it + 1);
         const bool live = KW == 1 || lo + it < hi;
-        uint8_t* slot = img0 + (NBUF == 2 ? (it & 1) * TT * TF_PG_SLOT : 0);
-        if (PRE && NBUF == 2) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the copies landed
+        uint8_t* slot = img0 + (NBUF == 2 ? (it & 1) * TF_PG_SLOT : 0);
         __syncthreads();
         if (NBUF == 2) {
             // the other image: its readers passed the barrier above
-            uint8_t* other = img0 + ((it + 1) & 1) * TT * TF_PG_SLOT;
-            store_x(other);
-            if (it + 1 < n_it) dma_x(n1, other);
+            store_x(img0 + ((it + 1) & 1) * TF_PG_SLOT);
             load_x(round_sb(it + 2));
         } else {
             store_x(slot);
             dma_x(round_sb(it), slot);
-            if (PRE) __builtin_amdgcn_s_waitcnt(0x0F70);
+            if (PRE) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the copies landed
             __syncthreads();
             load_x(n1);
         }
@@ -367,17 +350,15 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
 #pragma unroll
         for (int e = 0; e < 4; e++)
             xo[e] = slot + 512 * h + ((l32 ^ (2 * h + (e & 1) + 4 * (e >> 1))) << 4);
-        auto xfrag = [&](int tt, int pl, int s, int b) {
-            return *reinterpret_cast<const tf_pg_h8*>(xo[2 * (s & 1) + b] + TF_PG_SLOT * tt +
-                                                      16384 * pl + 1024 * (2 * s + b));
+        auto xfrag = [&](int pl, int s, int b) {
+            return *reinterpret_cast<const tf_pg_h8*>(xo[2 * (s & 1) + b] + 16384 * pl +
+                                                      1024 * (2 * s + b));
         };
-        tf_pg_f16v P[2][TT];
+        tf_pg_f16v P[2];
 #pragma unroll
         for (int ct = 0; ct < 2; ct++)
 #pragma unroll
-            for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) P[ct][tt][i] = 0.f;
+            for (int i = 0; i < 16; i++) P[ct][i] = 0.f;
 
         if constexpr (!Q6) {
             float dv[2], dm[2];
@@ -422,11 +403,9 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
                     }
 #pragma unroll
                     for (int b = 0; b < 2; b++) {
-                        tf_pg_h8 xf[TT][2];
+                        tf_pg_h8 xf[2];
 #pragma unroll
-                        for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-                            for (int pl = 0; pl < 2; pl++) xf[tt][pl] = xfrag(tt, pl, s, b);
+                        for (int pl = 0; pl < 2; pl++) xf[pl] = xfrag(pl, s, b);
                         tf_pg_h8 bw[2];
 #pragma unroll
                         for (int ct = 0; ct < 2; ct++) {
@@ -447,11 +426,9 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
 #pragma unroll
                         for (int pl = 0; pl < 2; pl++)
 #pragma unroll
-                            for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-                                for (int ct = 0; ct < 2; ct++)
-                                    P[ct][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                        xf[tt][pl], bw[ct], P[ct][tt], 0, 0, 0);
+                            for (int ct = 0; ct < 2; ct++)
+                                P[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[pl], bw[ct],
+                                                                               P[ct], 0, 0, 0);
                     }
                 }
                 TF_PG_FENCE();
@@ -462,32 +439,28 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
 #pragma unroll
             for (int ct = 0; ct < 2; ct++) wc[ct].hd = tf_pg_ld16(wn[ct], woff[ct]);
             // acc += 2^-e (d P - 32 dmin M); C rows 8 k + 4 h + r = tokens
+            const uint8_t* aux = slot + TF_PG_IMG;
+            // M: K = part (half h) x 8 sub-blocks
+            const tf_pg_h8 xs = *reinterpret_cast<const tf_pg_h8*>(aux + (32 * h + l32) * 16);
+            tf_pg_f16v M[2];
 #pragma unroll
-            for (int tt = 0; tt < TT; tt++) {
-                const uint8_t* aux = slot + TF_PG_SLOT * tt + TF_PG_IMG;
-                // M: K = part (half h) x 8 sub-blocks
-                const tf_pg_h8 xs = *reinterpret_cast<const tf_pg_h8*>(aux + (32 * h + l32) * 16);
-                tf_pg_f16v M[2];
+            for (int ct = 0; ct < 2; ct++) {
 #pragma unroll
-                for (int ct = 0; ct < 2; ct++) {
+                for (int i = 0; i < 16; i++) M[ct][i] = 0.f;
+                M[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs, mv[ct], M[ct], 0, 0, 0);
+            }
+            const float* xinv = reinterpret_cast<const float*>(aux + TF_PG_SUMS);
 #pragma unroll
-                    for (int i = 0; i < 16; i++) M[ct][i] = 0.f;
-                    M[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs, mv[ct], M[ct], 0, 0, 0);
-                }
-                const float* xinv = reinterpret_cast<const float*>(aux + TF_PG_SUMS);
+            for (int k = 0; k < 4; k++) {
+                const float4 fi = *reinterpret_cast<const float4*>(xinv + 8 * k + 4 * h);
+                const float fv[4] = {fi.x, fi.y, fi.z, fi.w};
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const float4 fi = *reinterpret_cast<const float4*>(xinv + 8 * k + 4 * h);
-                    const float fv[4] = {fi.x, fi.y, fi.z, fi.w};
+                for (int ct = 0; ct < 2; ct++)
 #pragma unroll
-                    for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const float t =
-                                dv[ct] * P[ct][tt][4 * k + r] - dm[ct] * M[ct][4 * k + r];
-                            acc[ct][tt][4 * k + r] = fmaf(fv[r], t, acc[ct][tt][4 * k + r]);
-                        }
-                }
+                    for (int r = 0; r < 4; r++) {
+                        const float t = dv[ct] * P[ct][4 * k + r] - dm[ct] * M[ct][4 * k + r];
+                        acc[ct][4 * k + r] = fmaf(fv[r], t, acc[ct][4 * k + r]);
+                    }
             }
         } else {
             float dv[2];
@@ -552,11 +525,9 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
                         const uint32_t mk = g ? m_hi : m_lo;
 #pragma unroll
                         for (int b = 0; b < 2; b++) {
-                            tf_pg_h8 xf[TT][2];
+                            tf_pg_h8 xf[2];
 #pragma unroll
-                            for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-                                for (int pl = 0; pl < 2; pl++) xf[tt][pl] = xfrag(tt, pl, s, b);
+                            for (int pl = 0; pl < 2; pl++) xf[pl] = xfrag(pl, s, b);
                             tf_pg_h8 bh[2], bl[2];
 #pragma unroll
                             for (int ct = 0; ct < 2; ct++) {
@@ -581,12 +552,9 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
 #pragma unroll
                             for (int m = 0; m < 3; m++)
 #pragma unroll
-                                for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-                                    for (int ct = 0; ct < 2; ct++)
-                                        P[ct][tt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                            xf[tt][m == 1], m == 2 ? bl[ct] : bh[ct], P[ct][tt], 0,
-                                            0, 0);
+                                for (int ct = 0; ct < 2; ct++)
+                                    P[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                        xf[m == 1], m == 2 ? bl[ct] : bh[ct], P[ct], 0, 0, 0);
                         }
                     }
                     TF_PG_FENCE();
@@ -598,26 +566,21 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
                 for (int ct = 0; ct < 2; ct++)
                     tf_pg_load_run<FMT>(wn[ct], woff[ct], odd_of(ct, n1), h, 4 + n, wc[ct]);
             }
+            const float* xinv = reinterpret_cast<const float*>(slot + TF_PG_IMG + TF_PG_SUMS);
 #pragma unroll
-            for (int tt = 0; tt < TT; tt++) {
-                const float* xinv = reinterpret_cast<const float*>(slot + TF_PG_SLOT * tt +
-                                                                   TF_PG_IMG + TF_PG_SUMS);
+            for (int k = 0; k < 4; k++) {
+                const float4 fi = *reinterpret_cast<const float4*>(xinv + 8 * k + 4 * h);
+                const float fv[4] = {fi.x, fi.y, fi.z, fi.w};
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const float4 fi = *reinterpret_cast<const float4*>(xinv + 8 * k + 4 * h);
-                    const float fv[4] = {fi.x, fi.y, fi.z, fi.w};
+                for (int ct = 0; ct < 2; ct++)
 #pragma unroll
-                    for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-                        for (int r = 0; r < 4; r++)
-                            acc[ct][tt][4 * k + r] = fmaf(fv[r], dv[ct] * P[ct][tt][4 * k + r],
-                                                          acc[ct][tt][4 * k + r]);
-                }
+                    for (int r = 0; r < 4; r++)
+                        acc[ct][4 * k + r] =
+                            fmaf(fv[r], dv[ct] * P[ct][4 * k + r], acc[ct][4 * k + r]);
             }
         }
     }
     if constexpr (KW > 1) {  // slices 1.. hand their sums to slice 0, added in slice order
-        static_assert(TT == 1, "one token tile per wave where the waves split K");
         __syncthreads();  // the images are read
         float* part = reinterpret_cast<float*>(lds);
         if (kw > 0) {
@@ -625,7 +588,7 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
             for (int ct = 0; ct < 2; ct++)
 #pragma unroll
                 for (int i = 0; i < 16; i++)
-                    part[(((kw - 1) * CW + cw) * 32 + 16 * ct + i) * 64 + lane] = acc[ct][0][i];
+                    part[(((kw - 1) * CW + cw) * 32 + 16 * ct + i) * 64 + lane] = acc[ct][i];
         }
         __syncthreads();
         if (kw > 0) return;
@@ -635,20 +598,17 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
             for (int ct = 0; ct < 2; ct++)
 #pragma unroll
                 for (int i = 0; i < 16; i++)
-                    acc[ct][0][i] += part[((q * CW + cw) * 32 + 16 * ct + i) * 64 + lane];
+                    acc[ct][i] += part[((q * CW + cw) * 32 + 16 * ct + i) * 64 + lane];
     }
     if constexpr (DUAL) {  // silu(gate) * up
         const int c = c0 + l32;
         if (c >= n_cols) return;
 #pragma unroll
-        for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int t = t0 + 32 * tt + 8 * (i >> 2) + 4 * h + (i & 3);
-                const float g = acc[0][tt][i];
-                if (t < n_tok)
-                    out[(size_t)t * ldo + c] = (g / (1.f + __expf(-g))) * acc[1][tt][i];
-            }
+        for (int i = 0; i < 16; i++) {
+            const int t = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
+            const float g = acc[0][i];
+            if (t < n_tok) out[(size_t)t * ldo + c] = (g / (1.f + __expf(-g))) * acc[1][i];
+        }
         return;
     }
 #pragma unroll
@@ -656,13 +616,10 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
         const int c = c0 + 32 * ct + l32;
         if (c >= n_cols) continue;
 #pragma unroll
-        for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int t = t0 + 32 * tt + 8 * (i >> 2) + 4 * h + (i & 3);
-                if (t >= n_tok) continue;
-                out[(size_t)t * ldo + c] = acc[ct][tt][i];
-            }
+        for (int i = 0; i < 16; i++) {
+            const int t = t0 + 8 * (i >> 2) + 4 * h + (i & 3);
+            if (t < n_tok) out[(size_t)t * ldo + c] = acc[ct][i];
+        }
     }
 }
 
@@ -681,21 +638,21 @@ __device__ __forceinline__ bool tf_pg_tile(int ntx, int n_ct, int& tx, int& ct) 
 
 // Waves per SIMD: 3 where the registers allow it (Q4_K without conversion
 // registers), else 2, or what four images of LDS (136 KB) leave room for.
-template <int FMT, int TT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false>
-__global__ __launch_bounds__(64 * CW * KW, KW * NBUF * TT >= 4 ? CW * KW / 4
-                                           : PRE && FMT == TF_PG_W4 && TT == 1 ? 3
-                                                                               : 2) void
+template <int FMT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false>
+__global__ __launch_bounds__(64 * CW * KW, KW * NBUF >= 4            ? CW * KW / 4
+                                           : PRE && FMT == TF_PG_W4 ? 3
+                                                                    : 2) void
 tf_gemm_kq_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
                   const float* __restrict__ x, const uint8_t* __restrict__ ximg,
                   float* __restrict__ out, int n_rows, int n_cols, int col_bytes, int n_tok,
                   int n_split, int ldo, long long split_stride) {
-    __shared__ __align__(16) uint8_t lds[KW * NBUF * TT * TF_PG_SLOT];
+    __shared__ __align__(16) uint8_t lds[KW * NBUF * TF_PG_SLOT];
     constexpr int COLS = (DUAL ? 32 : 64) * CW;
     int tx, ct;
-    if (!tf_pg_tile((n_tok + 32 * TT - 1) / (32 * TT), (n_cols + COLS - 1) / COLS, tx, ct)) return;
-    tf_pg_body<FMT, TT, CW, KW, PRE, NBUF, DUAL>(
+    if (!tf_pg_tile((n_tok + 31) / 32, (n_cols + COLS - 1) / COLS, tx, ct)) return;
+    tf_pg_body<FMT, CW, KW, PRE, NBUF, DUAL>(
         lds, w, w2, x, ximg, out + (size_t)blockIdx.z * (size_t)split_stride, ldo, n_rows, n_cols,
-        col_bytes, n_tok, n_split, tx * 32 * TT, ct);
+        col_bytes, n_tok, n_split, tx * 32, ct);
 }
 
 // q, k and v of a prompt in one launch (their outputs side by side in rows of
@@ -711,7 +668,7 @@ __global__ __launch_bounds__(256, 2) void tf_pg_qkv_kernel(TfPgQkv m, const uint
     if (i) ct -= m.ct[i - 1];
     float* o = out + (size_t)blockIdx.z * (size_t)split_stride + m.col[i];
     auto go = [&](auto fmt) {
-        tf_pg_body<decltype(fmt)::value, 1, 4, 1, true, 1, false>(
+        tf_pg_body<decltype(fmt)::value, 4, 1, true, 1, false>(
             lds, m.w[i], nullptr, nullptr, ximg, o, ldo, n_rows, m.n_cols[i], m.col_bytes[i], n_tok,
             n_split, tx * 32, ct);
     };
@@ -901,15 +858,15 @@ struct TfPgJob {
     hipStream_t stream;
 };
 
-template <int FMT, int TT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false>
+template <int FMT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false>
 void tf_pg_go(const TfPgJob& j) {
     const int cols = (DUAL ? 32 : 64) * CW;
-    const size_t tiles = (size_t)((j.n_tok + 32 * TT - 1) / (32 * TT)) *
+    const size_t tiles = (size_t)((j.n_tok + 31) / 32) *
                          (size_t)((j.n_cols + cols - 1) / cols);
     // 8 x ceil(tiles / 8) workgroups (the kernel maps them XCD by XCD; the
     // padding exits at once)
     const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, j.n_split);
-    hipLaunchKernelGGL((tf_gemm_kq_kernel<FMT, TT, CW, KW, PRE, NBUF, DUAL>), grid,
+    hipLaunchKernelGGL((tf_gemm_kq_kernel<FMT, CW, KW, PRE, NBUF, DUAL>), grid,
                        dim3(64 * CW * KW), 0, j.stream, j.w, j.w2, j.x, j.img, j.out, j.n_rows,
                        j.n_cols, j.col_bytes, j.n_tok, j.n_split, j.ldo,
                        (long long)j.n_tok * j.n_cols);
@@ -962,22 +919,22 @@ void tf_pg_f32(bool q6, const TfPgJob& j) {
     };
     if (!q6) {
         if (cost(256, 1, 2.8f, 3.0f) <= cost(128, 4, 2.0f, 8.6f))
-            tf_pg_go<TF_PG_W4, 1, 4, 1, false, 1>(j);
+            tf_pg_go<TF_PG_W4, 4, 1, false, 1>(j);
         else
-            tf_pg_go<TF_PG_W4, 1, 2, 4, false, 1>(j);
+            tf_pg_go<TF_PG_W4, 2, 4, false, 1>(j);
         return;
     }
     const float whole = cost(256, 1, 4.4f, 3.7f), half = cost(128, 2, 6.5f, 4.9f),
                 quarter = cost(64, 4, 6.0f, 7.0f);
     if ((uintptr_t)j.w & 2) {  // unaligned loads: the same order
-        if (whole <= half) tf_pg_go<TF_PG_W6U, 1, 4, 1, false, 1>(j);
-        else tf_pg_go<TF_PG_W6U, 1, 2, 2, false, 2>(j);
+        if (whole <= half) tf_pg_go<TF_PG_W6U, 4, 1, false, 1>(j);
+        else tf_pg_go<TF_PG_W6U, 2, 2, false, 2>(j);
     } else if (whole <= half && whole <= quarter) {
-        tf_pg_go<TF_PG_W6, 1, 4, 1, false, 1>(j);
+        tf_pg_go<TF_PG_W6, 4, 1, false, 1>(j);
     } else if (half <= quarter) {
-        tf_pg_go<TF_PG_W6, 1, 2, 2, false, 2>(j);
+        tf_pg_go<TF_PG_W6, 2, 2, false, 2>(j);
     } else {
-        tf_pg_go<TF_PG_W6, 1, 1, 4, false, 1>(j);
+        tf_pg_go<TF_PG_W6, 1, 4, false, 1>(j);
     }
 }
 
@@ -1046,10 +1003,10 @@ int tf_pg_gemm(const uint8_t* w, int block_bytes, const uint8_t* img, int n_rows
     *part = TfPgPart{ws, n_split, (long long)slice};
     TfPgJob j{w, nullptr, nullptr, img, ws, n_rows, n_cols, col_bytes, n_tok, n_split, n_cols,
               tf_stream(stream)};
-    if (!q6) tf_pg_go<TF_PG_W4, 1, 4, 1, true, 1>(j);
-    else if (block_bytes == 212) tf_pg_go<TF_PG_W6C, 1, 4, 1, true, 1>(j);
-    else if ((uintptr_t)w & 2) tf_pg_go<TF_PG_W6U, 1, 4, 1, true, 1>(j);
-    else tf_pg_go<TF_PG_W6, 1, 4, 1, true, 1>(j);
+    if (!q6) tf_pg_go<TF_PG_W4, 4, 1, true, 1>(j);
+    else if (block_bytes == 212) tf_pg_go<TF_PG_W6C, 4, 1, true, 1>(j);
+    else if ((uintptr_t)w & 2) tf_pg_go<TF_PG_W6U, 4, 1, true, 1>(j);
+    else tf_pg_go<TF_PG_W6, 4, 1, true, 1>(j);
     return TF_LAUNCH_RESULT();
 }
 
@@ -1104,9 +1061,9 @@ int tf_pg_gate_up(const uint8_t* gate, const uint8_t* up, const uint8_t* img, fl
     // a short prompt: half the columns a workgroup and K split over its waves
     // (2048 -> 2 x 11008 at 20 tokens, 86 workgroups: 31 us)
     if (tiles_of(n_tok, n_cols, 32, 128) < (size_t)tf_device_cus() * 3 / 4)
-        tf_pg_go<TF_PG_W4, 1, 2, 4, true, 1, true>(j);
+        tf_pg_go<TF_PG_W4, 2, 4, true, 1, true>(j);
     else
-        tf_pg_go<TF_PG_W4, 1, 4, 1, true, 1, true>(j);
+        tf_pg_go<TF_PG_W4, 4, 1, true, 1, true>(j);
     return TF_LAUNCH_RESULT();
 }
 
