@@ -242,7 +242,8 @@ int tf_gemv_q8_0_qkv(const uint8_t *wq, const uint8_t *wk, const uint8_t *wv,
 
 /* kernels/gemm.cu:6 gemm_q4_k (matmul.rs:1269-1323 gemm): out[t][j] =
  * sum_k W[k][j] x[t][k], x f32, fp32 accuracy (matrix cores on exact
- * integer weights and a three-part bf16 split of x; scales in fp32).
+ * integer weights and x in two f16 parts under one power of two per token
+ * and 256 values, 22 bits of each value; scales in fp32).
  * n_rows % 4 == 0 (floor(n_rows/256) super-blocks are used, as the
  * reference), x and out 16-byte aligned, w and col_bytes 4-byte aligned. */
 int tf_gemm_q4k_f32(const uint8_t *w, const float *x, float *out, int n_rows,
@@ -523,8 +524,8 @@ int tf_model_generate(tf_model *m, const int *forced, int n_forced, int pos0,
                       int n_gen, int *tokens, int use_graph, tf_stream_t stream);
 /* cuda/forward.rs:42-71 forward_greedy for n_tok > 1 (the prompt): the
  * tokens at positions pos0 .. pos0+n_tok-1 go through the n_tok-row forward
- * in chunks of 256 (the prefill GEMMs and attention, f32 activations, as the
- * reference's prefill), their K/V rows are written to the cache, and
+ * in chunks of min(1024, max_seq) (the prefill GEMMs and attention, f32
+ * activations, as the reference's prefill), their K/V rows are written to the cache, and
  * *next_token receives the argmax of the last token's logits (left on the
  * device as after a decode step).  Continue with tf_model_generate(forced =
  * {*next_token}, pos0 + n_tok, ...).  Weights must be Q4_K / Q6_K.  Blocks on
