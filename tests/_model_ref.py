@@ -127,6 +127,62 @@ class RefModel:
         return logits, oracle.argmax(logits)
 
 
+def prefill64(cfg, layers, embedding, tokens):
+    """The prompt's forward in 64 bits, K and V rounded to f16 where the attention
+    reads them: (K and V of each layer [n, kv width], hidden rows [n, n_embd]) for
+    positions 0 .. n-1.  A matrix without a ggml type (12, 14) has the mix's."""
+    from _util import q4k_dequant, q6k_dequant
+
+    E, F, H, KV, hd = (cfg[k] for k in ("n_embd", "n_ff", "n_head", "n_kv", "head_dim"))
+    T = len(tokens)
+
+    def deq(wm, k, q6k):
+        w = np.ascontiguousarray(wm[0])
+        if len(wm) > 2:
+            q6k = wm[2] == 14
+        blk = w.reshape(-1, 210 if q6k else 144)
+        return (q6k_dequant if q6k else q4k_dequant)(blk).reshape(w.shape[0], k).astype(np.float64)
+
+    def norm(a, w):
+        return a / np.sqrt((a * a).mean(1, keepdims=True) + cfg["rms_eps"]) * w
+
+    ang = np.arange(T)[:, None] * cfg["rope_theta"] ** (-2.0 * np.arange(hd // 2) / hd)
+    c, s = np.cos(ang)[:, None], np.sin(ang)[:, None]
+
+    def rope(a, n):
+        a = a.reshape(T, n, hd)
+        a0, a1 = a[..., : hd // 2], a[..., hd // 2:]
+        return np.concatenate([a0 * c - a1 * s, a0 * s + a1 * c], -1).reshape(T, n * hd)
+
+    def bias(L, name):
+        return 0.0 if L.get(name) is None else L[name].astype(np.float64)
+
+    x = deq(embedding, E, True)[tokens]
+    future = np.triu(np.ones((T, T), bool), 1)
+    Ks, Vs = [], []
+    for L in layers:
+        a = norm(x, L["attn_norm"])
+        q = rope(a @ deq(L["wq"], E, False).T + bias(L, "bq"), H)
+        k = rope(a @ deq(L["wk"], E, False).T + bias(L, "bk"), KV)
+        v = a @ deq(L["wv"], E, True).T + bias(L, "bv")
+        Ks.append(k)
+        Vs.append(v)
+        kh, vh = k.astype(np.float16).astype(np.float64), v.astype(np.float16).astype(np.float64)
+        att = np.empty((T, H * hd))
+        for h in range(H):
+            d, g = slice(h * hd, (h + 1) * hd), h // (H // KV)
+            sc = q[:, d] @ kh[:, g * hd:(g + 1) * hd].T / np.sqrt(hd)
+            sc[future] = -np.inf
+            sc = np.exp(sc - sc.max(1, keepdims=True))
+            att[:, d] = sc / sc.sum(1, keepdims=True) @ vh[:, g * hd:(g + 1) * hd]
+        x = x + att @ deq(L["wo"], H * hd, False).T
+        a = norm(x, L["ffn_norm"])
+        g, u = a @ deq(L["gate"], E, False).T, a @ deq(L["up"], E, False).T
+        with np.errstate(over="ignore"):
+            x = x + (g / (1 + np.exp(-g)) * u) @ deq(L["down"], F, L["down_q6k"]).T
+    return Ks, Vs, x
+
+
 class RefModelMixed:
     """CPU reference decode step for any mix of Q4_K / Q6_K / Q5_0 / Q8_0
     matrices ((bytes, col_bytes, ggml type) tuples), assembled in the
