@@ -161,6 +161,11 @@ __global__ __launch_bounds__(256) void tf_attn_prefill_kernel(
 //       step s stands for key 16 s + 8 (i / 4) + 4 h + i % 4, which is how
 //       the scores already lie, so P needs no exchange; the V operand is two
 //       transposing LDS reads (ds_read_b64_tr_b16: four keys of a lane's dim).
+// At head_dim 64, which fp32 vector arithmetic served before, the products of second
+// parts come first in each sum, where it is still small, so that half of the additions
+// round 2^-11 as much (registers for both parts' operands: head_dim 128 has none).
+// Error against 64 bits for 5 tokens at 20, 40 and 300 keys 1.44, 1.62 and 2.25e-7 (part
+// by part 1.86, 2.08 and 2.88; the vector ALU 1.49, 1.79 and 3.59), at the same time.
 // LDS rows keep their 16-byte chunks xor-ed with the row, so that 16 K rows, or
 // the 4 rows x 64 bytes of a transposing read, fall on distinct banks.
 // What bounds it: long contexts, the matrix cores (two products per score and per
@@ -176,6 +181,7 @@ __global__ __launch_bounds__(256) void tf_attn_prefill_kernel(
 // 2.5e-7 at 512, before 6.7e-7 and 2.7e-7.
 #define TF_PM_WAVES 8
 #define TF_PM_T 32  // keys per tile, rows per workgroup
+#define TF_PM_FEW 16  // keys of a workgroup that head_dim 64 takes in fp32
 
 template <int HD>
 struct TfPmLds {
@@ -231,32 +237,36 @@ __device__ __forceinline__ uint32_t tf_div_by(uint32_t r, uint32_t d, uint32_t m
     return t * d > r ? t - 1 : t;
 }
 
-// A head_dim 64 row in which something is not finite, in fp32 as the vector form
-// takes it (an infinity in q, K or V times one f16 part of the other operand is NaN
-// where the product is not): a NaN or -inf score is no key, a +inf one makes the row
-// NaN.  The row's 16 threads take four dims each, one key after the other.
+// A head_dim 64 row in fp32, by 16 threads of four dims each, one key after the other.
+// For rows in which something is not finite: an infinity in q, K or V times one f16
+// part of the other operand is NaN where the product is not.  A NaN or -inf score is
+// no key, a +inf one makes the row NaN, as in the vector form.  And for workgroups of
+// at most TF_PM_FEW keys, where the matrix cores' sums and P's 22 bits are what is left
+// of the error (2, 5 and 12 keys: 4.5, 6.9 and 8.8e-8 against 64 bits, 3.9, 6.2 and
+// 8.4 here, 4.1, 6.3 and 8.5 on the vector ALU before; from 20 keys on the matrix
+// cores are the better: 1.4 against 1.5e-7).  5.0 us for 5 tokens either way.
 __device__ __noinline__ float4 tf_attn_row64(const float* q, const uint8_t* kbase,
                                              const uint8_t* vbase, uint32_t row_bytes, int n_keys,
                                              float scale) {
     const int m = threadIdx.x & 15;
     const float4 a = *reinterpret_cast<const float4*>(q + 4 * m);
+    auto score = [&](int t) {
+        const uint2 k = *reinterpret_cast<const uint2*>(kbase + (size_t)t * row_bytes + 8 * m);
+        return scale * tf_row16_sum(a.x * tf_h2f(k.x) + a.y * tf_h2f(k.x >> 16) +
+                                    a.z * tf_h2f(k.y) + a.w * tf_h2f(k.y >> 16));
+    };
     float mx = -1e30f, l = 0.f;
+    for (int t = 0; t < n_keys; t++) mx = fmaxf(mx, score(t));
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int t = 0; t < n_keys; t++) {
-        const size_t off = (size_t)t * row_bytes + 8 * m;
-        const uint2 k = *reinterpret_cast<const uint2*>(kbase + off);
-        const uint2 v = *reinterpret_cast<const uint2*>(vbase + off);
-        const float s = scale * tf_row16_sum(a.x * tf_h2f(k.x) + a.y * tf_h2f(k.x >> 16) +
-                                             a.z * tf_h2f(k.y) + a.w * tf_h2f(k.y >> 16));
-        const float m_new = fmaxf(mx, s);
-        const float alpha = __expf(mx - m_new);
-        const float e = s > -1e29f ? __expf(s - m_new) : 0.f;
-        mx = m_new;
-        l = l * alpha + e;
-        acc.x = acc.x * alpha + e * tf_h2f(v.x);
-        acc.y = acc.y * alpha + e * tf_h2f(v.x >> 16);
-        acc.z = acc.z * alpha + e * tf_h2f(v.y);
-        acc.w = acc.w * alpha + e * tf_h2f(v.y >> 16);
+        const uint2 v = *reinterpret_cast<const uint2*>(vbase + (size_t)t * row_bytes + 8 * m);
+        const float s = score(t);
+        const float e = s > -1e29f ? __expf(s - mx) : 0.f;
+        l += e;
+        acc.x += e * tf_h2f(v.x);
+        acc.y += e * tf_h2f(v.x >> 16);
+        acc.z += e * tf_h2f(v.y);
+        acc.w += e * tf_h2f(v.y >> 16);
     }
     const float inv = 1.f / fmaxf(l, 1e-20f);
     return make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
@@ -288,6 +298,15 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
     const uint32_t row_bytes = (uint32_t)n_kv * ROWB;
     const uint8_t* kbase = reinterpret_cast<const uint8_t*>(kc) + (size_t)kv_h * ROWB;
     const uint8_t* vbase = reinterpret_cast<const uint8_t*>(vc) + (size_t)kv_h * ROWB;
+    if (HD == 64 && kv_len <= TF_PM_FEW) {
+        const int r = r0 + (tid >> 4), qo = tf_div_by(r, G, g_inv);
+        if (r < n_rows) {
+            const size_t row = ((size_t)qo * n_head + (size_t)kv_h * G + (r - qo * G)) * HD;
+            *reinterpret_cast<float4*>(out + row + 4 * (tid & 15)) =
+                tf_attn_row64(q + row, kbase, vbase, row_bytes, pos0 + qo + 1, scale);
+        }
+        return;
+    }
     uint8_t* kt = lds + wave * L::WAVE;
     uint8_t* vt = kt + L::TILE;
 
@@ -409,11 +428,25 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
         tf_f32x16 sc;
 #pragma unroll
         for (int i = 0; i < 16; i++) sc[i] = 0.f;
+        auto k_frag = [&](int st) {
+            return *reinterpret_cast<const tf_h8*>(kt + l32 * ROWB + 16 * ((2 * st + h) ^ ksw));
+        };
+        if constexpr (HD == 64) {  // the second parts first, see above
+            tf_h8 ka[ST];
 #pragma unroll
-        for (int st = 0; st < ST; st++) {
-            const tf_h8 ka = *reinterpret_cast<const tf_h8*>(kt + l32 * ROWB + 16 * ((2 * st + h) ^ ksw));
-            sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qb[st][0], sc, 0, 0, 0);
-            sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qb[st][1], sc, 0, 0, 0);
+            for (int st = 0; st < ST; st++) ka[st] = k_frag(st);
+#pragma unroll
+            for (int pl = 1; pl >= 0; pl--)
+#pragma unroll
+                for (int st = 0; st < ST; st++)
+                    sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[st], qb[st][pl], sc, 0, 0, 0);
+        } else {
+#pragma unroll
+            for (int st = 0; st < ST; st++) {
+                const tf_h8 ka = k_frag(st);
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qb[st][0], sc, 0, 0, 0);
+                sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qb[st][1], sc, 0, 0, 0);
+            }
         }
         if (more) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the K tile has been read
@@ -474,21 +507,40 @@ __global__ __launch_bounds__(64 * TF_PM_WAVES, 2) void tf_attn_prefill_mfma_kern
         l += ls;
         if (more) tf_wait_vm<NC>();  // V of tile j
         else tf_wait_vm<0>();
+        auto v_frag = [&](int s, int db) {
+            const tf_lds_u8* vp = (const tf_lds_u8*)(vt + vrow + 16 * s * ROWB + 64 * (db ^ vsw));
+            const tf_h4 v0 = __builtin_bit_cast(
+                tf_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                           (__attribute__((address_space(3))) tf_s4*)vp));
+            const tf_h4 v1 = __builtin_bit_cast(
+                tf_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                           (__attribute__((address_space(3))) tf_s4*)(vp + 8 * ROWB)));
+            return __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
+        if constexpr (HD == 64) {
+            tf_h8 vf[2][DB];
 #pragma unroll
-        for (int s = 0; s < 2; s++)
+            for (int s = 0; s < 2; s++)
 #pragma unroll
-            for (int db = 0; db < DB; db++) {
-                const tf_lds_u8* vp = (const tf_lds_u8*)(vt + vrow + 16 * s * ROWB + 64 * (db ^ vsw));
-                const tf_h4 v0 = __builtin_bit_cast(
-                    tf_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                               (__attribute__((address_space(3))) tf_s4*)vp));
-                const tf_h4 v1 = __builtin_bit_cast(
-                    tf_h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                               (__attribute__((address_space(3))) tf_s4*)(vp + 8 * ROWB)));
-                const tf_h8 vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pa[s][0], o[db], 0, 0, 0);
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pa[s][1], o[db], 0, 0, 0);
-            }
+                for (int db = 0; db < DB; db++) vf[s][db] = v_frag(s, db);
+#pragma unroll
+            for (int pl = 1; pl >= 0; pl--)
+#pragma unroll
+                for (int s = 0; s < 2; s++)
+#pragma unroll
+                    for (int db = 0; db < DB; db++)
+                        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[s][db], pa[s][pl], o[db],
+                                                                       0, 0, 0);
+        } else {
+#pragma unroll
+            for (int s = 0; s < 2; s++)
+#pragma unroll
+                for (int db = 0; db < DB; db++) {
+                    const tf_h8 vf = v_frag(s, db);
+                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pa[s][0], o[db], 0, 0, 0);
+                    o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pa[s][1], o[db], 0, 0, 0);
+                }
+        }
         if (more) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the V tile has been read
             issue(vbase, vt, t0 + TF_PM_WAVES * TF_PM_T, true);
