@@ -220,7 +220,10 @@ __device__ __forceinline__ void tf_pg_store_x(const tf_pg_f4 (&xr)[NP][2], uint8
 // PRE: x is already in images (ximg, [token tile of 32][super-block], TF_PG_SLOT
 // bytes each) and is copied into LDS; otherwise the workgroup converts x itself,
 // into one image a slice or, NBUF 2, two in turn.  out has rows of ldo floats.
-template <int FMT, int CW, int KW, bool PRE, int NBUF, bool DUAL>
+// FINE (Q6_K): the products of h0 and the weights' f16 values are scaled and added to
+// the sum after every 64 values; all smaller ones, those of h1 and the remainders
+// among them, have accumulators of their own.
+template <int FMT, int CW, int KW, bool PRE, int NBUF, bool DUAL, bool FINE>
 __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint8_t* __restrict__ w,
                                            const uint8_t* __restrict__ w2,
                                            const float* __restrict__ x,
@@ -490,6 +493,29 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
             TF_PG_FENCE();
 #pragma unroll
             for (int ct = 0; ct < 2; ct++) tf_pg_load_hdr<FMT>(wn[ct], woff[ct], odd_of(ct, n1), wc[ct]);
+            auto fold = [&](tf_pg_f16v (&p)[2]) {  // acc += 2^-e d p, p = 0
+                const float* xinv = reinterpret_cast<const float*>(slot + TF_PG_IMG + TF_PG_SUMS);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const float4 fi = *reinterpret_cast<const float4*>(xinv + 8 * k + 4 * h);
+                    const float fv[4] = {fi.x, fi.y, fi.z, fi.w};
+#pragma unroll
+                    for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const int i = 4 * k + r;
+                            acc[ct][i] = fmaf(fv[r], dv[ct] * p[ct][i], acc[ct][i]);
+                            p[ct][i] = 0.f;
+                        }
+                }
+            };
+            [[maybe_unused]] tf_pg_f16v lo[2];
+            if constexpr (FINE) {
+#pragma unroll
+                for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) lo[ct][i] = 0.f;
+            }
 #pragma unroll
             for (int n = 0; n < 2; n++) {
                 uint32_t qh[2][4], qh8[2][4];
@@ -550,13 +576,16 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
                                 }
                             }
 #pragma unroll
-                            for (int m = 0; m < 3; m++)
+                            for (int m = 0; m < (FINE ? 4 : 3); m++)
 #pragma unroll
-                                for (int ct = 0; ct < 2; ct++)
-                                    P[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                        xf[m == 1], m == 2 ? bl[ct] : bh[ct], P[ct], 0, 0, 0);
+                                for (int ct = 0; ct < 2; ct++) {
+                                    tf_pg_f16v& p = FINE && m > 0 ? lo[ct] : P[ct];
+                                    p = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                        xf[m & 1], m >= 2 ? bl[ct] : bh[ct], p, 0, 0, 0);
+                                }
                         }
                     }
+                    if constexpr (FINE) fold(P);
                     TF_PG_FENCE();
 #pragma unroll
                     for (int ct = 0; ct < 2; ct++)
@@ -566,18 +595,8 @@ __device__ __forceinline__ void tf_pg_body(uint8_t* __restrict__ lds, const uint
                 for (int ct = 0; ct < 2; ct++)
                     tf_pg_load_run<FMT>(wn[ct], woff[ct], odd_of(ct, n1), h, 4 + n, wc[ct]);
             }
-            const float* xinv = reinterpret_cast<const float*>(slot + TF_PG_IMG + TF_PG_SUMS);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const float4 fi = *reinterpret_cast<const float4*>(xinv + 8 * k + 4 * h);
-                const float fv[4] = {fi.x, fi.y, fi.z, fi.w};
-#pragma unroll
-                for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        acc[ct][4 * k + r] =
-                            fmaf(fv[r], dv[ct] * P[ct][4 * k + r], acc[ct][4 * k + r]);
-            }
+            if constexpr (FINE) fold(lo);
+            else fold(P);
         }
     }
     if constexpr (KW > 1) {  // slices 1.. hand their sums to slice 0, added in slice order
@@ -638,9 +657,10 @@ __device__ __forceinline__ bool tf_pg_tile(int ntx, int n_ct, int& tx, int& ct) 
 
 // Waves per SIMD: 3 where the registers allow it (Q4_K without conversion
 // registers), else 2, or what four images of LDS (136 KB) leave room for.
-template <int FMT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false>
+template <int FMT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false, bool FINE = false>
 __global__ __launch_bounds__(64 * CW * KW, KW * NBUF >= 4            ? CW * KW / 4
                                            : PRE && FMT == TF_PG_W4 ? 3
+                                           : FINE                   ? 1
                                                                     : 2) void
 tf_gemm_kq_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
                   const float* __restrict__ x, const uint8_t* __restrict__ ximg,
@@ -650,14 +670,15 @@ tf_gemm_kq_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
     constexpr int COLS = (DUAL ? 32 : 64) * CW;
     int tx, ct;
     if (!tf_pg_tile((n_tok + 31) / 32, (n_cols + COLS - 1) / COLS, tx, ct)) return;
-    tf_pg_body<FMT, CW, KW, PRE, NBUF, DUAL>(
+    tf_pg_body<FMT, CW, KW, PRE, NBUF, DUAL, FINE>(
         lds, w, w2, x, ximg, out + (size_t)blockIdx.z * (size_t)split_stride, ldo, n_rows, n_cols,
         col_bytes, n_tok, n_split, tx * 32, ct);
 }
 
 // q, k and v of a prompt in one launch (their outputs side by side in rows of
 // ldo floats): the column tiles of the three matrices one after the other.
-__global__ __launch_bounds__(256, 2) void tf_pg_qkv_kernel(TfPgQkv m, const uint8_t* __restrict__ ximg,
+template <bool FINE>
+__global__ __launch_bounds__(256, FINE ? 1 : 2) void tf_pg_qkv_kernel(TfPgQkv m, const uint8_t* __restrict__ ximg,
                                                            float* __restrict__ out, int ldo,
                                                            int n_rows, int n_tok, int n_split,
                                                            long long split_stride) {
@@ -668,7 +689,7 @@ __global__ __launch_bounds__(256, 2) void tf_pg_qkv_kernel(TfPgQkv m, const uint
     if (i) ct -= m.ct[i - 1];
     float* o = out + (size_t)blockIdx.z * (size_t)split_stride + m.col[i];
     auto go = [&](auto fmt) {
-        tf_pg_body<decltype(fmt)::value, 4, 1, true, 1, false>(
+        tf_pg_body<decltype(fmt)::value, 4, 1, true, 1, false, FINE>(
             lds, m.w[i], nullptr, nullptr, ximg, o, ldo, n_rows, m.n_cols[i], m.col_bytes[i], n_tok,
             n_split, tx * 32, ct);
     };
@@ -858,7 +879,7 @@ struct TfPgJob {
     hipStream_t stream;
 };
 
-template <int FMT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false>
+template <int FMT, int CW, int KW, bool PRE, int NBUF, bool DUAL = false, bool FINE = false>
 void tf_pg_go(const TfPgJob& j) {
     const int cols = (DUAL ? 32 : 64) * CW;
     const size_t tiles = (size_t)((j.n_tok + 31) / 32) *
@@ -866,10 +887,25 @@ void tf_pg_go(const TfPgJob& j) {
     // 8 x ceil(tiles / 8) workgroups (the kernel maps them XCD by XCD; the
     // padding exits at once)
     const dim3 grid((unsigned)(8 * ((tiles + 7) / 8)), 1, j.n_split);
-    hipLaunchKernelGGL((tf_gemm_kq_kernel<FMT, CW, KW, PRE, NBUF, DUAL>), grid,
+    hipLaunchKernelGGL((tf_gemm_kq_kernel<FMT, CW, KW, PRE, NBUF, DUAL, FINE>), grid,
                        dim3(64 * CW * KW), 0, j.stream, j.w, j.w2, j.x, j.img, j.out, j.n_rows,
                        j.n_cols, j.col_bytes, j.n_tok, j.n_split, j.ldo,
                        (long long)j.n_tok * j.n_cols);
+}
+
+// tf_pg_go for Q6_K weights, FINE where K is short.  A super-block is 48 additions to
+// one fp32 sum in the matrix cores, 1.7e-7 of the result whatever K.  The form before
+// them scaled and added every 16 values, an error that grows with K but begins lower:
+// against 64 bits 0.91, 1.14, 1.50, 1.70 and 2.11e-7 at K = 256, 512, 1024, 1280 and
+// 2048.  FINE has 0.90, 0.93, 0.98 and 1.01e-7 at the first four.  It costs 8.9
+// against 7.8 us for 256 -> 2000 at 64 tokens and 25.2 against 20.8 for 1024 -> 4096 at
+// 300 (9.6 and 43.1 before); sums of 128 or 32 values in one accumulator gave 1.3 and
+// 1.04e-7 at K = 256 and 22.9 and 29.2 us at K = 1024.
+bool tf_pg_fine(int n_rows) { return n_rows / 256 <= 5; }
+template <int FMT, int CW, int KW, bool PRE, int NBUF>
+void tf_pg_go6(const TfPgJob& j) {
+    if (tf_pg_fine(j.n_rows)) tf_pg_go<FMT, CW, KW, PRE, NBUF, false, true>(j);
+    else tf_pg_go<FMT, CW, KW, PRE, NBUF>(j);
 }
 
 size_t tiles_of(int n_tok, int n_cols, int toks, int cols) {
@@ -927,14 +963,14 @@ void tf_pg_f32(bool q6, const TfPgJob& j) {
     const float whole = cost(256, 1, 4.4f, 3.7f), half = cost(128, 2, 6.5f, 4.9f),
                 quarter = cost(64, 4, 6.0f, 7.0f);
     if ((uintptr_t)j.w & 2) {  // unaligned loads: the same order
-        if (whole <= half) tf_pg_go<TF_PG_W6U, 4, 1, false, 1>(j);
-        else tf_pg_go<TF_PG_W6U, 2, 2, false, 2>(j);
+        if (whole <= half) tf_pg_go6<TF_PG_W6U, 4, 1, false, 1>(j);
+        else tf_pg_go6<TF_PG_W6U, 2, 2, false, 2>(j);
     } else if (whole <= half && whole <= quarter) {
-        tf_pg_go<TF_PG_W6, 4, 1, false, 1>(j);
+        tf_pg_go6<TF_PG_W6, 4, 1, false, 1>(j);
     } else if (half <= quarter) {
-        tf_pg_go<TF_PG_W6, 2, 2, false, 2>(j);
+        tf_pg_go6<TF_PG_W6, 2, 2, false, 2>(j);
     } else {
-        tf_pg_go<TF_PG_W6, 1, 4, false, 1>(j);
+        tf_pg_go6<TF_PG_W6, 1, 4, false, 1>(j);
     }
 }
 
@@ -1004,9 +1040,9 @@ int tf_pg_gemm(const uint8_t* w, int block_bytes, const uint8_t* img, int n_rows
     TfPgJob j{w, nullptr, nullptr, img, ws, n_rows, n_cols, col_bytes, n_tok, n_split, n_cols,
               tf_stream(stream)};
     if (!q6) tf_pg_go<TF_PG_W4, 4, 1, true, 1>(j);
-    else if (block_bytes == 212) tf_pg_go<TF_PG_W6C, 4, 1, true, 1>(j);
-    else if ((uintptr_t)w & 2) tf_pg_go<TF_PG_W6U, 4, 1, true, 1>(j);
-    else tf_pg_go<TF_PG_W6, 4, 1, true, 1>(j);
+    else if (block_bytes == 212) tf_pg_go6<TF_PG_W6C, 4, 1, true, 1>(j);
+    else if ((uintptr_t)w & 2) tf_pg_go6<TF_PG_W6U, 4, 1, true, 1>(j);
+    else tf_pg_go6<TF_PG_W6, 4, 1, true, 1>(j);
     return TF_LAUNCH_RESULT();
 }
 
@@ -1031,9 +1067,13 @@ int tf_pg_qkv(const uint8_t* const w[3], const int block_bytes[3], const int n_c
     TF_CHECK_ARG(img && slice <= ws_floats);
     const int n_split = tf_pg_splits(tiles, n_rows / 256, slice, ws_floats);
     *part = TfPgPart{ws, n_split, (long long)slice};
-    hipLaunchKernelGGL(tf_pg_qkv_kernel, dim3((unsigned)(8 * ((tiles + 7) / 8)), 1, n_split),
-                       dim3(256), 0, tf_stream(stream), m, img, ws, col, n_rows, n_tok, n_split,
-                       (long long)slice);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)(8 * ((tiles + 7) / 8)), 1, n_split), dim3(256), 0,
+                           tf_stream(stream), m, img, ws, col, n_rows, n_tok, n_split,
+                           (long long)slice);
+    };
+    if (tf_pg_fine(n_rows)) go(tf_pg_qkv_kernel<true>);
+    else go(tf_pg_qkv_kernel<false>);
     return TF_LAUNCH_RESULT();
 }
 

@@ -15,7 +15,7 @@ import torch
 
 from taraference_amd import synth
 from _gpu import KEEP, P, S, call, dev, empty, host
-from _util import assert_gemv_close, gemm_ref
+from _util import assert_gemv_close, gemm_ref, q6k_dequant
 
 pytestmark = pytest.mark.gpu
 
@@ -77,6 +77,30 @@ def test_gemm_scales_of_x(gpu, fmt):
     x[7] = np.float32(1e-38)  # subnormal products with the block scales still count
     x[8] = 1
     run(fmt, 768, 200, x)
+
+
+@pytest.mark.parametrize("k,n,t,bar", [
+    (256, 2000, 20, 0.95e-7),   # one super-block
+    (512, 900, 64, 1.1e-7),     # 2 of 64 columns and K / 4
+    (1280, 4100, 130, 1.1e-7),  # the last width that adds 64 values at a time
+    (1536, 1000, 40, 1.85e-7),  # whole super-blocks
+])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_gemm_q6k_error(gpu, k, n, t, bar, shift):
+    """Q6_K is no further from 64 bits than sums that were scaled every 16 values: 0.91,
+    1.14, 1.70 and 1.85e-7 of the result's 2-norm for normal x and scales over their
+    whole range (48 products a value in one sum have 1.7e-7)."""
+    rng = np.random.default_rng(k)
+    blk = synth.q6k_blocks(rng, n * k // 256)
+    blk[:, 192:208] = rng.integers(-128, 128, (len(blk), 16)).astype(np.int8).view(np.uint8)
+    w = blk.reshape(n, -1)
+    x = rng.standard_normal((t, k)).astype(np.float32)
+    buf = dev(np.concatenate([np.zeros(shift, np.uint8), w.reshape(-1)]))
+    out = empty(t * n)
+    print(f"gemm q6k error {k}x{n} tok={t} shift={shift}", flush=True)
+    call("tf_gemm_q6k_f32", P(buf) + shift, P(dev(x)), P(out), k, n, w.shape[1], t, S())
+    ref = x.astype(np.float64) @ q6k_dequant(blk).reshape(n, k).astype(np.float64).T
+    assert np.linalg.norm(host(out).reshape(t, n) - ref) <= bar * np.linalg.norm(ref)
 
 
 @pytest.mark.parametrize("fmt,n_rows,n_cols,n_tok", [
