@@ -59,7 +59,7 @@ struct TfB32Job {
     const float* norm_w;  // TF_B32_SRC_NORM
     float eps;
     const float* part;  // TF_B32_SRC_FLASH: [head][split](m, l, O[head_dim])
-    int parts, head_dim;  // parts: 8 or 16
+    int parts, head_dim;  // parts: 8, 16 or 24
     int paired;  // task 2j: column j of w[0], 2j + 1: of w[1]; out[0] = silu(.) * (.)
 };
 
@@ -171,7 +171,9 @@ __device__ __forceinline__ void tf_b32_stage(const TfB32Job& jb, uint8_t* lds) {
         for (int i = threadIdx.x; i < G * 8; i += blockDim.x) {
             float4 v;
             if constexpr (SK == TF_B32_SRC_FLASH)
-                v = jb.parts == 8 ? tf_b32_merge4<1>(jb, 4 * i) : tf_b32_merge4<2>(jb, 4 * i);
+                v = jb.parts == 8    ? tf_b32_merge4<1>(jb, 4 * i)
+                    : jb.parts == 16 ? tf_b32_merge4<2>(jb, 4 * i)
+                                     : tf_b32_merge4<3>(jb, 4 * i);
             else v = *reinterpret_cast<const float4*>(jb.x + 4 * i);
             if constexpr (SK == TF_B32_SRC_NORM) {
                 const float4 w = *reinterpret_cast<const float4*>(jb.norm_w + 4 * i);
@@ -743,9 +745,12 @@ int tf_b32_norm_qkv(const float* x, const float* norm_w, float eps, const uint8_
     return rc;
 }
 
+// Each workgroup of wo merges all heads for itself, which grows with the partials:
+// 16 steps of six 896-wide layers take 3592 us with it at 16 partials and 3681 with
+// the merge's own launch, 3636 and 3689 at 24, 3705 and 3671 at 32.
 bool tf_b32_flash_out_fits(int n_head, int head_dim, int parts) {
     return n_head > 0 && head_dim > 0 && head_dim % 32 == 0 && n_head * head_dim <= 2048 &&
-           (parts == 8 || parts == 16);
+           (parts == 8 || parts == 16 || parts == 24);
 }
 
 int tf_b32_flash_out(const uint8_t* w, const float* partial, int n_head, int head_dim, int parts,

@@ -724,8 +724,10 @@ struct tf_model {
 
     // Tokens of a prompt that go through the layers together.  The reference
     // takes 256 (types.rs MAX_BATCH); the weights are read and unpacked once a
-    // chunk and a chunk's tiles have to fill 256 CUs, so a longer one pays:
-    // 700 tokens of two 3B layers in one chunk / in three.
+    // chunk and a chunk's tiles have to fill 256 CUs, so a longer one pays: two 3B
+    // layers and the head take 1250, 1136 and 962 us for 700 tokens in chunks of
+    // 256, 512 and 1024, and 3364, 2827, 2480 and 2347 for 2048 in chunks up to
+    // 2048.  1024 holds the workspace to 160 MB at that width.
     static constexpr int kPrefillChunk = 1024;
 
     // The prompt forward of forward.rs:42-71 forward_greedy / :360-404
@@ -734,7 +736,7 @@ struct tf_model {
     // n_tok > 1: rms_norm rows, GEMMs, add_bias, rope, copy_kv, prefill
     // attention, GEMM + add for wo and down, silu_mul), K/V appended at
     // positions pos0 .. pos0+n-1; then the last row's logits and argmax
-    // (logits_from_last), as the decode step computes them.  Per layer nine
+    // (logits_from_last), as the decode step computes them.  Per layer ten
     // launches: each GEMM's K slices are added by the kernel that reads them.
     void prefill(hipStream_t s, const int* tokens, int n, int pos0) {
         const tf_model_config& c = cfg;
@@ -750,7 +752,7 @@ struct tf_model {
             pf_g = alloc<float>((size_t)CH * F);
             pf_tok = alloc<int>(CH);
             pf_img = alloc<uint8_t>(tf_pg_image_bytes(std::max(E, F), CH));
-            // the GEMM slices: two of a full chunk's widest output, and more of a short one's
+            // the GEMM slices: four of a full chunk's q, k and v, and more of a short one's
             pf_ws_floats = std::max((size_t)4 * CH * (E + 2 * kvd), (size_t)4 << 20);
             pf_ws = alloc<float>(pf_ws_floats);
             pf_x = alloc<float>((size_t)CH * E);

@@ -1014,11 +1014,11 @@ int tf_pg_add_row(float* x, const TfPgPart& part, int row, int n, tf_stream_t st
     return TF_LAUNCH_RESULT();
 }
 
-// Slices of K for `tiles` output tiles: about 2.5 workgroups a CU in all, as
-// many as fit ws (a 700-token prompt of two 3B layers at 1, 1.5, 2, 2.5, 3, 4
-// a CU: 1190, 1096, 1137, 1095, 1096, 1104 us; 100 tokens: 524, 540, 541, 559,
-// 555, 563.  More slices shorten the GEMM and lengthen the kernel that adds
-// them; at 2, three slices of 176 tiles are one workgroup more than two a CU.)
+// Slices of K for `tiles` output tiles: about 2.5 workgroups a CU in all, as many as
+// fit ws.  Two 3B layers and the head at 1, 1.5, 2, 2.5 and 3 a CU: 1065, 981, 1010,
+// 962 and 966 us for 700 tokens, 1327, 1292, 1285, 1285 and 1291 for 1024, 580, 568,
+// 575, 583 and 598 for 300, no more than 2 % apart for 20 to 180.  More slices shorten
+// the GEMM and lengthen the kernel that adds them.
 static int tf_pg_splits(size_t tiles, int nb, size_t slice, size_t ws_floats) {
     const size_t target = 5 * (size_t)tf_device_cus() / 2;
     int n = tiles >= target ? 1 : (int)((target + tiles / 2) / tiles);

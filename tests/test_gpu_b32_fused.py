@@ -51,7 +51,8 @@ class Ref(RefModelMixed):
     (4, 2, 512, 257, 40),      # one block a quad
     (17, 17, 768, 1003, 40),   # 34 blocks: the last round of a quad nearly empty
     (32, 4, 256, 130, 1024),   # the widest row, 16 partials
-    (8, 8, 256, 64, 1600),     # 24 partials: merged by their own launch
+    (8, 8, 256, 64, 1600),     # 24 partials
+    (8, 8, 256, 64, 2100),     # 32 partials: merged by their own launch
 ])
 def test_fused_layers(gpu, tmp_path, heads, kv, ff, vocab, max_seq):
     from taraference_amd.model import DecodeModel
@@ -124,11 +125,12 @@ def test_norm_gate_up_as_separate_launches(gpu, heads, kv):
     b.close()
 
 
-@pytest.mark.parametrize("heads,kv,max_seq", [(14, 2, 60), (5, 5, 900), (14, 2, 1100), (32, 4, 1535)])
+@pytest.mark.parametrize("heads,kv,max_seq", [(14, 2, 60), (5, 5, 900), (14, 2, 1100), (32, 4, 1535),
+                                              (14, 2, 1600), (32, 4, 2047)])
 def test_merge_wo_as_separate_launches(gpu, heads, kv, max_seq):
     """One layer whose FFN adds nothing (gate 0): the logits are those of the
-    C ABI's own sequence with tf_flash_decode_reduce and tf_gemv_q5_0_f32, at 8
-    and at 16 partials."""
+    C ABI's own sequence with tf_flash_decode_reduce and tf_gemv_q5_0_f32, at 8,
+    16 and 24 partials."""
     e, hd, vocab = 64 * heads, 64, 130
     cfg = dict(n_layer=1, n_embd=e, n_ff=256, n_head=heads, n_kv=kv, head_dim=hd, n_vocab=vocab,
                rope_theta=1e6, rms_eps=1e-6)
@@ -146,7 +148,7 @@ def test_merge_wo_as_separate_launches(gpu, heads, kv, max_seq):
         m.forward(tok, pos)
     pos, tok = len(toks) - 1, toks[-1]
     ns = m.lib.tf_flash_decode_n_split(kv, max_seq)
-    assert ns == (16 if max_seq >= 1024 else 8)
+    assert ns == max(8, max_seq // 512 * 8) <= 24
     x, xb, q, k, att = empty(e), empty(e), empty(e), empty(kv * hd), empty(e)
     part, lg = empty(heads * ns * (2 + hd)), empty(vocab)
     xq, xd = empty(e, torch.int8), empty(e // 32)
