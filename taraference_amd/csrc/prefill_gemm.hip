@@ -1052,6 +1052,7 @@ int tf_pg_qkv(const uint8_t* const w[3], const int block_bytes[3], const int n_c
     TfPgQkv m{};
     int ct = 0, col = 0;
     for (int i = 0; i < 3; i++) {
+        TF_CHECK_ARG(block_bytes[i] == 144 || block_bytes[i] == 210);  // no compact form
         const bool q6 = block_bytes[i] != 144;
         const int rc = tf_pg_check(q6, w[i], ws, n_rows, n_cols[i], col_bytes[i], n_tok, block_bytes[i]);
         if (rc) return rc;
