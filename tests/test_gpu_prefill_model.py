@@ -140,6 +140,7 @@ def test_prefill_tiles_and_chunks(gpu, n_prompt, n_more, ff):
     (256, 512, 33, ("wq", "gate")),        # blocks and columns of 210 bytes: every other at 2 mod 4
     (512, 2560, 300, ("wk", "wo", "up")),
     (768, 1024, 70, ("wq", "wk", "gate", "up", "down")),
+    (1536, 2048, 40, ("wq", "wo", "gate")),  # rows whose super-blocks are added whole
 ])
 def test_prefill_q6k_matrices(gpu, e, ff, n, q6, shift):
     """Q6_K where the usual mix has Q4_K: q / k / v of mixed types in one launch, gate
