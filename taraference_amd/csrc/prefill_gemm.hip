@@ -17,7 +17,8 @@
 // keeps 22 bits.  A super-block therefore accumulates in the matrix cores (two
 // MFMAs per 16 values for Q4_K; three for Q6_K, the remainder against h0 only,
 // what is left out being below 2^-23 of the largest product), and d, dmin and
-// 2^-e are applied in fp32 once per super-block.
+// 2^-e are applied in fp32 once per super-block (short Q6_K rows: all four
+// products, and every 64 values, see FINE).
 //
 // What bounds it: the matrix cores and the vector ALU about equally.  Per
 // super-block a wave's 32 x 64 tile is 64 MFMAs of 32 cycles (Q6_K: 96), and
